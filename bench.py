@@ -416,7 +416,7 @@ def measured_traffic(kind: str, n: int):
 # contains it (the flux kernel has one per direction); their per-dispatch
 # values are averaged.
 KERNEL_SYMBOLS = {
-    "prep": ("colloc_centred_kernel<true>", "ghost_collocate_kernel", "qmhd::prep_kernel"),
+    "prep": ("prep_kernel<true, 8>",),
     "reconstruct": ("reconstruct_kernel<double, 7>", "reconstruct_fallback_kernel<double, 7>"),
     "flux": ("flux_kernel<double, 7, false, ",),
     "cell_emf": ("cell_emf_kernel<double, 7, false, 16, 16>",),

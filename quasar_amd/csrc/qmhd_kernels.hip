@@ -15,6 +15,7 @@
 #include "qmhd_queue.hpp"
 #include "qmhd_stencil.hpp"
 
+#include <algorithm>
 #include <cstdint>
 #include <stdexcept>
 
@@ -122,90 +123,39 @@ __device__ __forceinline__ double ulp_of(double v) {
   return ldexp(0.5, e - 52);
 }
 
-// Prepare kernel: collocated Bx/By of `u` over the padded grid, and on interior
-// cells (a) the admissible fraction of u against `base` (stage check), (b) the
-// live-state admissibility under both collocations, (c) the relative div(B)
-// residual/scale maxima.  Results go to `status` through order-independent
-// atomics.
+// Whether a cell state is finite with rho > 0 and internal energy q > 0 beyond
+// any rounding of q: then convex_q's q, which rounds in another order, is
+// positive too.  (False only says that convex_q has to decide.)
+__device__ __forceinline__ bool clearly_admissible(const St<double>& s, double bx, double by) {
+  const double kin = 0.5 * (s.mx * s.mx + s.my * s.my + s.mz * s.mz) * frcp(s.rho);
+  const double mag = 0.5 * (bx * bx + by * by + s.bz * s.bz);
+  const double q = (s.en - kin) - mag;
+  return s.rho > 0.0 && q > 32.0 * Lim<double>::eps * (__builtin_fabs(s.en) + kin + mag) + 1e-290;
+}
+
 __device__ __forceinline__ double ok_or_zero(double v) { return fin(v) ? v : 0.0; }
 
-// Centred collocation of the staggered field on every padded cell whose
-// stencil lies inside the grid (the outer ghost layers take the one-sided
-// closures of ghost_collocate_kernel).  EXACT: correctly rounded (the FP64
-// form); otherwise a fused multiply-add sum (the FP32 forms).
-template <bool EXACT>
-__device__ __forceinline__ void colloc_centred_kernel_tile(
-    const Blk& qb, const GridD& g, const double* __restrict__ bxf, const double* __restrict__ byf,
-    double* __restrict__ bxc, double* __restrict__ byc) {
-#include "tiles/colloc_centred_kernel.inc"
-}
-
-template <bool EXACT>
-__global__ __launch_bounds__(256) void colloc_centred_kernel(GridD g, const double* __restrict__ bxf,
-                                                             const double* __restrict__ byf,
-                                                             double* __restrict__ bxc, double* __restrict__ byc) {
-  [[maybe_unused]] const Blk qb = Blk::xcd_tiled();
-#include "tiles/colloc_centred_kernel.inc"
-}
-
-// Queue form of colloc_centred_kernel (one launch over the tiles of many runs).
-template <bool EXACT>
-struct colloc_centred_kernel_q {
-  struct Args {
-    GridD g;
-    const double* bxf;
-    const double* byf;
-    double* bxc;
-    double* byc;
-  };
-  static __device__ __forceinline__ void run(const Blk& qb, const Args& a) {
-    colloc_centred_kernel_tile<EXACT>(qb, queue_arg(a.g), queue_arg(a.bxf), queue_arg(a.byf), queue_arg(a.bxc),
-                                      queue_arg(a.byc));
-  }
-  static void launch(dim3 grid, dim3 block, hipStream_t s, const Args& a) {
-    hipLaunchKernelGGL((colloc_centred_kernel<EXACT>), grid, block, 0, s, a.g, a.bxf, a.byf, a.bxc, a.byc);
-  }
-  static const void* tag() {
-    static const char t = 0;
-    return &t;
-  }
-};
-
-// colloc_centred_kernel over the tile queue, one workgroup per tile: the same text, the
-// arguments read from the tile's run record.
-template <bool EXACT>
-__global__ __launch_bounds__(256) void colloc_centred_kernel_queue(
-    const typename colloc_centred_kernel_q<EXACT>::Args* __restrict__ qargs, const QueueRun* __restrict__ qruns,
-    int qnruns) {
-  const QueueTile qtile = queue_tile(qruns, qnruns);
-  [[maybe_unused]] const Blk qb = qtile.blk;
-  const typename colloc_centred_kernel_q<EXACT>::Args& qa = qargs[qtile.run];
-  GridD g = qa.g;
-  const double* __restrict__ bxf = queue_arg(qa.bxf);
-  const double* __restrict__ byf = queue_arg(qa.byf);
-  double* __restrict__ bxc = queue_arg(qa.bxc);
-  double* __restrict__ byc = queue_arg(qa.byc);
-#include "tiles/colloc_centred_kernel.inc"
-}
-template <bool EXACT>
-struct QueueTiles<colloc_centred_kernel_q<EXACT>> {
-  static constexpr auto kernel = &colloc_centred_kernel_queue<EXACT>;
-};
-
-// The admissible fraction of a stage candidate against its base
+// Collocated Bx/By of `u` on every padded cell (W faces; EXACT: correctly
+// rounded, the FP64 form; otherwise a fused multiply-add sum), and on the
+// interior cells the admissible fraction of a stage candidate against its base
 // (status.theta[slot]; with theta_both the other collocation into theta[3])
 // and the live-state preflights (admissibility under both collocations, the
-// relative div B residual) over the interior cells, from the collocated
-// field.  Each thread covers kRowsPerThread rows.
+// relative div B residual).  One pass: 8 planes read, 2 written.  At 2048^2 a
+// stage's collocation, ghost strips and checks as three kernels, the checks
+// reading the candidate and its base (16 planes) and bisecting with divisions
+// in every cell, took 262 us; now 106 us.  A division-free sign test decides
+// all but the cells at the edge of the admissible set; those read the base.
+template <bool EXACT, int W>
 __device__ __forceinline__ void prep_kernel_tile(
-    const Blk& qb, const GridD& g, const StateView& u, const double* __restrict__ bxc, const double* __restrict__ byc,
+    const Blk& qb, const GridD& g, const StateView& u, double* __restrict__ bxc, double* __restrict__ byc,
     const StateView& base, const double* __restrict__ base_bxc, const double* __restrict__ base_byc, int theta_slot,
     int theta_co, int theta_both, int live_checks, int solver_owned, StepStatus* __restrict__ status) {
 #include "tiles/prep_kernel.inc"
 }
 
-__global__ __launch_bounds__(256) void prep_kernel(GridD g, StateView u, const double* __restrict__ bxc,
-                                                   const double* __restrict__ byc, StateView base,
+template <bool EXACT, int W>
+__global__ __launch_bounds__(256) void prep_kernel(GridD g, StateView u, double* __restrict__ bxc,
+                                                   double* __restrict__ byc, StateView base,
                                                    const double* __restrict__ base_bxc,
                                                    const double* __restrict__ base_byc, int theta_slot,
                                                    int theta_co, int theta_both, int live_checks,
@@ -215,12 +165,13 @@ __global__ __launch_bounds__(256) void prep_kernel(GridD g, StateView u, const d
 }
 
 // Queue form of prep_kernel (one launch over the tiles of many runs).
+template <bool EXACT, int W>
 struct prep_kernel_q {
   struct Args {
     GridD g;
     StateView u;
-    const double* bxc;
-    const double* byc;
+    double* bxc;
+    double* byc;
     StateView base;
     const double* base_bxc;
     const double* base_byc;
@@ -232,12 +183,12 @@ struct prep_kernel_q {
     StepStatus* status;
   };
   static __device__ __forceinline__ void run(const Blk& qb, const Args& a) {
-    prep_kernel_tile(qb, queue_arg(a.g), queue_arg(a.u), queue_arg(a.bxc), queue_arg(a.byc), queue_arg(a.base),
+    prep_kernel_tile<EXACT, W>(qb, queue_arg(a.g), queue_arg(a.u), queue_arg(a.bxc), queue_arg(a.byc), queue_arg(a.base),
                      queue_arg(a.base_bxc), queue_arg(a.base_byc), queue_arg(a.theta_slot), queue_arg(a.theta_co),
                      queue_arg(a.theta_both), queue_arg(a.live_checks), queue_arg(a.solver_owned), queue_arg(a.status));
   }
   static void launch(dim3 grid, dim3 block, hipStream_t s, const Args& a) {
-    hipLaunchKernelGGL((prep_kernel), grid, block, 0, s, a.g, a.u, a.bxc, a.byc, a.base, a.base_bxc, a.base_byc,
+    hipLaunchKernelGGL((prep_kernel<EXACT, W>), grid, block, 0, s, a.g, a.u, a.bxc, a.byc, a.base, a.base_bxc, a.base_byc,
                        a.theta_slot, a.theta_co, a.theta_both, a.live_checks, a.solver_owned, a.status);
   }
   static const void* tag() {
@@ -248,15 +199,16 @@ struct prep_kernel_q {
 
 // prep_kernel over the tile queue, one workgroup per tile: the same text, the
 // arguments read from the tile's run record.
-__global__ __launch_bounds__(256) void prep_kernel_queue(const prep_kernel_q::Args* __restrict__ qargs,
-    const QueueRun* __restrict__ qruns, int qnruns) {
+template <bool EXACT, int W>
+__global__ __launch_bounds__(256) void prep_kernel_queue(
+    const typename prep_kernel_q<EXACT, W>::Args* __restrict__ qargs, const QueueRun* __restrict__ qruns, int qnruns) {
   const QueueTile qtile = queue_tile(qruns, qnruns);
   [[maybe_unused]] const Blk qb = qtile.blk;
-  const prep_kernel_q::Args& qa = qargs[qtile.run];
+  const typename prep_kernel_q<EXACT, W>::Args& qa = qargs[qtile.run];
   GridD g = qa.g;
   StateView u = queue_arg(qa.u);
-  const double* __restrict__ bxc = queue_arg(qa.bxc);
-  const double* __restrict__ byc = queue_arg(qa.byc);
+  double* __restrict__ bxc = queue_arg(qa.bxc);
+  double* __restrict__ byc = queue_arg(qa.byc);
   StateView base = queue_arg(qa.base);
   const double* __restrict__ base_bxc = queue_arg(qa.base_bxc);
   const double* __restrict__ base_byc = queue_arg(qa.base_byc);
@@ -268,65 +220,9 @@ __global__ __launch_bounds__(256) void prep_kernel_queue(const prep_kernel_q::Ar
   StepStatus* __restrict__ status = queue_arg(qa.status);
 #include "tiles/prep_kernel.inc"
 }
-template <>
-struct QueueTiles<prep_kernel_q> {
-  static constexpr auto kernel = &prep_kernel_queue;
-};
-
-// Collocation of the outer ghost layers: bx on the ng columns at each x end,
-// by on the ng rows at each y end (the one-sided closures live there).
-__device__ __forceinline__ void ghost_collocate_kernel_tile(
-    const Blk& qb, const GridD& g, const double* __restrict__ bxf, const double* __restrict__ byf,
-    double* __restrict__ bxc, double* __restrict__ byc) {
-#include "tiles/ghost_collocate_kernel.inc"
-}
-
-__global__ __launch_bounds__(256) void ghost_collocate_kernel(GridD g, const double* __restrict__ bxf,
-                                                              const double* __restrict__ byf,
-                                                              double* __restrict__ bxc, double* __restrict__ byc) {
-  [[maybe_unused]] const Blk qb = Blk::native();
-#include "tiles/ghost_collocate_kernel.inc"
-}
-
-// Queue form of ghost_collocate_kernel (one launch over the tiles of many runs).
-struct ghost_collocate_kernel_q {
-  struct Args {
-    GridD g;
-    const double* bxf;
-    const double* byf;
-    double* bxc;
-    double* byc;
-  };
-  static __device__ __forceinline__ void run(const Blk& qb, const Args& a) {
-    ghost_collocate_kernel_tile(qb, queue_arg(a.g), queue_arg(a.bxf), queue_arg(a.byf), queue_arg(a.bxc),
-                                queue_arg(a.byc));
-  }
-  static void launch(dim3 grid, dim3 block, hipStream_t s, const Args& a) {
-    hipLaunchKernelGGL((ghost_collocate_kernel), grid, block, 0, s, a.g, a.bxf, a.byf, a.bxc, a.byc);
-  }
-  static const void* tag() {
-    static const char t = 0;
-    return &t;
-  }
-};
-
-// ghost_collocate_kernel over the tile queue, one workgroup per tile: the same text, the
-// arguments read from the tile's run record.
-__global__ __launch_bounds__(256) void ghost_collocate_kernel_queue(
-    const ghost_collocate_kernel_q::Args* __restrict__ qargs, const QueueRun* __restrict__ qruns, int qnruns) {
-  const QueueTile qtile = queue_tile(qruns, qnruns);
-  [[maybe_unused]] const Blk qb = qtile.blk;
-  const ghost_collocate_kernel_q::Args& qa = qargs[qtile.run];
-  GridD g = qa.g;
-  const double* __restrict__ bxf = queue_arg(qa.bxf);
-  const double* __restrict__ byf = queue_arg(qa.byf);
-  double* __restrict__ bxc = queue_arg(qa.bxc);
-  double* __restrict__ byc = queue_arg(qa.byc);
-#include "tiles/ghost_collocate_kernel.inc"
-}
-template <>
-struct QueueTiles<ghost_collocate_kernel_q> {
-  static constexpr auto kernel = &ghost_collocate_kernel_queue;
+template <bool EXACT, int W>
+struct QueueTiles<prep_kernel_q<EXACT, W>> {
+  static constexpr auto kernel = &prep_kernel_queue<EXACT, W>;
 };
 
 // Stand-alone collocation (readback of bx/by and the launch-level ABI).
@@ -2229,18 +2125,21 @@ void launch_prep(const GridD& g, const StateView& u, double* bxc, double* byc, c
                  const double* base_bxc, const double* base_byc, int theta_slot, int theta_co, int theta_both,
                  int live_checks, int solver_owned, StepStatus* status, hipStream_t stream, bool exact) {
   const dim3 b(64, 4);
-  if (exact)
-    go<colloc_centred_kernel_q<true>>(blocks2d(g.nx + 2 * g.ng, g.ny + 2 * g.ng, b), b, stream, g, u.c[5], u.c[6], bxc,
-                                      byc);
+  const dim3 grid = blocks2d(g.nx + 2 * g.ng, g.ny + 2 * g.ng, b);
+  auto prep = [&](auto q) {
+    go<decltype(q)>(grid, b, stream, g, u, bxc, byc, base, base_bxc, base_byc, theta_slot, theta_co, theta_both,
+                    live_checks, solver_owned, status);
+  };
+  // The padded extents hold the halo's full window (2 ng + 1 cells at least).
+  auto by_form = [&](auto exact_q, auto fma_q) { exact ? prep(exact_q) : prep(fma_q); };
+  if (g.ng >= 4)
+    by_form(prep_kernel_q<true, 8>{}, prep_kernel_q<false, 8>{});
+  else if (g.ng == 3)
+    by_form(prep_kernel_q<true, 6>{}, prep_kernel_q<false, 6>{});
+  else if (g.ng == 2)
+    by_form(prep_kernel_q<true, 4>{}, prep_kernel_q<false, 4>{});
   else
-    go<colloc_centred_kernel_q<false>>(blocks2d(g.nx + 2 * g.ng, g.ny + 2 * g.ng, b), b, stream, g, u.c[5], u.c[6],
-                                       bxc, byc);
-  const int nghost = 2 * g.ng * (g.ny + 2 * g.ng) + 2 * g.ng * (g.nx + 2 * g.ng);
-  go<ghost_collocate_kernel_q>(dim3((nghost + 255) / 256), dim3(256), stream, g, u.c[5], u.c[6], bxc, byc);
-  if (theta_slot < 0 && !live_checks) return;
-  // prep_kernel's grid starts at padded cell -ng: interior threads only.
-  go<prep_kernel_q>(blocks2d(g.nx + 2 * g.ng, g.ny + 2 * g.ng, dim3(64, 4 * kRowsPerThread)), b, stream, g, u, bxc,
-                    byc, base, base_bxc, base_byc, theta_slot, theta_co, theta_both, live_checks, solver_owned, status);
+    by_form(prep_kernel_q<true, 2>{}, prep_kernel_q<false, 2>{});
 }
 
 void launch_collocate(const GridD& g, int axis, int co, const double* face, double* cell, hipStream_t stream) {
@@ -2259,7 +2158,9 @@ void launch_reconstruct(const GridD& g, int dir, int order, double gamma, const 
   const int slo = dir == 0 ? flags.side[0] : flags.side[2];
   const int shi = dir == 0 ? flags.side[1] : flags.side[3];
   const dim3 grid = blocks2d(lx, ly, b);
-  const dim3 fb_grid(64), fb_block(256);
+  // No more blocks than the list can fill: a queue batch launches every run's.
+  const std::size_t slots = (static_cast<std::size_t>(lx) * ly + 255) / 256;
+  const dim3 fb_block(256), fb_grid(static_cast<unsigned>(std::min<std::size_t>(64, slots)));
   const T gamma_t = T(gamma);
   auto faces = [&](auto q) {
     go<decltype(q)>(grid, b, stream, g, dir, gamma_t, slo, shi, u, bxc, byc, out, eq, fb_count, fb_list);
@@ -2306,7 +2207,8 @@ void launch_reconstruct_learned(const GridD& g, int dir, int order, double gamma
   const T gamma_t = T(gamma);
   // The plain list can hold a large share of the faces: enough blocks to fill
   // the device at the MP kernel's occupancy.
-  const dim3 list_grid(static_cast<unsigned>(list_blocks)), list_block(256);
+  const std::size_t slots = (static_cast<std::size_t>(lx) * ly + 255) / 256;
+  const dim3 list_block(256), list_grid(static_cast<unsigned>(std::min<std::size_t>(list_blocks, slots)));
   go<counter_pair_reset_kernel_q>(dim3(1), dim3(64), stream, fb_count, fb2_count);
   const dim3 cb(kCheapTiles[cheap_tile][0], kCheapTiles[cheap_tile][1]);
   auto cheap = [&](auto q) {
@@ -2321,7 +2223,7 @@ void launch_reconstruct_learned(const GridD& g, int dir, int order, double gamma
     default: cheap(cheap_reconstruct_kernel_q<T, kCheapTiles[4][0], kCheapTiles[4][1]>{}); break;
   }
   // The list holds at most the launch's faces.
-  const dim3 slot_grid(static_cast<unsigned>((static_cast<std::size_t>(lx) * ly + 255) / 256));
+  const dim3 slot_grid(static_cast<unsigned>(slots));
   const unsigned long long* list_count = fb_count;
   const unsigned long long* list = fb_list;
   auto listed = [&](auto q) {

@@ -97,156 +97,243 @@ __host__ __device__ __forceinline__ double cr_sum(const double* t) {
   return hi == 0.0 ? 0.0 : hi;
 }
 
-// Correctly rounded sum of N finite terms, certified fast path: the terms are
-// accumulated in double-double (Ogita-Rump-Oishi Sum2: s plus the exact
-// two-sum errors summed in e), whose distance from the exact sum is at most
-// (N-1)^2 eps^2 sum|t| (bounded here by 512 eps^2 sum|t|).  s + e = r + rr
-// exactly with r = fl(s + e); the exact sum lies within that bound of r + rr,
-// so r is its correctly rounded value whenever |rr| plus the bound stays below
-// half the spacing to r's neighbours (a quarter ulp when |r| is a power of
-// two, whose lower neighbour is half an ulp away).  Otherwise -- exact ties,
-// heavy cancellation, zero -- the full expansion decides.  Same value as
-// cr_sum<N>.
-template <int N>
-__host__ __device__ __forceinline__ double cr_sum_fast(const double* t) {
+// s + e = a + b exactly (Knuth's two-sum).
+__host__ __device__ __forceinline__ void two_sum(double a, double b, double& s, double& e) {
 #pragma clang fp contract(off)
-  double s = t[0], e = 0.0, mag = __builtin_fabs(t[0]);
+  s = a + b;
+  const double bv = s - a;
+  e = (a - (s - bv)) + (b - bv);
+}
+
+// Correctly rounded sum of the finite terms that each(f) hands to f, in four
+// chained accumulators: every two-sum error moves one accumulator down, so
+// only the last one rounds, 2^-159 of the running magnitude and below, and the
+// four are rounded from the top with cr_sum's half-even correction.  The rare
+// path behind certified_sum; its registers (cr_sum<16> keeps 16 partials) do
+// not grow with the number of terms.
+template <class E>
+__host__ __device__ __forceinline__ double cr_sum_chain(E each) {
+#pragma clang fp contract(off)
+  double c[4] = {0.0, 0.0, 0.0, 0.0};
+  each([&](double t) {
+    two_sum(c[0], t, c[0], t);
+    two_sum(c[1], t, c[1], t);
+    two_sum(c[2], t, c[2], t);
+    c[3] += t;
+  });
 #pragma unroll
-  for (int k = 1; k < N; ++k) {
-    const double a = s, b = t[k];
-    s = a + b;
-    const double bv = s - a;
-    e = e + ((a - (s - bv)) + (b - bv));
-    mag = mag + __builtin_fabs(b);
-  }
-  const double r = s + e;
-  const double bv = r - s;
-  const double rr = (s - (r - bv)) + (e - bv);
+  for (int pass = 0; pass < 3; ++pass)
+#pragma unroll
+    for (int q = 2; q >= 0; --q) two_sum(c[q], c[q + 1], c[q], c[q + 1]);
+  const double t[4] = {c[3], c[2], c[1], c[0]};
+  return cr_sum<4>(t);
+}
+
+// Whether s + e, within `bound` of the exact sum of terms whose magnitudes add
+// to mag, fixes its correctly rounded value r: the sum lies between
+// r + (rr - bound) and r + (rr + bound) with r + rr = s + e, so r is the
+// rounded value when both ends round to r.
+__host__ __device__ __forceinline__ bool certified_sum(double s, double e, double mag, double& r) {
+#pragma clang fp contract(off)
+  double rr;
+  two_sum(s, e, r, rr);
   const double eps = 2.220446049250313080847e-16;
   const double bound = 512.0 * eps * eps * mag;
-  if (r != 0.0 && __builtin_isfinite(r) && __builtin_isfinite(mag)) {
-    int ex;
-    const double mant = __builtin_frexp(r, &ex);  // |mant| in [0.5, 1), ulp(r) = 2^(ex-53)
-    const double half_gap = __builtin_ldexp(1.0, __builtin_fabs(mant) == 0.5 ? ex - 55 : ex - 54);
-    if (__builtin_fabs(rr) + bound < half_gap) return r;
+  if (mag == 0.0) {
+    r = 0.0;
+    return true;
   }
-  return cr_sum<N>(t);
+  return r != 0.0 && r + (rr + bound) == r && r + (rr - bound) == r;
 }
 
-// Integer-weight stencil sum_k w_k s_k / D with the numerator correctly rounded
-// from the error-free products (mhd_staggering.hpp:59-70): the value of the
-// reference's exact rational collocation.
+// a / b with the refined reciprocal y of b: the quotient's residual is exact,
+// so one correction rounds it (Markstein 1990).  Callers keep a, b and the
+// quotient away from the ends of the exponent range.  The host divides.
+__host__ __device__ __forceinline__ double quot(double a, double b, double y) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const double q = a * y;
+  return __builtin_fma(__builtin_fma(-b, q, a), y, q);
+#else
+  (void)y;
+  return a / b;
+#endif
+}
+
 template <int W>
-__host__ __device__ __forceinline__ double rational_stencil(const double* w, const double* s, double denom) {
+struct CentredRow;
+template <>
+struct CentredRow<8> {
+  static constexpr double w[8] = {-191.0, 1879.0, -9531.0, 68323.0, 68323.0, -9531.0, 1879.0, -191.0};
+  static constexpr double d = 120960.0;
+};
+template <>
+struct CentredRow<6> {
+  static constexpr double w[6] = {11.0, -93.0, 802.0, 802.0, -93.0, 11.0};
+  static constexpr double d = 1440.0;
+};
+template <>
+struct CentredRow<4> {
+  static constexpr double w[4] = {-1.0, 13.0, 13.0, -1.0};
+  static constexpr double d = 24.0;
+};
+template <>
+struct CentredRow<2> {
+  static constexpr double w[2] = {1.0, 1.0};
+  static constexpr double d = 2.0;
+};
+
+// Centred cell average sum_k w_k s_k / d with the numerator correctly rounded
+// (mhd_staggering.hpp:59-70): the value of the reference's exact rational
+// collocation.  The numerator is a compensated dot product (Ogita, Rump and
+// Oishi's Dot2: at most 64 eps^2/4 sum|w s| from the exact sum, bounded by
+// certified_sum's 512 eps^2); ties and heavy cancellation take the chain.
+template <int W>
+__host__ __device__ __forceinline__ double colloc_centred(const double* s) {
 #pragma clang fp contract(off)
-  bool finite = true;
+  using R = CentredRow<W>;
+  double sum = R::w[0] * s[0], e = __builtin_fma(R::w[0], s[0], -sum), mag = __builtin_fabs(sum);
 #pragma unroll
-  for (int k = 0; k < W; ++k) finite = finite && __builtin_isfinite(s[k]);
-  if (!finite) {
+  for (int k = 1; k < W; ++k) {
+    const double p = R::w[k] * s[k], lo = __builtin_fma(R::w[k], s[k], -p);
+    double t;
+    two_sum(sum, p, sum, t);
+    e = e + (t + lo);
+    mag = mag + __builtin_fabs(p);
+  }
+  if (!__builtin_isfinite(mag)) {
     double acc = 0.0;
 #pragma unroll
-    for (int k = 0; k < W; ++k) acc = acc + w[k] * s[k];
-    return acc / denom;
+    for (int k = 0; k < W; ++k) acc = acc + R::w[k] * s[k];
+    return acc / R::d;
   }
-  double t[2 * W];
+  double r;
+  if (!certified_sum(sum, e, mag, r))
+    r = cr_sum_chain([&](auto f) {
 #pragma unroll
-  for (int k = 0; k < W; ++k) {
-    const double hi = w[k] * s[k];
-    t[2 * k] = hi;
-    t[2 * k + 1] = fma(w[k], s[k], -hi);
-  }
-  return cr_sum_fast<2 * W>(t) / denom;
+      for (int k = 0; k < W; ++k) {
+        const double p = R::w[k] * s[k];
+        f(p);
+        f(__builtin_fma(R::w[k], s[k], -p));
+      }
+    });
+  // A numerator near the bottom of the exponent range leaves no exact residual.
+  return __builtin_fabs(r) < 0x1p-900 ? r / R::d : quot(r, R::d, 1.0 / R::d);
 }
 
-// Correctly rounded sum as cr_sum<N>, with the expansion compacted in a loop
-// (fsum's partials); for the rarely taken paths, where a small register
-// footprint matters more than speed.
-__host__ __device__ __noinline__ inline double cr_sum_loop(const double* t, int n) {
-#pragma clang fp contract(off)
-  double partials[40];
-  int np = 0;
-#pragma unroll 1
-  for (int k = 0; k < n; ++k) {
-    double x = t[k];
-    if (x == 0.0) continue;
-    int i = 0;
-#pragma unroll 1
-    for (int q = 0; q < np; ++q) {
-      double y = partials[q];
-      if (__builtin_fabs(x) < __builtin_fabs(y)) {
-        const double tmp = x;
-        x = y;
-        y = tmp;
-      }
-      const double hi = x + y;
-      const double lo = y - (hi - x);
-      if (lo != 0.0) partials[i++] = lo;
-      x = hi;
-    }
-    np = i;
-    partials[np++] = x;
-  }
-  if (np == 0) return 0.0;
-  int left = np;
-  double hi = partials[--left];
-  double lo = 0.0;
-#pragma unroll 1
-  while (left > 0) {
-    const double x = hi;
-    const double y = partials[--left];
-    hi = x + y;
-    lo = y - (hi - x);
-    if (lo != 0.0) break;
-  }
-  if (left > 0 && ((lo < 0.0 && partials[left - 1] < 0.0) || (lo > 0.0 && partials[left - 1] > 0.0))) {
-    const double y = lo * 2.0;
-    const double x = hi + y;
-    if (y == x - hi) hi = x;
-  }
-  return hi == 0.0 ? 0.0 : hi;
+// The centred rule as a plain fused multiply-add sum (the FP32 forms).
+template <int W>
+__host__ __device__ __forceinline__ double colloc_centred_fma(const double* s) {
+  using R = CentredRow<W>;
+  if (W == 2) return 0.5 * (s[0] + s[1]);
+  double acc = 0.0;
+#pragma unroll
+  for (int k = 0; k < W; ++k) acc = fma(R::w[k], s[k], acc);
+  return acc * (1.0 / R::d);
 }
 
 // One-sided closure of the outer ghost layers (mhd_staggering.hpp:111-173): the
 // 4-point Gauss integral over cell `rel` of the barycentric interpolant through
-// `width` consecutive faces, as a correctly rounded sum of the rounded
+// W consecutive faces, as a correctly rounded sum of the rounded
 // product-quotient terms ((w_q b_k) s_k / (x_q - k)) / den_q, den_q the
-// correctly rounded sum of b_k / (x_q - k).
-__host__ __device__ __noinline__ inline double one_sided_average(const double* s, int width, int rel) {
+// correctly rounded sum of b_k / (x_q - k).  den depends on (rel, q) alone and
+// is tabulated.  The 4 W terms are summed in double-double and certified; they
+// are formed again, by division, for the chain where that fails, so none is
+// stored.  (Formed
+// once, stored and expanded in registers with den summed on the device, the
+// two ghost strips took 28 us at any grid size, a quarter of a small step.)
+template <int W>
+__host__ __device__ __forceinline__ double one_sided_den(int rel, int q) {
+  static constexpr double den8[8][4] = {
+      {0x1.14f137d46e474p+4, 0x1.f8c80074d005bp+2, 0x1.e3d859725c52ap+3, 0x1.6ed7d2561d6f0p+6},
+      {-0x1.c0b0434cf8e66p+6, -0x1.3c6f3601b40bdp+5, -0x1.ca7f4af371dd1p+5, -0x1.20535ab48e7fep+8},
+      {0x1.41765e1bef6dap+8, 0x1.8104008bc977fp+6, 0x1.c9a41cf316120p+6, 0x1.f2c2483909587p+8},
+      {-0x1.02309860b4de3p+9, -0x1.0df8dc157721cp+7, -0x1.0df8dc157721cp+7, -0x1.02309860b4de3p+9},
+      {0x1.f2c248390954fp+8, 0x1.c9a41cf316120p+6, 0x1.8104008bc977fp+6, 0x1.41765e1bef6b8p+8},
+      {-0x1.20535ab48e7dcp+8, -0x1.ca7f4af371dd1p+5, -0x1.3c6f3601b40bdp+5, -0x1.c0b0434cf8e50p+6},
+      {0x1.6ed7d2561d6cfp+6, 0x1.e3d859725c52ep+3, 0x1.f8c80074d005ap+2, 0x1.14f137d46e463p+4},
+      {-0x1.824ee835b8992p+3, -0x1.61cd59d5b2438p+0, -0x1.5b7ffefc1a937p-2, -0x1.3659f02596131p-3}};
+  static constexpr double den6[6][4] = {
+      {0x1.0f05b79641acep+4, 0x1.c687647dc0f8ap+2, 0x1.84ad714acf13ap+3, 0x1.0cbe64ec6cd53p+6},
+      {-0x1.38625562bca1bp+6, -0x1.8efd9d3fa7e1bp+4, -0x1.f7e3664b456ffp+4, -0x1.1b3dd70cc1219p+7},
+      {0x1.28a9afe25a02dp+7, 0x1.3a39774832ef3p+5, 0x1.3a39774832ef3p+5, 0x1.28a9afe25a02dp+7},
+      {-0x1.1b3dd70cc1219p+7, -0x1.f7e3664b456ffp+4, -0x1.8efd9d3fa7e1bp+4, -0x1.38625562bca2ap+6},
+      {0x1.0cbe64ec6cd3bp+6, 0x1.84ad714acf13dp+3, 0x1.c687647dc0f89p+2, 0x1.0f05b79641abep+4},
+      {-0x1.8aa796fef0833p+3, -0x1.86dbe50cf3676p+0, -0x1.a7472137ee67cp-2, -0x1.96243e36dcae5p-3}};
+  static constexpr double den4[4][4] = {
+      {0x1.069ea7d427ea4p+4, 0x1.858123c63e0bcp+2, 0x1.18376dbf83e1fp+3, 0x1.4faeffb4b3380p+5},
+      {-0x1.67d435f5506d8p+5, -0x1.86f6eebf146a6p+3, -0x1.86f6eebf146a6p+3, -0x1.67d435f5506ecp+5},
+      {0x1.4faeffb4b338ap+5, 0x1.18376dbf83e21p+3, 0x1.858123c63e0bcp+2, 0x1.069ea7d427eadp+4},
+      {-0x1.97149b513699cp+3, -0x1.c30812c3758b4p+0, -0x1.18327f9fd4d54p-1, -0x1.28e67e0075ea1p-2}};
+  static constexpr double den2[2][4] = {
+      {0x1.ef456e91b52c8p+3, 0x1.217522dc95a71p+2, 0x1.217522dc95a71p+2, 0x1.ef456e91b52cep+3},
+      {-0x1.aef610ccf8cefp+3, -0x1.23a0b30a91550p+1, -0x1.c999f1fda6dfap-1, -0x1.1cfe9e4de8eeep-1}};
+  if constexpr (W == 8) return den8[rel][q];
+  if constexpr (W == 6) return den6[rel][q];
+  if constexpr (W == 4) return den4[rel][q];
+  return den2[rel][q];
+}
+
+template <int W, bool DIVIDE, class F>
+__host__ __device__ __forceinline__ void one_sided_terms(const double* s, int rel, F f) {
 #pragma clang fp contract(off)
-  const double xq[4] = {0.0694318442029737124, 0.3300094782075718676, 0.6699905217924281324,
-                        0.9305681557970262876};
-  const double wq[4] = {0.1739274225687269287, 0.3260725774312730713, 0.3260725774312730713,
-                        0.1739274225687269287};
-  double bary[8];
-  double c = 1.0;  // (-1)^k C(width-1, k), exact small integers
-#pragma unroll 1
-  for (int k = 0; k < width; ++k) {
-    bary[k] = (k % 2 == 0) ? c : -c;
-    c = c * double(width - 1 - k) / double(k + 1);
-  }
-  bool finite = true;
-#pragma unroll 1
-  for (int k = 0; k < width; ++k) finite = finite && __builtin_isfinite(s[k]);
-  double terms[32];
-  int n = 0;
-#pragma unroll 1
+  constexpr double xq[4] = {0.0694318442029737124, 0.3300094782075718676, 0.6699905217924281324,
+                            0.9305681557970262876};
+  constexpr double wq[2] = {0.1739274225687269287, 0.3260725774312730713};
+#pragma nounroll
   for (int q = 0; q < 4; ++q) {
-    const double x = double(rel) + xq[q];
-    double dt[8];
-#pragma unroll 1
-    for (int k = 0; k < width; ++k) dt[k] = bary[k] / (x - double(k));
-    const double den = cr_sum_loop(dt, width);
-    const double wscaled = wq[q] / 1.0;
-#pragma unroll 1
-    for (int k = 0; k < width; ++k) terms[n++] = (((wscaled * bary[k]) * s[k]) / (x - double(k))) / den;
+    const double x = double(rel) + (q < 2 ? (q == 0 ? xq[0] : xq[1]) : (q == 2 ? xq[2] : xq[3]));
+    const double wn = (q == 0 || q == 3) ? wq[0] : wq[1];
+    const double den = one_sided_den<W>(rel, q), iden = frcp(den);
+    double c = 1.0;  // (-1)^k C(W-1, k), exact small integers
+#pragma unroll
+    for (int k = 0; k < W; ++k) {
+      const double xk = x - double(k);
+      const double a = (wn * ((k % 2 == 0) ? c : -c)) * s[k];
+      f(DIVIDE ? (a / xk) / den : quot(quot(a, xk, frcp(xk)), den, iden));
+      c = c * double(W - 1 - k) / double(k + 1);
+    }
   }
-  if (!finite) {
-    double acc = 0.0;
-#pragma unroll 1
-    for (int k = 0; k < n; ++k) acc = acc + terms[k];
-    return acc;
-  }
-  return cr_sum_loop(terms, n);
+}
+
+template <int W>
+__host__ __device__ __forceinline__ double one_sided(const double* s, int rel) {
+#pragma clang fp contract(off)
+  bool zero = true;
+#pragma unroll
+  for (int k = 0; k < W; ++k) zero = zero && s[k] == 0.0;
+  if (zero) return 0.0;
+  double sum = 0.0, e = 0.0, mag = 0.0, plain = 0.0;
+  one_sided_terms<W, false>(s, rel, [&](double t) {
+    double lo;
+    two_sum(sum, t, sum, lo);
+    e = e + lo;
+    mag = mag + __builtin_fabs(t);
+    plain = plain + t;
+  });
+  if (!__builtin_isfinite(mag)) return plain;
+  // Quotients near the bottom of the exponent range have no exact residual:
+  // they are divided.
+  double r;
+  if (!certified_sum(sum, e, mag, r) || mag < 0x1p-900)
+    r = cr_sum_chain([&](auto f) { one_sided_terms<W, true>(s, rel, f); });
+  return r;
+}
+
+// First face of the W-face window of padded cell `cell` (faces and cells
+// lo .. hi of the line): centred, moved inside the line at its ends.
+template <int W>
+__host__ __device__ __forceinline__ int colloc_start(int cell, int lo, int hi) {
+  int start = cell - (W / 2 - 1);
+  start = start < lo ? lo : start;
+  return start + W - 1 > hi ? hi - W + 1 : start;
+}
+
+// Cell average from the window's faces s, the cell `rel` faces after its first
+// face: the centred rule, or the one-sided closure where the window was moved.
+template <int W, bool EXACT>
+__host__ __device__ __forceinline__ double colloc_window(const double* s, int rel) {
+  if (rel == W / 2 - 1) return EXACT ? colloc_centred<W>(s) : colloc_centred_fma<W>(s);
+  return one_sided<W>(s, rel);
 }
 
 // Learned form: a face normal to `dir` (x faces dir 0, y faces dir 1) is
@@ -276,173 +363,30 @@ __host__ __device__ __forceinline__ bool face_states_read_back(const GridD& g, i
   return any != 0;
 }
 
-// Centred high-order cell average (8/6/4/2 taps) when the centred stencil
-// lies inside the padded grid (every interior cell); false in the outer ghost
-// layers, whose values need the one-sided closure.
-__host__ __device__ __forceinline__ bool face_to_cell_centred(const GridD& g, const double* f, int axis, int cell,
-                                                              int fixed, double& out) {
-  const int n = axis == 0 ? g.nx : g.ny;
-  const int width = colloc_width(n + 2 * g.ng, g.ng);
-  const int lo = -g.ng, hi = n + g.ng - 1;
-  if (width == 1) {
-    out = axis_face(g, f, axis, cell, fixed);
-    return true;
-  }
-  const int start_c = cell - (width / 2 - 1);
-  // The window's samples are read before the range test (from a window moved
-  // inside the grid when the test fails), so they need not wait behind it.
-  const bool inside = start_c >= lo && start_c + width - 1 <= hi;
-  const int s0 = inside ? start_c : lo;
-  double s[8];
-#pragma unroll
-  for (int k = 0; k < 8; ++k) s[k] = k < width ? axis_face(g, f, axis, s0 + k, fixed) : 0.0;
-  if (!inside) return false;
-  if (width == 8) {
-    const double w[8] = {-191.0, 1879.0, -9531.0, 68323.0, 68323.0, -9531.0, 1879.0, -191.0};
-    out = rational_stencil<8>(w, s, 120960.0);
-  } else if (width == 6) {
-    const double w[6] = {11.0, -93.0, 802.0, 802.0, -93.0, 11.0};
-    out = rational_stencil<6>(w, s, 1440.0);
-  } else if (width == 4) {
-    const double w[4] = {-1.0, 13.0, 13.0, -1.0};
-    out = rational_stencil<4>(w, s, 24.0);
-  } else {
-    const double w[2] = {1.0, 1.0};
-    out = rational_stencil<2>(w, s, 2.0);
-  }
-  return true;
-}
-
-// The centred rule of face_to_cell_centred with a plain fused multiply-add
-// sum (the FP32 forms' collocation: not correctly rounded).
-__host__ __device__ __forceinline__ bool face_to_cell_centred_fma(const GridD& g, const double* f, int axis, int cell,
-                                                                  int fixed, double& out) {
-  const int n = axis == 0 ? g.nx : g.ny;
-  const int width = colloc_width(n + 2 * g.ng, g.ng);
-  const int lo = -g.ng, hi = n + g.ng - 1;
-  if (width == 1) {
-    out = axis_face(g, f, axis, cell, fixed);
-    return true;
-  }
-  const int start_c = cell - (width / 2 - 1);
-  // As face_to_cell_centred: the samples are read before the range test.
-  const bool inside = start_c >= lo && start_c + width - 1 <= hi;
-  const int s0 = inside ? start_c : lo;
-  double x[8];
-#pragma unroll
-  for (int k = 0; k < 8; ++k) x[k] = k < width ? axis_face(g, f, axis, s0 + k, fixed) : 0.0;
-  if (!inside) return false;
-  double acc = 0.0;
-  if (width == 8) {
-    const double w[8] = {-191.0, 1879.0, -9531.0, 68323.0, 68323.0, -9531.0, 1879.0, -191.0};
-#pragma unroll
-    for (int k = 0; k < 8; ++k) acc = fma(w[k], x[k], acc);
-    out = acc * (1.0 / 120960.0);
-  } else if (width == 6) {
-    const double w[6] = {11.0, -93.0, 802.0, 802.0, -93.0, 11.0};
-#pragma unroll
-    for (int k = 0; k < 6; ++k) acc = fma(w[k], x[k], acc);
-    out = acc * (1.0 / 1440.0);
-  } else if (width == 4) {
-    const double w[4] = {-1.0, 13.0, 13.0, -1.0};
-#pragma unroll
-    for (int k = 0; k < 4; ++k) acc = fma(w[k], x[k], acc);
-    out = acc * (1.0 / 24.0);
-  } else {
-    out = 0.5 * (x[0] + x[1]);
-  }
-  return true;
-}
-
-// The one-sided closure of width W with the expansion kept in registers (the
-// same correctly rounded value as one_sided_average); for the ghost-layer
-// kernel, where register use does not limit anything else.
-template <int W>
-__host__ __device__ __forceinline__ double one_sided_unrolled(const double* s, int rel) {
-#pragma clang fp contract(off)
-  const double xq[4] = {0.0694318442029737124, 0.3300094782075718676, 0.6699905217924281324,
-                        0.9305681557970262876};
-  const double wq[4] = {0.1739274225687269287, 0.3260725774312730713, 0.3260725774312730713,
-                        0.1739274225687269287};
-  double bary[W];
-  double c = 1.0;
-#pragma unroll
-  for (int k = 0; k < W; ++k) {
-    bary[k] = (k % 2 == 0) ? c : -c;
-    c = c * double(W - 1 - k) / double(k + 1);
-  }
-  bool finite = true;
-#pragma unroll
-  for (int k = 0; k < W; ++k) finite = finite && __builtin_isfinite(s[k]);
-  double terms[4 * W];
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const double x = double(rel) + xq[q];
-    double dt[W];
-#pragma unroll
-    for (int k = 0; k < W; ++k) dt[k] = bary[k] / (x - double(k));
-    const double den = cr_sum<W>(dt);
-    const double wscaled = wq[q] / 1.0;
-#pragma unroll
-    for (int k = 0; k < W; ++k) terms[q * W + k] = (((wscaled * bary[k]) * s[k]) / (x - double(k))) / den;
-  }
-  if (!finite) {
-    double acc = 0.0;
-#pragma unroll
-    for (int k = 0; k < 4 * W; ++k) acc = acc + terms[k];
-    return acc;
-  }
-  return cr_sum<4 * W>(terms);
-}
-
-// face_to_cell with the register-resident one-sided closures.
-__host__ __device__ inline double face_to_cell_ghost(const GridD& g, const double* f, int axis, int cell, int fixed) {
-  double v;
-  if (face_to_cell_centred(g, f, axis, cell, fixed, v)) return v;
-  const int n = axis == 0 ? g.nx : g.ny;
-  const int width = colloc_width(n + 2 * g.ng, g.ng);
-  const int lo = -g.ng, hi = n + g.ng - 1;
-  int start = cell - (width / 2 - 1);
-  if (start < lo) start = lo;
-  if (start + width - 1 > hi) start = hi - width + 1;
-  double s[8];
-  for (int k = 0; k < width; ++k) s[k] = axis_face(g, f, axis, start + k, fixed);
-  if (width == 8) return one_sided_unrolled<8>(s, cell - start);
-  if (width == 6) return one_sided_unrolled<6>(s, cell - start);
-  if (width == 4) return one_sided_unrolled<4>(s, cell - start);
-  return one_sided_unrolled<2>(s, cell - start);
-}
-
 // High-order cell average (8/6/4/2 taps, one-sided closures in the outer
 // ghosts), mhd_staggering.hpp:175-236.
-__host__ __device__ inline double face_to_cell(const GridD& g, const double* f, int axis, int cell, int fixed) {
+template <int W>
+__host__ __device__ __forceinline__ double face_to_cell_w(const GridD& g, const double* f, int axis, int cell, int fixed) {
   const int n = axis == 0 ? g.nx : g.ny;
-  const int width = colloc_width(n + 2 * g.ng, g.ng);
-  const int lo = -g.ng, hi = n + g.ng - 1;
-  if (width == 1) return axis_face(g, f, axis, cell, fixed);
-  const int start_c = cell - (width / 2 - 1);
-  double s[8];
-  if (start_c >= lo && start_c + width - 1 <= hi) {
-    for (int k = 0; k < width; ++k) s[k] = axis_face(g, f, axis, start_c + k, fixed);
-    if (width == 8) {
-      const double w[8] = {-191.0, 1879.0, -9531.0, 68323.0, 68323.0, -9531.0, 1879.0, -191.0};
-      return rational_stencil<8>(w, s, 120960.0);
-    }
-    if (width == 6) {
-      const double w[6] = {11.0, -93.0, 802.0, 802.0, -93.0, 11.0};
-      return rational_stencil<6>(w, s, 1440.0);
-    }
-    if (width == 4) {
-      const double w[4] = {-1.0, 13.0, 13.0, -1.0};
-      return rational_stencil<4>(w, s, 24.0);
-    }
-    const double w[2] = {1.0, 1.0};
-    return rational_stencil<2>(w, s, 2.0);
-  }
-  int start = start_c < lo ? lo : start_c;
-  if (start + width - 1 > hi) start = hi - width + 1;
-  for (int k = 0; k < width; ++k) s[k] = axis_face(g, f, axis, start + k, fixed);
-  return one_sided_average(s, width, cell - start);
+  const int start = colloc_start<W>(cell, -g.ng, n + g.ng - 1);
+  double s[W];
+#pragma unroll
+  for (int k = 0; k < W; ++k) s[k] = axis_face(g, f, axis, start + k, fixed);
+  return colloc_window<W, true>(s, cell - start);
+}
+
+__host__ __device__ inline double face_to_cell(const GridD& g, const double* f, int axis, int cell, int fixed) {
+  const int width = colloc_width((axis == 0 ? g.nx : g.ny) + 2 * g.ng, g.ng);
+  if (width == 8) return face_to_cell_w<8>(g, f, axis, cell, fixed);
+  if (width == 6) return face_to_cell_w<6>(g, f, axis, cell, fixed);
+  if (width == 4) return face_to_cell_w<4>(g, f, axis, cell, fixed);
+  if (width == 2) return face_to_cell_w<2>(g, f, axis, cell, fixed);
+  return axis_face(g, f, axis, cell, fixed);
+}
+
+// The same value (every padded cell takes one rule).
+__host__ __device__ inline double face_to_cell_ghost(const GridD& g, const double* f, int axis, int cell, int fixed) {
+  return face_to_cell(g, f, axis, cell, fixed);
 }
 
 // First-order (two bounding faces) cell average used by the low-order retry.
@@ -452,8 +396,7 @@ __host__ __device__ __forceinline__ double face_to_cell_lo(const GridD& g, const
   if (cell >= n + g.ng - 1) return a;
   const double b = axis_face(g, f, axis, cell + 1, fixed);
   const double s[2] = {a, b};
-  const double w[2] = {1.0, 1.0};
-  return rational_stencil<2>(w, s, 2.0);
+  return colloc_centred<2>(s);
 }
 
 // ---------------------------------------------------------------------------
