@@ -11,6 +11,7 @@
 // readbacks are byte compatible.  State planes are FP64; interface states and
 // fluxes are of the kernel's arithmetic type T.
 
+#include "qmhd_face.hpp"
 #include "qmhd_kernels.hpp"
 #include "qmhd_queue.hpp"
 #include "qmhd_stencil.hpp"
@@ -354,8 +355,7 @@ struct QueueTiles<reconstruct_kernel_q<T, ORDER>> {
 };
 
 // Learned form: the characteristic MP states of the faces on the cheap
-// reconstruction's list (one thread per list slot, the grid sized for the
-// longest list); a face whose MP states (or their normal-field update) are not
+// reconstruction's list (a bounded grid strides over the list); a face whose MP states (or their normal-field update) are not
 // admissible goes on the second list, for the full fallback chain.
 template <class T, int ORDER>
 __device__ __forceinline__ void reconstruct_list_kernel_tile(
@@ -733,24 +733,6 @@ struct QueueTiles<cheap_reconstruct_kernel_q<T, TX, TY>> {
 // ---------------------------------------------------------------------------
 // Face flux with transverse Gauss quadrature and the CFL face rate.
 
-// LF: the order-1 Lax-Friedrichs flux (a launch parameter, resolved at
-// compile time so an HLLD kernel carries no other solver); cheap: the learned
-// form's HLL flux (Davis speeds); otherwise HLLD.  irL, irR: 1/rho of the two
-// states (rotation leaves rho in place).
-template <bool LF, class T>
-__device__ __forceinline__ St<T> riemann(const St<T>& L, T irL, const St<T>& R, T irR, int dir, T gamma,
-                                         bool cheap = false) {
-  const St<T> lr = rot(L, dir), rr = rot(R, dir);
-  St<T> f;
-  if (LF)
-    f = lf_flux(lr, rr, irL, irR, gamma);
-  else if (cheap)
-    f = hll_davis_flux(lr, rr, irL, irR, gamma);
-  else
-    f = hlld_flux(lr, rr, irL, irR, gamma);
-  return rot(f, dir);
-}
-
 // |v_n| and c_fast of one face state (1/rho supplied) in the direction
 // `dir`; infinite when the state is not admissible.
 template <class T>
@@ -791,138 +773,43 @@ __device__ __forceinline__ T face_speed(const St<T>& L, T irL, const St<T>& R, T
 
 // The learned form's flux of a face whose two cells the indicator left
 // unflagged: one HLL flux (Davis speeds) at its face-average states, the rate
-// from those states.  flux_face and the cheap-face kernel share it, so both
-// give the same bits.
+// from those states.  The plain list's flux and the cheap-face kernel share
+// it, so both give the same bits.
 template <class T, int ORDER>
 __device__ __forceinline__ void cheap_face_flux(const St<T>& baseL, const St<T>& baseR, int dir, T gamma, St<T>& f,
                                                 T& smax) {
   const T irL = frcp(baseL.rho), irR = frcp(baseR.rho);
   smax = face_speed(baseL, irL, baseR, irR, dir, ORDER, gamma);
-  f = riemann<false>(baseL, irL, baseR, irR, dir, gamma, true);
+  f = rot(hll_davis_flux(rot(baseL, dir), rot(baseR, dir), irL, irR, gamma), dir);
 }
 
-// Face flux and face rate (0.5 * signal speed / spacing) of face ko.
+// Face flux and, with a rate plane, the face rate (0.5 * signal speed /
+// spacing) of face ko.
 template <class T>
 __device__ __forceinline__ void store_face(const GridD& g, int dir, const FluxView<T>& flux, double* __restrict__ rate,
                                            std::size_t ko, const St<T>& f, T smax) {
 #pragma unroll
   for (int c = 0; c < 8; ++c) flux.c[c][ko] = comp(f, c);
+  if (!rate) return;
   const double sp = static_cast<double>(smax);
   const double spacing = dir == 0 ? g.dx : g.dy;
   rate[ko] = (fin(sp) && sp >= 0.0) ? (sp * 0.5) / spacing : Lim<double>::inf();
 }
 
-// One thread per face in [0,nx] x [0,ny].  Writes the face flux (F_n of the
-// normal field is zero), and the face signal speed max(|v_n|)+max(c_f) over
-// the face average and every Gauss point, scaled by 0.5/spacing.  (The
-// learned form's unflagged faces take cheap_face_flux instead, in the cheap
-// reconstruction or, for faces whose cheap states were inadmissible, in
-// flux_plain_list_kernel.)
-template <class T, int ORDER, bool LF>
-__device__ __forceinline__ void flux_face(const GridD& g, int dir, int periodic_dir, T gamma,
-                                          const IfaceView<T>& in, const FluxView<T>& flux, double* __restrict__ rate,
-                                          int i, int j) {
-  int si = i, sj = j;
-  if (periodic_dir) {
-    if (dir == 0 && i == g.nx) si = 0;
-    if (dir == 1 && j == g.ny) sj = 0;
-  }
-  const std::size_t ko = idx(g, i, j);
-  const std::size_t k = idx(g, si, sj);
-  St<T> baseL, baseR;
-#pragma unroll
-  for (int c = 0; c < 8; ++c) {
-    set_comp(baseL, c, in.c[c][k]);
-    set_comp(baseR, c, in.c[8 + c][k]);
-  }
-  St<T> f;
-  // One reciprocal of rho per state, shared by its admissibility test, its
-  // signal speed and its Riemann solve.
-  const T ibL = frcp(baseL.rho), ibR = frcp(baseR.rho);
-  T smax = face_speed(baseL, ibL, baseR, ibR, dir, ORDER, gamma);
-  if (ORDER != 5 && ORDER != 7) {
-    f = riemann<LF>(baseL, ibL, baseR, ibR, dir, gamma);
-  } else {
-    constexpr int H = ORDER == 5 ? 2 : 3;
-    constexpr int NQ = ORDER == 5 ? 3 : 4;
-    const std::size_t step = dir == 0 ? static_cast<std::size_t>(g.pitch) : 1;
-    // Recover the point states at the Gauss nodes from 2H+1 face averages.
-    St<T> pl[NQ], pr[NQ];
-#pragma unroll
-    for (int c = 0; c < 16; ++c) {
-      T s[2 * H + 1];
-#pragma unroll
-      for (int t = 0; t < 2 * H + 1; ++t) s[t] = in.c[c][k + (t - H) * step];
-      bool constant = true;
-#pragma unroll
-      for (int t = 0; t < 2 * H + 1; ++t) constant = constant && s[t] == s[H];
-#pragma unroll
-      for (int q = 0; q < NQ; ++q) {
-        T v = s[H];
-        if (!constant) {
-          v = T(0);
-#pragma unroll
-          for (int t = 0; t < 2 * H + 1; ++t)
-            v += T(ORDER == 5 ? c_rows.mp5_point[q][t] : c_rows.mp7_point[q][t]) * s[t];
-        }
-        if (c < 8)
-          set_comp(pl[q], c, v);
-        else
-          set_comp(pr[q], c - 8, v);
-      }
-    }
-    bool ok = true;
-    int first_bad = NQ;
-    T irl[NQ], irr[NQ];
-#pragma unroll
-    for (int q = 0; q < NQ; ++q) {
-      irl[q] = frcp(pl[q].rho);
-      irr[q] = frcp(pr[q].rho);
-      const bool good = admissible_state_ir(pl[q], irl[q], gamma) && admissible_state_ir(pr[q], irr[q], gamma);
-      if (!good && first_bad == NQ) first_bad = q;
-      ok = ok && good;
-    }
-    // Rate: the face average plus every point before the first inadmissible one.
-#pragma unroll
-    for (int q = 0; q < NQ; ++q)
-      if (q < first_bad) smax = fmax(smax, face_speed(pl[q], irl[q], pr[q], irr[q], dir, ORDER, gamma));
-    // Gauss average of the point fluxes, accumulated point by point in the
-    // same summation order, with the exact constant-flux shortcut (all point
-    // fluxes equal -> that flux) tracked as a running flag.  With an
-    // inadmissible point the face takes the flux of its face averages: one
-    // pass of the same loop at weight 1 (w * v = v exactly), so the kernel
-    // holds one solver per node and no separate one for that case.
-    if (!ok) {
-      pl[0] = baseL;
-      pr[0] = baseR;
-      irl[0] = ibL;
-      irr[0] = ibR;
-    }
-    T acc[8], first[8];
-    bool same[8];
-#pragma unroll
-    for (int q = 0; q < NQ; ++q) {
-      if (q > 0 && !ok) break;
-      const St<T> fq = riemann<LF>(pl[q], irl[q], pr[q], irr[q], dir, gamma);
-      const T w = ok ? T(ORDER == 5 ? c_rows.mp5_gauss[q] : c_rows.mp7_gauss[q]) : T(1);
-#pragma unroll
-      for (int c = 0; c < 8; ++c) {
-        const T v = comp(fq, c);
-        if (q == 0) {
-          first[c] = v;
-          same[c] = v == v;
-          acc[c] = w * v;
-        } else {
-          same[c] = same[c] && v == first[c];
-          acc[c] += w * v;
-        }
-      }
-    }
-#pragma unroll
-    for (int c = 0; c < 8; ++c) set_comp(f, c, same[c] ? first[c] : acc[c]);
-  }
-  store_face(g, dir, flux, rate, ko, f, smax);
-}
+// Flux and, with a rate plane, the signal speed max(|v_n|) + max(c_f) over the
+// face average and every Gauss point, scaled by 0.5/spacing, of the faces
+// [0,nx] x [0,ny], one thread each.  (The learned form's unflagged faces take
+// cheap_face_flux instead.)  MP5/MP7: qmhd_face.hpp's node loop over the
+// block's neighbour differences in LDS.  The tiles keep the differences under
+// 43 KB in FP64 and give every half-wave 32 consecutive LDS words: 16 x 16 for
+// x faces (lines along y), 32 x 8 for y faces.  2048^2 FP64,
+// x / y faces: 955 / 861 us with one unrolled solve per node and the samples
+// read from global memory (238 VGPRs, 5.7k VALU instructions a face), 553 / 535
+// us now with the rate and 540 / 519 us without (219 / 243 VGPRs, about 3.3k),
+// both at two waves per SIMD; forced to three it spills 22 VGPRs and takes 819
+// / 795 us.  In the hardware's tile order the x faces take 565 us.
+constexpr int kFluxTiles[2][2] = {{16, 16}, {32, 8}};
+constexpr int kFluxListBlock = 64;
 
 // One instantiation per direction: the direction's component swaps and
 // stencil stride fold at compile time.
@@ -936,7 +823,7 @@ __device__ __forceinline__ void flux_kernel_tile(
 template <class T, int ORDER, bool LF, int DIR>
 __global__ __launch_bounds__(256) void flux_kernel(GridD g, int periodic_dir, T gamma, IfaceView<T> in,
                                                    FluxView<T> flux, double* __restrict__ rate) {
-  [[maybe_unused]] const Blk qb = Blk::native();
+  [[maybe_unused]] const Blk qb = ORDER >= 5 ? Blk::xcd_tiled() : Blk::native();
 #include "tiles/flux_kernel.inc"
 }
 
@@ -992,8 +879,9 @@ struct QueueTiles<flux_kernel_q<T, ORDER, LF, DIR>> {
 // the launch (plain flux) and the unflagged faces whose cheap states were
 // inadmissible (the cheap flux of their plain states); the cheap
 // reconstruction stored every other face's flux.  Ghost-row entries are
-// skipped; a periodic high face takes its low partner's flux.  One thread per
-// list slot, the grid sized for the longest list.
+// skipped; a periodic high face takes its low partner's flux.  A bounded grid
+// strides over the list; one wave per block, its lanes' neighbour differences
+// in LDS (24 KB in FP32).
 template <class T, int ORDER, int DIR>
 __device__ __forceinline__ void flux_plain_list_kernel_tile(const Blk& qb, const GridD& g, int periodic_dir, T gamma,
                                                               const IfaceView<T>& in, const FluxView<T>& flux,
@@ -1005,7 +893,7 @@ __device__ __forceinline__ void flux_plain_list_kernel_tile(const Blk& qb, const
 }
 
 template <class T, int ORDER, int DIR>
-__global__ __launch_bounds__(256) void flux_plain_list_kernel(GridD g, int periodic_dir, T gamma,
+__global__ __launch_bounds__(kFluxListBlock) void flux_plain_list_kernel(GridD g, int periodic_dir, T gamma,
                                                               IfaceView<T> in, FluxView<T> flux,
                                                               double* __restrict__ rate,
                                                               const uint8_t* __restrict__ cell_flags,
@@ -1047,7 +935,7 @@ struct flux_plain_list_kernel_q {
 // flux_plain_list_kernel over the tile queue, one workgroup per tile: the same text, the
 // arguments read from the tile's run record.
 template <class T, int ORDER, int DIR>
-__global__ __launch_bounds__(256) void flux_plain_list_kernel_queue(
+__global__ __launch_bounds__(kFluxListBlock) void flux_plain_list_kernel_queue(
     const typename flux_plain_list_kernel_q<T, ORDER, DIR>::Args* __restrict__ qargs,
     const QueueRun* __restrict__ qruns, int qnruns) {
   const QueueTile qtile = queue_tile(qruns, qnruns);
@@ -2205,8 +2093,9 @@ void launch_reconstruct_learned(const GridD& g, int dir, int order, double gamma
   const int slo = dir == 0 ? flags.side[0] : flags.side[2];
   const int shi = dir == 0 ? flags.side[1] : flags.side[3];
   const T gamma_t = T(gamma);
-  // The plain list can hold a large share of the faces: enough blocks to fill
-  // the device at the MP kernel's occupancy.
+  // Enough blocks to fill the device at the MP kernel's occupancy (the plain
+  // list can hold a large share of the faces), no more than the list can fill:
+  // one block per possible slot spent 25 us at 4096^2 on blocks without work.
   const std::size_t slots = (static_cast<std::size_t>(lx) * ly + 255) / 256;
   const dim3 list_block(256), list_grid(static_cast<unsigned>(std::min<std::size_t>(list_blocks, slots)));
   go<counter_pair_reset_kernel_q>(dim3(1), dim3(64), stream, fb_count, fb2_count);
@@ -2222,12 +2111,10 @@ void launch_reconstruct_learned(const GridD& g, int dir, int order, double gamma
     case 3: cheap(cheap_reconstruct_kernel_q<T, kCheapTiles[3][0], kCheapTiles[3][1]>{}); break;
     default: cheap(cheap_reconstruct_kernel_q<T, kCheapTiles[4][0], kCheapTiles[4][1]>{}); break;
   }
-  // The list holds at most the launch's faces.
-  const dim3 slot_grid(static_cast<unsigned>(slots));
   const unsigned long long* list_count = fb_count;
   const unsigned long long* list = fb_list;
   auto listed = [&](auto q) {
-    go<decltype(q)>(slot_grid, list_block, stream, g, dir, gamma_t, u, bxc, byc, out, eq, list_count, list, fb2_count,
+    go<decltype(q)>(list_grid, list_block, stream, g, dir, gamma_t, u, bxc, byc, out, eq, list_count, list, fb2_count,
                     fb2_list, plain_total);
   };
   const unsigned long long* fb2c = fb2_count;
@@ -2249,6 +2136,7 @@ void launch_flux(const GridD& g, int dir, int order, int hll_only, const Flags4&
                  const IfaceView<T>& in, const FluxView<T>& flux, double* rate, hipStream_t stream,
                  dim3 b) {
   const T gm = T(gamma);
+  if (order == 5 || order == 7) b = dim3(kFluxTiles[dir][0], kFluxTiles[dir][1]);
   const dim3 grid = blocks2d(g.nx + 1, g.ny + 1, b);
   const int periodic = dir == 0 ? (flags.side[0] == 0 && flags.side[1] == 0) : (flags.side[2] == 0 && flags.side[3] == 0);
   auto one_lane = [&](auto qx, auto qy) {
@@ -2281,16 +2169,16 @@ template <class T>
 void launch_flux_learned(const GridD& g, int dir, int order, const Flags4& flags, double gamma,
                          const IfaceView<T>& in, const FluxView<T>& flux, double* rate, const uint8_t* cell_flags,
                          const unsigned long long* fb_count, const unsigned long long* fb_list, hipStream_t stream,
-                         dim3 b, int list_blocks) {
+                         int list_blocks) {
   if (order != 5 && order != 7) throw std::invalid_argument("flux launch: the learned form runs MP5/MP7");
   const T gm = T(gamma);
   const int periodic = dir == 0 ? (flags.side[0] == 0 && flags.side[1] == 0) : (flags.side[2] == 0 && flags.side[3] == 0);
   // The list holds at most the reconstruction launch's faces.
   const std::size_t max_list = dir == 0 ? static_cast<std::size_t>(g.nx + 1) * (g.ny + 2 * g.ng)
                                         : static_cast<std::size_t>(g.nx + 2 * g.ng) * (g.ny + 1);
-  const dim3 list_grid(static_cast<unsigned>((max_list + 255) / 256)), list_block(256);
-  (void)list_blocks;
-  (void)b;
+  const std::size_t fill = static_cast<std::size_t>(list_blocks) * 256 / kFluxListBlock;
+  const dim3 list_block(kFluxListBlock),
+      list_grid(static_cast<unsigned>(std::min(fill, (max_list + kFluxListBlock - 1) / kFluxListBlock)));
   auto listed = [&](auto q) {
     go<decltype(q)>(list_grid, list_block, stream, g, periodic, gm, in, flux, rate, cell_flags, fb_count, fb_list);
   };
@@ -2436,7 +2324,7 @@ hipError_t upload_quad_rows(const QuadRows& rows) {
 #define QMHD_INSTANTIATE_LEARNED(T)                                                                                \
   template void launch_flux_learned<T>(const GridD&, int, int, const Flags4&, double, const IfaceView<T>&,         \
                                        const FluxView<T>&, double*, const uint8_t*, const unsigned long long*,      \
-                                       const unsigned long long*, hipStream_t, dim3, int);                         \
+                                       const unsigned long long*, hipStream_t, int);                               \
   template void launch_reconstruct_learned<T>(const GridD&, int, int, double, const Flags4&, const StateView&,     \
                                               const double*, const double*, const uint8_t*, const IfaceView<T>&,  \
                                               int*, unsigned long long*, unsigned long long*, unsigned long long*, \

@@ -87,7 +87,7 @@ template <class T>
 void launch_flux_learned(const GridD& g, int dir, int order, const Flags4& flags, double gamma,
                          const IfaceView<T>& in, const FluxView<T>& flux, double* rate, const uint8_t* cell_flags,
                          const unsigned long long* fb_count, const unsigned long long* fb_list, hipStream_t stream,
-                         dim3 b, int list_blocks);
+                         int list_blocks);
 template <class T>
 void launch_reconstruct_learned(const GridD& g, int dir, int order, double gamma, const Flags4& flags,
                                 const StateView& u, const double* bxc, const double* byc, const uint8_t* cell_flags,
@@ -96,6 +96,8 @@ void launch_reconstruct_learned(const GridD& g, int dir, int order, double gamma
                                 unsigned long long* fb2_list, unsigned long long* plain_total,
                                 const FluxView<T>& flux, double* rate, hipStream_t stream, int list_blocks = 1024,
                                 int cheap_tile = 0);
+// `rate` may be null (no signal speeds wanted); `block` shapes the orders
+// without transverse quadrature (MP5/MP7 take their LDS tile).
 template <class T>
 void launch_flux(const GridD& g, int dir, int order, int hll_only, const Flags4& flags, double gamma,
                  const IfaceView<T>& in, const FluxView<T>& flux, double* rate, hipStream_t stream,

@@ -977,6 +977,11 @@ struct QuadRows {
   double mp5_gauss[3];
   double mp7_point[4][7];
   double mp7_gauss[4];
+  // The point rows as weights of the neighbour differences s[m+1] - s[m]
+  // about the centre sample, and the running-mean weights of the Gauss
+  // average, w_q / (w_0 + .. + w_q); in FP64 and rounded to FP32.
+  double mp5_step[3][4], mp5_mean[3], mp7_step[4][6], mp7_mean[4];
+  float mp5_step_f[3][4], mp5_mean_f[3], mp7_step_f[4][6], mp7_mean_f[4];
 };
 
 }  // namespace qmhd

@@ -39,7 +39,7 @@ namespace qmhd {
 // kernel from 4.45 to 4.30 ms and the learned cell E_z from 111 to 97 us per
 // launch.  It does not suit launches where only the first workgroups have
 // work (the compact face lists, where it put every active workgroup on one
-// XCD: 2-3x slower) nor the FP64 flux kernel (2.6 % slower).
+// XCD: 2-3x slower).
 constexpr unsigned kXcds = 8;
 
 struct Blk {

@@ -5,6 +5,32 @@
 
 namespace qmhd {
 
+// step[m]: weight of s[m+1] - s[m] in the row's value less the centre sample:
+// the weights beyond the difference on the right of the centre, minus those
+// before it on the left.
+template <int N>
+static void difference_row(const double* w, double* step, float* step_f) {
+  constexpr int H = N / 2;
+  for (int m = 0; m < N - 1; ++m) {
+    long double sum = 0.0L;
+    if (m >= H)
+      for (int t = m + 1; t < N; ++t) sum += w[t];
+    else
+      for (int t = 0; t <= m; ++t) sum -= w[t];
+    step[m] = static_cast<double>(sum);
+    step_f[m] = static_cast<float>(sum);
+  }
+}
+
+static void mean_row(const double* w, int n, double* mean, float* mean_f) {
+  long double sum = 0.0L;
+  for (int q = 0; q < n; ++q) {
+    sum += w[q];
+    mean[q] = static_cast<double>(w[q] / sum);
+    mean_f[q] = static_cast<float>(w[q] / sum);
+  }
+}
+
 void build_quad_rows(QuadRows& r) {
   const double p5[3][5] = {{-0.0392523473402346598, 0.312987195324173573, 0.910833333333333384,
                             -0.216320528657506839, 0.0317523473402346601},
@@ -35,6 +61,10 @@ void build_quad_rows(QuadRows& r) {
   r.mp7_gauss[1] = 0.326072577431273103;
   r.mp7_gauss[2] = 0.326072577431273103;
   r.mp7_gauss[3] = 0.173927422568726925;
+  for (int q = 0; q < 3; ++q) difference_row<5>(r.mp5_point[q], r.mp5_step[q], r.mp5_step_f[q]);
+  for (int q = 0; q < 4; ++q) difference_row<7>(r.mp7_point[q], r.mp7_step[q], r.mp7_step_f[q]);
+  mean_row(r.mp5_gauss, 3, r.mp5_mean, r.mp5_mean_f);
+  mean_row(r.mp7_gauss, 4, r.mp7_mean, r.mp7_mean_f);
 }
 
 }  // namespace qmhd

@@ -471,7 +471,6 @@ class Solver {
       fxp[c] = fx_[c].p;
       fyp[c] = fy_[c].p;
     }
-    (void)want_rates;
     if (learned_ && order == order_) {
       if (!indicator_set_)
         throw std::invalid_argument("MhdSolver2D: indicator 'mlp' needs its network (set_indicator) before stepping");
@@ -486,10 +485,13 @@ class Solver {
       faces_issued_ += static_cast<long long>(g_.nx + 1) * (g_.ny + 2 * g_.ng) +
                        static_cast<long long>(g_.nx + 2 * g_.ng) * (g_.ny + 1);
     }
+    // Only the live state's face rates are reduced to a timestep.
+    double* rx = want_rates ? rate_x_.p : nullptr;
+    double* ry = want_rates ? rate_y_.p : nullptr;
     if (fp32_)
-      issue_faces_as<float>(r, order, hll, ip, fxp, fyp);
+      issue_faces_as<float>(r, order, hll, ip, fxp, fyp, rx, ry);
     else
-      issue_faces_as<double>(r, order, hll, ip, fxp, fyp);
+      issue_faces_as<double>(r, order, hll, ip, fxp, fyp, rx, ry);
   }
 
   template <class T>
@@ -506,24 +508,25 @@ class Solver {
   }
 
   template <class T>
-  void issue_faces_as(Register& r, int order, int hll, double* const* ip, double* const* fxp, double* const* fyp) {
+  void issue_faces_as(Register& r, int order, int hll, double* const* ip, double* const* fxp, double* const* fyp,
+                      double* rx, double* ry) {
     const uint8_t* cf = learned_ && order == order_ ? flags() : nullptr;
     clock_.timed(QMHD_KERNEL_RECONSTRUCT, stream_,
-                 [&] { issue_reconstruct<T>(r, 0, order, ip, reinterpret_cast<int*>(eqx_.p), fxp, rate_x_.p); });
+                 [&] { issue_reconstruct<T>(r, 0, order, ip, reinterpret_cast<int*>(eqx_.p), fxp, rx); });
     auto flux = [&](int dir, double* const* fp, double* rate) {
       clock_.timed(QMHD_KERNEL_FLUX, stream_, [&] {
         if (cf)
           launch_flux_learned<T>(g_, dir, order, field_, gamma_, iface_as<T>(ip), flux_as<T>(fp), rate, cf,
-                                 fb_count(), fb_list(), stream_, tuning_.flux, tuning_.list_blocks);
+                                 fb_count(), fb_list(), stream_, tuning_.list_blocks);
         else
           launch_flux<T>(g_, dir, order, hll, field_, gamma_, iface_as<T>(ip), flux_as<T>(fp), rate, stream_,
                          tuning_.flux);
       });
     };
-    flux(0, fxp, rate_x_.p);
+    flux(0, fxp, rx);
     clock_.timed(QMHD_KERNEL_RECONSTRUCT, stream_,
-                 [&] { issue_reconstruct<T>(r, 1, order, ip, reinterpret_cast<int*>(eqy_.p), fyp, rate_y_.p); });
-    flux(1, fyp, rate_y_.p);
+                 [&] { issue_reconstruct<T>(r, 1, order, ip, reinterpret_cast<int*>(eqy_.p), fyp, ry); });
+    flux(1, fyp, ry);
   }
 
   // Cell E_z, corner E_z and the fused update of one stage.
@@ -1239,15 +1242,15 @@ void prepare_emf_tables(const qmhd::GridD& d, int order, bool hll_only, const qm
   qmhd::launch_cell_emf<double>(d, order, f, gamma, qmhd::view(u8), s.plane(0), s.plane(1), t.cell_ez, stream);
   qmhd::launch_eq_flags(d, 0, qmhd::iface(const_cast<double* const*>(ifx16)), t.xface_no_jump, stream);
   qmhd::launch_eq_flags(d, 1, qmhd::iface(const_cast<double* const*>(ify16)), t.yface_no_jump, stream);
-  // The face kernel writes all eight flux components and the face rate: the
+  // The face kernel writes all eight flux components: the
   // By (x faces) and Bx (y faces) components go to the tables, the rest to
   // work planes (two components share a plane; only the table is read).
   double* fx[8] = {s.plane(0), s.plane(1), s.plane(2), s.plane(3), s.plane(4), s.plane(5), t.xface_flux_by, s.plane(6)};
   qmhd::launch_flux(d, 0, order, hll_only ? 1 : 0, f, gamma, qmhd::iface(const_cast<double* const*>(ifx16)),
-                    qmhd::fluxv(fx), s.plane(7), stream);
+                    qmhd::fluxv(fx), nullptr, stream);
   double* fy[8] = {s.plane(0), s.plane(1), s.plane(2), s.plane(3), s.plane(4), t.yface_flux_bx, s.plane(5), s.plane(6)};
   qmhd::launch_flux(d, 1, order, hll_only ? 1 : 0, f, gamma, qmhd::iface(const_cast<double* const*>(ify16)),
-                    qmhd::fluxv(fy), s.plane(7), stream);
+                    qmhd::fluxv(fy), nullptr, stream);
 }
 
 // Corner E_z from prepared tables: the corner reads only the By flux of the
@@ -1306,9 +1309,9 @@ int qmhd_hlld_flux(const qmhd_grid* g, int dir, int order, int hll_only, const i
   return guarded([&] {
     const qmhd::GridD d = qmhd::to_grid(*g);
     qmhd::ensure_quad_rows();
-    const Scratch s = scratch_of(g, scratch);
+    (void)scratch_of(g, scratch);  // a missing workspace stays refused
     qmhd::launch_flux(d, dir, order, hll_only, qmhd::flags_of(flags4), gamma,
-                      qmhd::iface(const_cast<double* const*>(in16)), qmhd::fluxv(flux8), s.plane(0), st(stream));
+                      qmhd::iface(const_cast<double* const*>(in16)), qmhd::fluxv(flux8), nullptr, st(stream));
     qmhd::hip_check(hipGetLastError(), "hlld_flux");
   });
 }
