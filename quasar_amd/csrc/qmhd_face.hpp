@@ -28,6 +28,11 @@ namespace qmhd {
 __host__ __device__ __forceinline__ double fm(double a, double b, double c) { return __builtin_fma(a, b, c); }
 __host__ __device__ __forceinline__ float fm(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 
+__host__ __device__ __forceinline__ double lo2(double a, double b) { return __builtin_fmin(a, b); }
+__host__ __device__ __forceinline__ double hi2(double a, double b) { return __builtin_fmax(a, b); }
+__host__ __device__ __forceinline__ float lo2(float a, float b) { return __builtin_fminf(a, b); }
+__host__ __device__ __forceinline__ float hi2(float a, float b) { return __builtin_fmaxf(a, b); }
+
 // sqrt(x) and 1 / (2 sqrt(x)) of a positive normal x (Goldschmidt from the
 // hardware's reciprocal square root).
 __host__ __device__ __forceinline__ double sqrt_pos(double x, double& half_inv) {
@@ -99,10 +104,10 @@ __host__ __device__ __forceinline__ bool side_of(const St<T>& s, T gamma, Side<T
 template <class T>
 __host__ __device__ __forceinline__ T fast_of(const Side<T>& s, T bn2, T gamma) {
 #pragma clang fp contract(off)
-  const T a2 = gamma * __builtin_fmax(s.p, T(0)) * s.ir, c2 = bn2 * s.ir;
+  const T a2 = gamma * hi2(s.p, T(0)) * s.ir, c2 = bn2 * s.ir;
   const T sum = fm(s.bt2, s.ir, a2 + c2);
   T h;
-  const T disc = __builtin_fmax(fm(sum, sum, T(-4) * (a2 * c2)), Lim<T>::tiny);
+  const T disc = hi2(fm(sum, sum, T(-4) * (a2 * c2)), Lim<T>::tiny);
   return sqrt_pos(T(0.5) * (sum + sqrt_pos(disc, h)), h);
 }
 
@@ -112,7 +117,7 @@ template <class T>
 __host__ __device__ __forceinline__ T rate_of(const Side<T>& l, T cl, const Side<T>& r, T cr, int order) {
 #pragma clang fp contract(off)
   const T ul = qabs(l.vx), ur = qabs(r.vx);
-  const T v = order <= 1 ? __builtin_fmax(ul + cl, ur + cr) : __builtin_fmax(ul, ur) + __builtin_fmax(cl, cr);
+  const T v = order <= 1 ? hi2(ul + cl, ur + cr) : hi2(ul, ur) + hi2(cl, cr);
   return l.p > T(0) && r.p > T(0) && fin(v) ? v : Lim<T>::inf();
 }
 
@@ -132,8 +137,8 @@ __host__ __device__ __forceinline__ St<T> hlld_sides(const St<T>& L, const St<T>
   const T rhor = R.rho, mxr = R.mx, myr = R.my, mzr = R.mz, byr = R.by, bzr = R.bz;
   const T enL = fm(T(0.5), bn2 - l.bn2, L.en), enR = fm(T(0.5), bn2 - r.bn2, R.en);
   const T ptL = fm(T(0.5), bn2 + l.bt2, l.p), ptR = fm(T(0.5), bn2 + r.bt2, r.p);
-  const T cf = __builtin_fmax(l.cf, r.cf);
-  const T sl = __builtin_fmin(l.vx, r.vx) - cf, sr = __builtin_fmax(l.vx, r.vx) + cf;
+  const T cf = hi2(l.cf, r.cf);
+  const T sl = lo2(l.vx, r.vx) - cf, sr = hi2(l.vx, r.vx) + cf;
   const bool equal = L.rho == R.rho && L.mx == R.mx && L.my == R.my && L.mz == R.mz && L.en == R.en && L.bx == R.bx &&
                      L.by == R.by && L.bz == R.bz;
   // Equal states, like a supersonic face, take the physical flux of one side.
@@ -269,7 +274,7 @@ __host__ __device__ __forceinline__ St<T> solve_face(const St<T>& L, const St<T>
       cl = fast_of(l, l.bn2, gamma);
       cr = fast_of(r, r.bn2, gamma);
     }
-    smax = __builtin_fmax(smax, rate_of(l, cl, r, cr, order));
+    smax = hi2(smax, rate_of(l, cl, r, cr, order));
   }
   if constexpr (LF)
     return rot(lf_flux(L, R, l.ir, r.ir, gamma), dir);
@@ -379,7 +384,7 @@ __device__ __forceinline__ St<T> node_flux(const QuadRows& rows, const T* diff, 
     T speed = T(0);
     const St<T> f = solve_face<LF>(ra, rb, l, r, dir, ORDER, gamma, rate, speed);
     // The rate takes every point before the first inadmissible one.
-    if (rate && ok && q < R::NQ) smax = __builtin_fmax(smax, speed);
+    if (rate && ok && q < R::NQ) smax = hi2(smax, speed);
     const bool take = q < R::NQ || !ok;
     const T w = q == 0 || q == R::NQ ? T(1) : R::mean(rows, q);
 #pragma unroll

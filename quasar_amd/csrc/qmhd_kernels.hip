@@ -14,11 +14,13 @@
 #include "qmhd_face.hpp"
 #include "qmhd_kernels.hpp"
 #include "qmhd_queue.hpp"
+#include "qmhd_recon.hpp"
 #include "qmhd_stencil.hpp"
 
 #include <algorithm>
 #include <cstdint>
 #include <stdexcept>
+#include <type_traits>
 
 namespace qmhd {
 
@@ -240,21 +242,36 @@ __global__ __launch_bounds__(256) void collocate_kernel(GridD g, int axis, int c
   cell[idx(g, i, j)] = v;
 }
 
-// One thread per face normal to `dir`: dir 0 faces i in [0,nx], j in [-ng,ny+ng);
-// dir 1 faces i in [-ng,nx+ng), j in [0,ny].  Writes L (0..7) and R (8..15)
-// interface planes and the per-face "L == R" flag used by the CT 1-D shortcut.
+// Writes a face's L (0..7) and R (8..15) interface planes, from states in the
+// frame of its normal, and its "L == R" flag used by the CT 1-D shortcut.
 template <class T>
-__device__ __forceinline__ void write_faces(const IfaceView<T>& out, int* eq_flag, std::size_t k, const St<T>& ul,
-                                            const St<T>& ur) {
+__device__ __forceinline__ void write_faces(const IfaceView<T>& out, int dir, int* eq_flag, std::size_t k,
+                                            const St<T>& ul, const St<T>& ur) {
+  // Plane of component c: x and y components exchanged for y faces.
+  const int plane[8] = {0, dir == 0 ? 1 : 2, dir == 0 ? 2 : 1, 3, 4, dir == 0 ? 5 : 6, dir == 0 ? 6 : 5, 7};
 #pragma unroll
   for (int c = 0; c < 8; ++c) {
-    out.c[c][k] = comp(ul, c);
-    out.c[8 + c][k] = comp(ur, c);
+    out.c[plane[c]][k] = comp(ul, c);
+    out.c[8 + plane[c]][k] = comp(ur, c);
   }
   bool eq = true;
 #pragma unroll
   for (int c = 0; c < 8; ++c) eq = eq && (comp(ul, c) == comp(ur, c));
   eq_flag[k] = eq ? 1 : 0;
+}
+
+// Appends face k of every lane with `need` to a list (one atomic per wave;
+// every lane of the wave calls it).
+__device__ __forceinline__ void list_faces(bool need, std::size_t k, unsigned long long* __restrict__ count,
+                                           unsigned long long* __restrict__ list) {
+  const unsigned long long mask = __ballot(need);
+  if (mask == 0ull) return;
+  const int lane = static_cast<int>(__lane_id());
+  const int leader = __ffsll(static_cast<long long>(mask)) - 1;
+  unsigned long long base = 0;
+  if (lane == leader) base = atomicAdd(count, static_cast<unsigned long long>(__popcll(mask)));
+  base = __shfl(base, leader, 64);
+  if (need) list[base + __popcll(mask & ((1ull << lane) - 1ull))] = k;
 }
 
 // Face (i, j) of a reconstruction launch over dir 0 faces i in [0,nx],
@@ -268,12 +285,28 @@ __device__ __forceinline__ bool recon_face_of(const Blk& qb, const GridD& g, int
   return li < g.nx + 2 * g.ng && lj <= g.ny;
 }
 
-// One thread per face normal to `dir`.  Writes L (0..7) and R (8..15)
-// interface planes and the per-face "L == R" flag used by the CT 1-D shortcut.
-// For MP5/MP7 this kernel takes the characteristic MP path only: a face whose
-// MP states (or their normal-field update) are not admissible is appended to
-// `fb_list` (one atomic per wave) and redone, fallback chain included, by the
-// fallback kernel.
+// Waves per SIMD of the MP reconstruction: in FP64 two (256 registers; it would
+// take 264, mostly in the rarely taken exact basis: 563 against 392 us per x
+// launch at 2048^2), in FP32 four.
+template <class T>
+constexpr int kReconWaves = sizeof(T) == 4 ? 4 : 2;
+// Faces per block of the MP5/MP7 reconstruction (x faces, y faces) and the
+// cells the larger of the two stages.
+constexpr int kReconTiles[2][2] = {{64, 4}, {32, 8}};
+template <int ORDER>
+constexpr int recon_tile_cells() {
+  constexpr int more = ORDER == 5 ? 5 : 7;
+  constexpr int x = (kReconTiles[0][0] + more) * kReconTiles[0][1], y = kReconTiles[1][0] * (kReconTiles[1][1] + more);
+  return x > y ? x : y;
+}
+
+// One thread per face normal to `dir`.  For MP5/MP7 this kernel takes the
+// characteristic MP path of qmhd_recon.hpp; a face that does not settle there is
+// appended to `fb_list` and redone, fallback chain included, by the fallback
+// kernel.  2048^2, x / y faces: 700 us each with the reference's face per thread
+// and its cells read from global memory (5.2k VALU instructions in the code, its
+// L R = I loop seven times), 392 / 400 us now in FP64 (2.0k besides the exact
+// basis); FP32 at 1024^2 132 -> 49 us.
 template <class T, int ORDER>
 __device__ __forceinline__ void reconstruct_kernel_tile(
     const Blk& qb, const GridD& g, int dir, T gamma, int side_lo, int side_hi, const StateView& u,
@@ -283,7 +316,7 @@ __device__ __forceinline__ void reconstruct_kernel_tile(
 }
 
 template <class T, int ORDER>
-__global__ __launch_bounds__(256) void reconstruct_kernel(GridD g, int dir, T gamma, int side_lo, int side_hi,
+__global__ __launch_bounds__(256, kReconWaves<T>) void reconstruct_kernel(GridD g, int dir, T gamma, int side_lo, int side_hi,
                                                           StateView u, const double* __restrict__ bxc,
                                                           const double* __restrict__ byc, IfaceView<T> out,
                                                           int* __restrict__ eq_flag,
@@ -329,7 +362,7 @@ struct reconstruct_kernel_q {
 // reconstruct_kernel over the tile queue, one workgroup per tile: the same text, the
 // arguments read from the tile's run record.
 template <class T, int ORDER>
-__global__ __launch_bounds__(256) void reconstruct_kernel_queue(
+__global__ __launch_bounds__(256, kReconWaves<T>) void reconstruct_kernel_queue(
     const typename reconstruct_kernel_q<T, ORDER>::Args* __restrict__ qargs, const QueueRun* __restrict__ qruns,
     int qnruns) {
   const QueueTile qtile = queue_tile(qruns, qnruns);
@@ -2040,7 +2073,7 @@ template <class T>
 void launch_reconstruct(const GridD& g, int dir, int order, double gamma, const Flags4& flags, const StateView& u,
                         const double* bxc, const double* byc, const IfaceView<T>& out, int* eq,
                         unsigned long long* fb_count, unsigned long long* fb_list, hipStream_t stream) {
-  const dim3 b(64, 4);
+  const dim3 b = order >= 5 ? dim3(kReconTiles[dir][0], kReconTiles[dir][1]) : dim3(64, 4);
   const int lx = dir == 0 ? g.nx + 1 : g.nx + 2 * g.ng;
   const int ly = dir == 0 ? g.ny + 2 * g.ng : g.ny + 1;
   const int slo = dir == 0 ? flags.side[0] : flags.side[2];

@@ -411,52 +411,71 @@ struct CharBasis {
   bool identity;
 };
 
-// Primitive rows of wave k (unset entries zero).
+// Primitive right and left rows of wave k (unset entries zero).
 template <class T>
-__host__ __device__ __forceinline__ void basis_rows(const CharBasis<T>& B, int k, T* r, T* l) {
+__host__ __device__ __forceinline__ void basis_right(const CharBasis<T>& B, int k, T* r) {
 #pragma clang fp contract(off)
   const T rho = B.rho, sqrt_rho = B.sqrt_rho, alpha_f = B.alpha_f, alpha_s = B.alpha_s;
   const T beta1 = B.beta1, beta2 = B.beta2, sbn = B.sbn, rs2 = B.rs2, cf = B.cf, cs = B.cs;
-  const T qf = B.qf, qs = B.qs, Af = B.Af, As = B.As, Nf = B.Nf, inv_a2 = B.inv_a2, rho_a2 = B.rho_a2;
+  const T qf = B.qf, qs = B.qs, Af = B.Af, As = B.As, rho_a2 = B.rho_a2;
 #pragma unroll
-  for (int v = 0; v < 7; ++v) {
-    r[v] = T(0);
-    l[v] = T(0);
-  }
+  for (int v = 0; v < 7; ++v) r[v] = T(0);
   if (k == 0) {
     r[0] = rho * alpha_f; r[1] = -alpha_f * cf; r[2] = qs * beta1; r[3] = qs * beta2;
     r[4] = alpha_f * rho_a2; r[5] = As * beta1; r[6] = As * beta2;
-    l[1] = -Nf * alpha_f * cf; l[2] = Nf * qs * beta1; l[3] = Nf * qs * beta2;
-    l[4] = Nf * alpha_f / rho; l[5] = Nf * As * beta1 / rho; l[6] = Nf * As * beta2 / rho;
   } else if (k == 6) {
     r[0] = rho * alpha_f; r[1] = alpha_f * cf; r[2] = -qs * beta1; r[3] = -qs * beta2;
     r[4] = alpha_f * rho_a2; r[5] = As * beta1; r[6] = As * beta2;
-    l[1] = Nf * alpha_f * cf; l[2] = -Nf * qs * beta1; l[3] = -Nf * qs * beta2;
-    l[4] = Nf * alpha_f / rho; l[5] = Nf * As * beta1 / rho; l[6] = Nf * As * beta2 / rho;
   } else if (k == 1) {
     r[2] = -beta2 * rs2; r[3] = beta1 * rs2;
     r[5] = -sbn * beta2 * rs2 * sqrt_rho; r[6] = sbn * beta1 * rs2 * sqrt_rho;
-    l[2] = -beta2 * rs2; l[3] = beta1 * rs2;
-    l[5] = -sbn * beta2 * rs2 / sqrt_rho; l[6] = sbn * beta1 * rs2 / sqrt_rho;
   } else if (k == 5) {
     r[2] = -beta2 * rs2; r[3] = beta1 * rs2;
     r[5] = sbn * beta2 * rs2 * sqrt_rho; r[6] = -sbn * beta1 * rs2 * sqrt_rho;
-    l[2] = -beta2 * rs2; l[3] = beta1 * rs2;
-    l[5] = sbn * beta2 * rs2 / sqrt_rho; l[6] = -sbn * beta1 * rs2 / sqrt_rho;
   } else if (k == 2) {
     r[0] = rho * alpha_s; r[1] = -alpha_s * cs; r[2] = -qf * beta1; r[3] = -qf * beta2;
     r[4] = alpha_s * rho_a2; r[5] = -Af * beta1; r[6] = -Af * beta2;
-    l[1] = -Nf * alpha_s * cs; l[2] = -Nf * qf * beta1; l[3] = -Nf * qf * beta2;
-    l[4] = Nf * alpha_s / rho; l[5] = -Nf * Af * beta1 / rho; l[6] = -Nf * Af * beta2 / rho;
   } else if (k == 4) {
     r[0] = rho * alpha_s; r[1] = alpha_s * cs; r[2] = qf * beta1; r[3] = qf * beta2;
     r[4] = alpha_s * rho_a2; r[5] = -Af * beta1; r[6] = -Af * beta2;
+  } else {
+    r[0] = T(1);
+  }
+}
+template <class T>
+__host__ __device__ __forceinline__ void basis_left(const CharBasis<T>& B, int k, T* l) {
+#pragma clang fp contract(off)
+  const T rho = B.rho, sqrt_rho = B.sqrt_rho, alpha_f = B.alpha_f, alpha_s = B.alpha_s;
+  const T beta1 = B.beta1, beta2 = B.beta2, sbn = B.sbn, rs2 = B.rs2, cf = B.cf, cs = B.cs;
+  const T qf = B.qf, qs = B.qs, Af = B.Af, As = B.As, Nf = B.Nf, inv_a2 = B.inv_a2;
+#pragma unroll
+  for (int v = 0; v < 7; ++v) l[v] = T(0);
+  if (k == 0) {
+    l[1] = -Nf * alpha_f * cf; l[2] = Nf * qs * beta1; l[3] = Nf * qs * beta2;
+    l[4] = Nf * alpha_f / rho; l[5] = Nf * As * beta1 / rho; l[6] = Nf * As * beta2 / rho;
+  } else if (k == 6) {
+    l[1] = Nf * alpha_f * cf; l[2] = -Nf * qs * beta1; l[3] = -Nf * qs * beta2;
+    l[4] = Nf * alpha_f / rho; l[5] = Nf * As * beta1 / rho; l[6] = Nf * As * beta2 / rho;
+  } else if (k == 1) {
+    l[2] = -beta2 * rs2; l[3] = beta1 * rs2;
+    l[5] = -sbn * beta2 * rs2 / sqrt_rho; l[6] = sbn * beta1 * rs2 / sqrt_rho;
+  } else if (k == 5) {
+    l[2] = -beta2 * rs2; l[3] = beta1 * rs2;
+    l[5] = sbn * beta2 * rs2 / sqrt_rho; l[6] = -sbn * beta1 * rs2 / sqrt_rho;
+  } else if (k == 2) {
+    l[1] = -Nf * alpha_s * cs; l[2] = -Nf * qf * beta1; l[3] = -Nf * qf * beta2;
+    l[4] = Nf * alpha_s / rho; l[5] = -Nf * Af * beta1 / rho; l[6] = -Nf * Af * beta2 / rho;
+  } else if (k == 4) {
     l[1] = Nf * alpha_s * cs; l[2] = Nf * qf * beta1; l[3] = Nf * qf * beta2;
     l[4] = Nf * alpha_s / rho; l[5] = -Nf * Af * beta1 / rho; l[6] = -Nf * Af * beta2 / rho;
   } else {
-    r[0] = T(1);
     l[0] = T(1); l[4] = -inv_a2;
   }
+}
+template <class T>
+__host__ __device__ __forceinline__ void basis_rows(const CharBasis<T>& B, int k, T* r, T* l) {
+  basis_right(B, k, r);
+  basis_left(B, k, l);
 }
 
 // Conserved right column R[.][k] = M Rp[k] and left row L[k][.] = Lp[k] M^-1,
@@ -502,12 +521,13 @@ __host__ __device__ __forceinline__ void basis_lrow(const CharBasis<T>& B, const
 // order) with multiply-add contraction off, so the decision is that of the
 // reference arithmetic.
 template <class T>
-__host__ __device__ __forceinline__ void basis_build(const St<T>& s, T gamma, CharBasis<T>& B) {
+__host__ __device__ __forceinline__ void basis_scalars(const St<T>& s, T gamma, CharBasis<T>& B) {
 #pragma clang fp contract(off)
   // Primitive reference state (mhd_state.hpp:183-189, 228-239).
   const T rho = s.rho;
   const T vn = s.mx / rho, vt1 = s.my / rho, vt2 = s.mz / rho;
-  T p = (gamma - T(1)) * ((s.en - kinetic_from_momentum(s.mx, s.my, s.mz, rho)) - half_squared_norm3(s.bx, s.by, s.bz));
+  T p = (gamma - T(1)) *
+        ((s.en - kinetic_from_momentum(s.mx, s.my, s.mz, rho)) - half_squared_norm3(s.bx, s.by, s.bz));
   p = p > T(0) ? p : T(0);
   const T sqrt_rho = qsqrt(rho);
   const T bn = s.bx + T(0), bt1 = s.by + T(0), bt2 = s.bz + T(0);
@@ -598,34 +618,58 @@ __host__ __device__ __forceinline__ void basis_build(const St<T>& s, T gamma, Ch
   B.Nf = Nf;
   B.inv_a2 = inv_a2;
   B.rho_a2 = rho_a2;
-  // Loss of biorthogonality -> component-wise limiting (identity basis).
-  T R[7][7];
-#pragma unroll
-  for (int k = 0; k < 7; ++k) {
-    T r[7], l[7], col[7];
-    basis_rows(B, k, r, l);
-    basis_rcol(B, r, col);
-#pragma unroll
-    for (int v = 0; v < 7; ++v) R[v][k] = col[v];
-  }
-  // Row by row, in a rolled loop: one row of L live beside R (keeps the
-  // reconstruction kernel at two waves per SIMD).
+}
+
+// Whether L R = I within the reference's bound; a loss of biorthogonality sends
+// the face to component-wise limiting (identity basis).  A row of L at a time,
+// in a rolled loop.  In FP64 a column of R at a time too: the 7 x 7 columns
+// held beside the row are 98 registers, and set the occupancy of every kernel
+// that includes this.
+template <class T>
+__host__ __device__ __forceinline__ bool basis_usable(const CharBasis<T>& B) {
+#pragma clang fp contract(off)
   bool usable = true;
-#pragma nounroll
-  for (int i = 0; i < 7; ++i) {
-    T r[7], l[7], row[7];
-    basis_rows(B, i, r, l);
-    basis_lrow(B, l, row);
+  auto test = [&](int i, int j, const T* row, const T* col) {
+    T dot = row[0] * col[0];
+#pragma unroll
+    for (int k = 1; k < 7; ++k) dot = dot + row[k] * col[k];
+    const T expect = (i == j) ? T(1) : T(0);
+    usable = usable && fin(dot) && !(qabs(dot - expect) > T(1024) * Lim<T>::eps);
+  };
+  T cols[sizeof(T) == 4 ? 7 : 1][7];
+  if constexpr (sizeof(T) == 4) {
 #pragma unroll
     for (int j = 0; j < 7; ++j) {
-      T dot = row[0] * R[0][j];
-#pragma unroll
-      for (int k = 1; k < 7; ++k) dot = dot + row[k] * R[k][j];
-      const T expect = (i == j) ? T(1) : T(0);
-      usable = usable && fin(dot) && !(qabs(dot - expect) > T(1024) * Lim<T>::eps);
+      T r[7];
+      basis_right(B, j, r);
+      basis_rcol(B, r, cols[j]);
     }
   }
-  B.identity = !usable;
+#pragma nounroll
+  for (int i = 0; i < 7; ++i) {
+    T l[7], row[7];
+    basis_left(B, i, l);
+    basis_lrow(B, l, row);
+    if constexpr (sizeof(T) == 4) {
+#pragma unroll
+      for (int j = 0; j < 7; ++j) test(i, j, row, cols[j]);
+    } else {
+#pragma nounroll
+      for (int j = 0; j < 7; ++j) {
+        T r[7];
+        basis_right(B, j, r);
+        basis_rcol(B, r, cols[0]);
+        test(i, j, row, cols[0]);
+      }
+    }
+  }
+  return usable;
+}
+
+template <class T>
+__host__ __device__ __forceinline__ void basis_build(const St<T>& s, T gamma, CharBasis<T>& B) {
+  basis_scalars(s, gamma, B);
+  B.identity = !basis_usable(B);
 }
 
 // The conserved L and R (identity when the basis is not usable).

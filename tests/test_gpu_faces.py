@@ -1,0 +1,78 @@
+"""MP5/MP7 interface states and face fluxes against the oracle around the
+edges of the kernels' tiles (64 x 4 and 32 x 8 faces, 16 x 16 and 32 x 8
+fluxes, and the halos they stage), on smooth states, on states at rest with no
+transverse field, on supersonic ones and on ones far from unit density.  The
+bound is the one every launch of the ABI is held to: 1e-13 relative L1."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from gpu_helpers import call, flags, ptrs, qgrid, rel_l1_state, scratch, to_dev, to_host, zeros_dev
+from test_gpu_parity import face_mask, flux_mask
+
+pytestmark = pytest.mark.gpu
+G53 = 5.0 / 3.0
+
+
+def planes_of(state, nx, ny, ng):
+    rng = np.random.default_rng(1000 * nx + ny)
+    shape = (ny + 2 * ng, nx + 2 * ng)
+    y, x = np.mgrid[0:shape[0], 0:shape[1]]
+    w = lambda a, b: np.sin(2 * np.pi * (x / 17.0 + a)) * np.cos(2 * np.pi * (y / 13.0 + b))
+    rho, p = 1 + 0.3 * w(0.1, 0.2), 1 + 0.4 * w(0.3, 0.7)
+    v = [0.5 * w(0.2, 0.9), 0.4 * w(0.6, 0.1), 0.3 * w(0.8, 0.4)]
+    b = [0.6 + 0.2 * w(0.5, 0.5), 0.3 * w(0.4, 0.6), 0.2 * w(0.9, 0.3)]
+    if state == "at_rest":
+        v = [0 * rho] * 3
+        b = [0.75 + 0 * rho, 0 * rho, 0 * rho]
+        rho = np.where(x > shape[1] // 2, 0.125, 1.0)
+        p = np.where(x > shape[1] // 2, 0.1, 1.0)
+    elif state == "supersonic":
+        v = [8 * q for q in v]
+        rho = rho * np.where(rng.random(shape) < 0.1, 4.0, 1.0)
+    elif state == "dense":
+        rho, p = 1e4 * rho, 1e2 * p
+    en = p / (G53 - 1) + 0.5 * rho * sum(q * q for q in v) + 0.5 * sum(q * q for q in b)
+    return [np.ascontiguousarray(q).ravel() for q in (rho, *(rho * q for q in v), en, *b)]
+
+
+def compare(got, want, sides, what):
+    """NaN (faces no fallback makes admissible) at the same entries; the rest to the bound."""
+    finite = np.ones(len(want[0]), dtype=bool)
+    for a, b in zip(got, want):
+        np.testing.assert_array_equal(np.isfinite(a), np.isfinite(b))
+        finite &= np.isfinite(b)
+    got, want = [q[finite] for q in got], [q[finite] for q in want]
+    for side in sides:
+        for c in range(8):
+            assert rel_l1_state(got, want, c, side) <= 1e-13, (*what, side + c)
+
+
+@pytest.mark.parametrize("state", ["smooth", "at_rest", "supersonic", "dense"])
+@pytest.mark.parametrize("order,ng,nx,ny", [(7, 4, 15, 17), (7, 4, 63, 4), (7, 4, 65, 31), (5, 3, 31, 9), (5, 3, 64, 3),
+                                            (5, 4, 33, 32), (7, 4, 5, 8)])
+def test_faces_at_tile_edges(oracle, order, ng, nx, ny, state):
+    from quasar_amd import _lib
+    lib = _lib.load()
+    g, qg = oracle.grid(nx, ny, ng), qgrid(nx, ny, ng)
+    planes = planes_of(state, nx, ny, ng)
+    oracle.fill_ghosts(g, (0, 0, 0, 0), (0, 0, 0, 0), planes)
+    n = len(planes[0])
+    sc = scratch(qg)
+    for d in (0, 1):
+        ref16, ref8 = [np.zeros(n) for _ in range(16)], [np.zeros(n) for _ in range(8)]
+        oracle.reconstruct(g, d, order, (0, 0, 0, 0), G53, planes, ref16)
+        dev, out = to_dev(planes), zeros_dev(n, 16)
+        call(lib.qmhd_reconstruct, C.byref(qg), d, order, flags((0, 0, 0, 0)), G53, ptrs(dev), ptrs(out),
+             C.c_void_p(sc.data_ptr()), None)
+        m = face_mask(nx, ny, ng, d)
+        got, want = [q[m] for q in to_host(out)], [q[m] for q in ref16]
+        compare(got, want, (0, 8), ("state", d))
+        oracle.face_flux(g, d, order, 0, (0, 0, 0, 0), G53, ref16, ref8)
+        dev, out = to_dev(ref16), zeros_dev(n, 8)
+        call(lib.qmhd_hlld_flux, C.byref(qg), d, order, 0, flags((0, 0, 0, 0)), G53, ptrs(dev), ptrs(out),
+             C.c_void_p(sc.data_ptr()), None)
+        m = flux_mask(nx, ny, ng)
+        got, want = [q[m] for q in to_host(out)], [q[m] for q in ref8]
+        compare(got, want, (0,), ("flux", d))
