@@ -75,6 +75,13 @@ __host__ __device__ __forceinline__ float rcp_near(float x) {
 #endif
 }
 
+// Nothing moves across it in the device schedule: bounds what is live at once.
+__host__ __device__ __forceinline__ void schedule_fence() {
+#if defined(__HIP_DEVICE_COMPILE__)
+  __builtin_amdgcn_sched_barrier(0);
+#endif
+}
+
 // What the solver needs of one state, in the frame of the face normal.
 template <class T>
 struct Side {
@@ -281,6 +288,33 @@ __host__ __device__ __forceinline__ St<T> solve_face(const St<T>& L, const St<T>
   else
     return rot(hlld_sides(L, R, l, r, bn), dir);
 }
+
+// E_z = vy Bx - vx By of a recovered point, its components taken in order (rho,
+// mx, my, mz, E, Bx, By, Bz) so that four scalars live beside them.
+template <class T>
+struct PointEz {
+  T ir, vx, vy, q, mag, ez;
+  bool dense;
+  __host__ __device__ __forceinline__ void take(int c, T v) {
+#pragma clang fp contract(off)
+    switch (c) {
+      case 0: ir = rcp_near(v); dense = v > T(0); break;
+      case 1: vx = v * ir; mag = v * vx; break;
+      case 2: vy = v * ir; mag = fm(v, vy, mag); break;
+      case 3: mag = fm(v, v * ir, mag); break;
+      case 4: q = fm(T(-0.5), mag, v); mag = fm(T(0.5), mag, qabs(v)); break;
+      case 5: ez = vy * v; vy = v * v; break;
+      case 6: ez = fm(-vx, v, ez); vy = fm(v, v, vy); break;
+      default: vy = fm(v, v, vy); q = fm(T(-0.5), vy, q); mag = fm(T(0.5), vy, mag);
+    }
+  }
+  // Certainly admissible: rho > 0 and the internal energy positive beyond
+  // rounding (a NaN or infinity anywhere fails).
+  __host__ __device__ __forceinline__ bool sure() const { return dense & (q > T(32) * Lim<T>::eps * mag); }
+  // Neither certainly admissible nor certainly not: the internal energy is
+  // within rounding of zero.
+  __host__ __device__ __forceinline__ bool unsure() const { return dense & (qabs(q) <= T(32) * Lim<T>::eps * mag); }
+};
 
 // Neighbour-difference rows of the point recovery: point q is
 // s[H] + sum_m step[q][m] (s[m+1] - s[m]), and the running-mean weights of the

@@ -286,8 +286,11 @@ __device__ __forceinline__ bool recon_face_of(const Blk& qb, const GridD& g, int
 }
 
 // Waves per SIMD of the MP reconstruction: in FP64 two (256 registers; it would
-// take 264, mostly in the rarely taken exact basis: 563 against 392 us per x
-// launch at 2048^2), in FP32 four.
+// take 264, mostly in the rarely taken exact basis: 563 against 327 us per x
+// launch at 2048^2), in FP32 four (49 us per 1024^2 launch; 54 with no bound).
+// The listed faces' kernel is left unbounded: it holds the whole stencil in
+// registers and its time is one face's latency (learned rotor 768^2 16 us; 29
+// with the bound).
 template <class T>
 constexpr int kReconWaves = sizeof(T) == 4 ? 4 : 2;
 // Faces per block of the MP5/MP7 reconstruction (x faces, y faces) and the
@@ -305,8 +308,8 @@ constexpr int recon_tile_cells() {
 // appended to `fb_list` and redone, fallback chain included, by the fallback
 // kernel.  2048^2, x / y faces: 700 us each with the reference's face per thread
 // and its cells read from global memory (5.2k VALU instructions in the code, its
-// L R = I loop seven times), 392 / 400 us now in FP64 (2.0k besides the exact
-// basis); FP32 at 1024^2 132 -> 49 us.
+// L R = I loop seven times), 327 us now in FP64 (2.0k besides the exact basis;
+// 494 / 523 with the cells read from global memory); FP32 at 1024^2 132 -> 49 us.
 template <class T, int ORDER>
 __device__ __forceinline__ void reconstruct_kernel_tile(
     const Blk& qb, const GridD& g, int dir, T gamma, int side_lo, int side_hi, const StateView& u,
@@ -1044,20 +1047,46 @@ struct QueueTiles<cfl_reduce_kernel_q> {
 
 // ---------------------------------------------------------------------------
 // Cell-average E_z = vy Bx - vx By by tensor Gauss recovery (MP5: 3x3 points
-// from a 5x5 stencil, MP7: 4x4 from 7x7).  The block stages its cell stencil
-// (8 components) in LDS.
+// from a 5x5 stencil, MP7: 4x4 from 7x7).
+//
+// Bound by instruction issue (about 2000 VALU instructions per 64 cells in
+// FP64) with the LDS reads of the x pass behind it.  A wave owns 16 columns by
+// the NQ x nodes and marches up its rows: a row's 22 x 8 values go through a
+// wave-private LDS line (loaded one row ahead, no block barrier), its x point
+// values enter a window of 2H + 1 rows in registers, and the y values, E_z and
+// pressure test of the row below come from the window.  Point values are
+// weighted neighbour differences about the centre, so equal samples give that
+// sample with no comparison; a point is admissible when its internal energy is
+// positive beyond rounding, and rows with one that is within rounding of zero
+// are decided again, in the oracle's operations, after the march.  2048^2 FP64
+// 702 -> 391 us, 1024^2 FP32 119 -> 69 us, 64^2 FP64 28 -> 12 us, learned rotor
+// 768^2 35 -> 24 us, a queue of 24 learned runs 55 -> 30 us, against both passes
+// through LDS by 16 x 16 cells.
 
-// Cell E_z tiles (cells per block, BX x BY = 256 threads): the autotuner picks
-// one of kEmfTiles.
+// Cell E_z tiles: a block covers kEmfTiles[.][0] (at least 16) columns and
+// march times kEmfTiles[.][1] rows; the autotuner picks one.  With LEARNED a
+// BX x BY tile none of whose cells the indicator flagged takes the cell-average
+// E_z (second order) in every cell.
 constexpr int kEmfTiles[3][2] = {{16, 16}, {32, 8}, {8, 32}};
 
-// With LEARNED, a block none of whose cells the indicator flagged takes the
-// cell-average E_z (second order) for every cell, without staging its tile.
+// A wave that marches m rows spends m + 2H rows of x passes, a quarter of its
+// work per row: waves march four times as far (16 rows) when that leaves at
+// least this many blocks (two waves per SIMD), twice or once as far below
+// (64^2: 10 row steps one after the other, 12 us, in place of 22).
+constexpr unsigned kEmfBlocks = 512;
+
+// Orders this wave's LDS writes before its reads of other lanes' values (the
+// LDS serves a wave's accesses in order; this keeps the compiler to it).
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
 template <class T, int ORDER, bool LEARNED, int BX, int BY>
 __device__ __forceinline__ void cell_emf_kernel_tile(
     const Blk& qb, const GridD& g, int phys_x_high, int phys_y_high, T gamma, const StateView& u,
     const double* __restrict__ bxc, const double* __restrict__ byc, double* __restrict__ cell_ez,
-    const uint8_t* __restrict__ cell_flags) {
+    const uint8_t* __restrict__ cell_flags, int march) {
 #include "tiles/cell_emf_kernel.inc"
 }
 
@@ -1065,8 +1094,8 @@ template <class T, int ORDER, bool LEARNED, int BX, int BY>
 __global__ __launch_bounds__(256) void cell_emf_kernel(GridD g, int phys_x_high, int phys_y_high, T gamma,
                                                        StateView u, const double* __restrict__ bxc,
                                                        const double* __restrict__ byc, double* __restrict__ cell_ez,
-                                                       const uint8_t* __restrict__ cell_flags) {
-  [[maybe_unused]] const Blk qb = LEARNED ? Blk::xcd_tiled() : Blk::native();
+                                                       const uint8_t* __restrict__ cell_flags, int march) {
+  [[maybe_unused]] const Blk qb = Blk::xcd_tiled();
 #include "tiles/cell_emf_kernel.inc"
 }
 
@@ -1083,16 +1112,17 @@ struct cell_emf_kernel_q {
     const double* byc;
     double* cell_ez;
     const uint8_t* cell_flags;
+    int march;
   };
   static __device__ __forceinline__ void run(const Blk& qb, const Args& a) {
     cell_emf_kernel_tile<T, ORDER, LEARNED, BX, BY>(qb, queue_arg(a.g), queue_arg(a.phys_x_high),
                                                     queue_arg(a.phys_y_high), queue_arg(a.gamma), queue_arg(a.u),
                                                     queue_arg(a.bxc), queue_arg(a.byc), queue_arg(a.cell_ez),
-                                                    queue_arg(a.cell_flags));
+                                                    queue_arg(a.cell_flags), queue_arg(a.march));
   }
   static void launch(dim3 grid, dim3 block, hipStream_t s, const Args& a) {
     hipLaunchKernelGGL((cell_emf_kernel<T, ORDER, LEARNED, BX, BY>), grid, block, 0, s, a.g, a.phys_x_high,
-                       a.phys_y_high, a.gamma, a.u, a.bxc, a.byc, a.cell_ez, a.cell_flags);
+                       a.phys_y_high, a.gamma, a.u, a.bxc, a.byc, a.cell_ez, a.cell_flags, a.march);
   }
   static const void* tag() {
     static const char t = 0;
@@ -1118,6 +1148,7 @@ __global__ __launch_bounds__(256) void cell_emf_kernel_queue(
   const double* __restrict__ byc = queue_arg(qa.byc);
   double* __restrict__ cell_ez = queue_arg(qa.cell_ez);
   const uint8_t* __restrict__ cell_flags = queue_arg(qa.cell_flags);
+  int march = qa.march;
 #include "tiles/cell_emf_kernel.inc"
 }
 template <class T, int ORDER, bool LEARNED, int BX, int BY>
@@ -2235,10 +2266,13 @@ void launch_cell_emf(const GridD& g, int order, const Flags4& flags, double gamm
   const int pyh = flags.side[3] != 0 && flags.side[3] != 4;
   if (order == 5 || order == 7) {
     if (tile < 0 || tile > 2) throw std::invalid_argument("cell E_z launch: tile choice is 0..2");
-    const dim3 b(kEmfTiles[tile][0], kEmfTiles[tile][1]);
-    const dim3 grid = blocks2d(g.nx + 1, g.ny + 1, b);
+    const int columns = std::max(16, kEmfTiles[tile][0]);
+    auto blocks = [&](int m) { return blocks2d(g.nx + 1, g.ny + 1, dim3(columns, m * kEmfTiles[tile][1])); };
+    auto many = [&](int m) { return blocks(m).x * blocks(m).y >= kEmfBlocks; };
+    const int march = cell_flags ? 1 : many(4) ? 4 : many(2) ? 2 : 1;
+    const dim3 b(256), grid = blocks(march);
     auto launch = [&](auto q) {
-      go<decltype(q)>(grid, b, stream, g, pxh, pyh, T(gamma), u, bxc, byc, cell_ez, cell_flags);
+      go<decltype(q)>(grid, b, stream, g, pxh, pyh, T(gamma), u, bxc, byc, cell_ez, cell_flags, march);
     };
     // ORDER x learned x tile.
     auto by_tile = [&](auto k0, auto k1, auto k2) { tile == 0 ? launch(k0) : tile == 1 ? launch(k1) : launch(k2); };

@@ -302,13 +302,6 @@ __host__ __device__ __forceinline__ bool settle_state(St<T>& s, T v) {
   return ok;
 }
 
-// Keeps the two wave groups apart in the device schedule.
-__host__ __device__ __forceinline__ void schedule_fence() {
-#if defined(__HIP_DEVICE_COMPILE__)
-  __builtin_amdgcn_sched_barrier(0);
-#endif
-}
-
 // Interface states of a face in the frame of its normal; cell(c, q) is
 // component c (rho, mn, mt1, mt2, E, bn, bt1, bt2) of cell q of its union
 // stencil, bn its own normal field.  False leaves the face to

@@ -1,6 +1,6 @@
-"""MP5/MP7 interface states and face fluxes against the oracle around the
-edges of the kernels' tiles (64 x 4 and 32 x 8 faces, 16 x 16 and 32 x 8
-fluxes, and the halos they stage), on smooth states, on states at rest with no
+"""MP5/MP7 interface states, face fluxes and cell E_z against the oracle around
+the edges of the kernels' tiles (64 x 4 and 32 x 8 faces, 16 x 16 and 32 x 8
+fluxes, 16 columns by 4 to 16 rows of cell E_z, and the halos they stage), on smooth states, on states at rest with no
 transverse field, on supersonic ones and on ones far from unit density.  The
 bound is the one every launch of the ABI is held to: 1e-13 relative L1."""
 import ctypes as C
@@ -76,3 +76,40 @@ def test_faces_at_tile_edges(oracle, order, ng, nx, ny, state):
         m = flux_mask(nx, ny, ng)
         got, want = [q[m] for q in to_host(out)], [q[m] for q in ref8]
         compare(got, want, (0,), ("flux", d))
+
+
+@pytest.mark.parametrize("state", ["smooth", "at_rest", "supersonic", "dense", "thin"])
+@pytest.mark.parametrize("order,ng,nx,ny,sides", [(7, 4, 15, 17, 0), (7, 4, 16, 3, 1), (7, 4, 33, 64, 0), (5, 3, 31, 9, 1),
+                                                  (5, 3, 17, 16, 0), (7, 4, 18, 5, 1), (7, 4, 5, 8, 0)])
+def test_cell_ez_at_tile_edges(oracle, order, ng, nx, ny, sides, state):
+    """`thin` holds points of zero and negative pressure: those cells take the
+    cell-average E_z, and the decision is the oracle's."""
+    from quasar_amd import _lib
+    lib = _lib.load()
+    g, qg = oracle.grid(nx, ny, ng), qgrid(nx, ny, ng)
+    F = (sides,) * 4
+    planes = planes_of("smooth" if state == "thin" else state, nx, ny, ng)
+    if state == "thin":
+        kinetic = sum(planes[c] ** 2 for c in (1, 2, 3)) / (2 * planes[0])
+        rng = np.random.default_rng(3)
+        planes[4] = kinetic + 0.5 * sum(planes[c] ** 2 for c in (5, 6, 7)) + 0.3 * rng.random(len(kinetic))
+    oracle.fill_ghosts(g, F, F, planes)
+    n = len(planes[0])
+    ref16 = [[np.zeros(n) for _ in range(16)] for _ in range(2)]
+    for d in (0, 1):
+        oracle.reconstruct(g, d, order, F, G53, planes, ref16[d])
+    want = oracle.ct_emf(g, order, 0, F, G53, planes, *ref16)["cell_ez"]
+    dev, faces = to_dev(planes), zeros_dev(n, 32)
+    out, eq = zeros_dev(n, 3), zeros_dev(n, 2)
+    tables = _lib.QEmfTables(*[t.data_ptr() for t in out], *[t.data_ptr() for t in eq])
+    sc = scratch(qg)
+    for d in (0, 1):
+        call(lib.qmhd_reconstruct, C.byref(qg), d, order, flags(F), G53, ptrs(dev), ptrs(faces[16 * d:16 * d + 16]),
+             C.c_void_p(sc.data_ptr()), None)
+    call(lib.qmhd_ct_emf_prepare, C.byref(qg), order, 0, flags(F), G53, ptrs(dev), ptrs(faces[:16]), ptrs(faces[16:]),
+         C.byref(tables), C.c_void_p(sc.data_ptr()), None)
+    m = np.zeros((ny + 2 * ng, nx + 2 * ng), dtype=bool)
+    m[ng:ng + ny + (sides != 0), ng:ng + nx + (sides != 0)] = True
+    got, ref = to_host(out[:1])[0][m.ravel()], want[m.ravel()]
+    scale = np.abs(ref).sum()
+    assert np.abs(got - ref).sum() <= 1e-13 * max(scale, 1e-3 * len(ref)), (np.abs(got - ref).max(), scale)
