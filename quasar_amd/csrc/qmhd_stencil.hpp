@@ -675,32 +675,35 @@ __host__ __device__ __forceinline__ bool point_ez(const St<T>& st, T gamma, T& e
 // of the cell E_z, plus the exact one-dimensional shortcuts
 // (mhd_ct.hip:811-878).
 
+// Value at an edge from the averages around it: (-3, 29, -139, 533, 533, ..) /
+// 840 and (1, -8, 37, 37, ..) / 60, as half the inner pair's sum plus weighted
+// differences of the other pairs' sums from it.  Equal samples give that sample
+// exactly with no comparison, and there is no division (11 instructions; the
+// quotient of the weighted sum after seven comparisons takes 40).
 __host__ __device__ __forceinline__ double edge_interp(int order, const double* e) {
+#pragma clang fp contract(off)
   if (order >= 7) {
-    bool constant = true;
-#pragma unroll
-    for (int k = 1; k < 8; ++k) constant = constant && e[k] == e[0];
-    if (constant) return e[0];
-    return (-3.0 * e[0] + 29.0 * e[1] - 139.0 * e[2] + 533.0 * e[3] + 533.0 * e[4] - 139.0 * e[5] + 29.0 * e[6] -
-            3.0 * e[7]) / 840.0;
+    const double p = e[3] + e[4], a = e[2] + e[5], b = e[1] + e[6], c = e[0] + e[7];
+    return __builtin_fma(-3.0 / 840.0, c - p, __builtin_fma(29.0 / 840.0, b - p, __builtin_fma(-139.0 / 840.0, a - p, 0.5 * p)));
   }
   if (order >= 5) {
-    bool constant = true;
-#pragma unroll
-    for (int k = 1; k < 6; ++k) constant = constant && e[k] == e[0];
-    if (constant) return e[0];
-    return (e[0] - 8.0 * e[1] + 37.0 * e[2] + 37.0 * e[3] - 8.0 * e[4] + e[5]) / 60.0;
+    const double p = e[2] + e[3], a = e[1] + e[4], b = e[0] + e[5];
+    return __builtin_fma(1.0 / 60.0, b - p, __builtin_fma(-8.0 / 60.0, a - p, 0.5 * p));
   }
   return e[0] == e[1] ? e[0] : (e[0] + e[1]) / 2.0;
+}
+
+// A corner on a conducting side has no E_z.
+__host__ __device__ __forceinline__ bool corner_conducting(const GridD& g, const Flags4& m, int i, int j) {
+  return (i == 0 && (m.side[0] == 2 || m.side[0] == 3)) || (i == g.nx && m.side[1] == 2) ||
+         (j == 0 && m.side[2] == 2) || (j == g.ny && m.side[3] == 2);
 }
 
 template <class T, bool INTERIOR>
 __host__ __device__ __forceinline__ double corner_ez_impl(const GridD& g, int order, const Flags4& m, const FluxView<T>& fx,
                                                      const FluxView<T>& fy, const double* cell_ez,
                                                      const int* eqx, const int* eqy, int i, int j) {
-  const bool conducting = (i == 0 && (m.side[0] == 2 || m.side[0] == 3)) || (i == g.nx && m.side[1] == 2) ||
-                          (j == 0 && m.side[2] == 2) || (j == g.ny && m.side[3] == 2);
-  if (conducting) return 0.0;
+  if (corner_conducting(g, m, i, j)) return 0.0;
   const int lo = order >= 7 ? -4 : order >= 5 ? -3 : -1;
   const int nt = order >= 7 ? 8 : order >= 5 ? 6 : 2;
   const int rh = order >= 7 ? 3 : order >= 5 ? 2 : 0;  // transverse recovery half-width

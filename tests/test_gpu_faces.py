@@ -113,3 +113,41 @@ def test_cell_ez_at_tile_edges(oracle, order, ng, nx, ny, sides, state):
     got, ref = to_host(out[:1])[0][m.ravel()], want[m.ravel()]
     scale = np.abs(ref).sum()
     assert np.abs(got - ref).sum() <= 1e-13 * max(scale, 1e-3 * len(ref)), (np.abs(got - ref).max(), scale)
+
+
+@pytest.mark.parametrize("data", ["smooth", "x_only", "y_only", "uniform"])
+@pytest.mark.parametrize("order,ng,nx,ny,sides", [(7, 4, 15, 17, (0, 0, 0, 0)), (7, 4, 40, 33, (1, 1, 0, 0)),
+                                                  (7, 4, 16, 9, (2, 2, 2, 2)), (5, 3, 47, 16, (1, 1, 1, 1)),
+                                                  (5, 4, 31, 5, (0, 0, 2, 1)), (7, 4, 5, 48, (1, 2, 0, 0))])
+def test_corner_at_tile_edges(oracle, order, ng, nx, ny, sides, data):
+    """Corner E_z over 16 x 16 blocks that hold the boundary, with data whose
+    one-dimensional shortcuts are taken everywhere, in places and nowhere; the
+    bound is the one of the launches above."""
+    from quasar_amd import _lib
+    lib = _lib.load()
+    g, qg = oracle.grid(nx, ny, ng), qgrid(nx, ny, ng)
+    planes = [p.reshape(ny + 2 * ng, nx + 2 * ng).copy() for p in planes_of("smooth", nx, ny, ng)]
+    if data in ("x_only", "uniform"):
+        planes = [np.broadcast_to(p[:1], p.shape).copy() for p in planes]
+    if data in ("y_only", "uniform"):
+        planes = [np.broadcast_to(p[:, :1], p.shape).copy() for p in planes]
+    if data == "x_only":
+        planes[5][:] = planes[5][0, 0]
+    if data == "y_only":
+        planes[6][:] = planes[6][0, 0]
+    planes = [p.ravel() for p in planes]
+    oracle.fill_ghosts(g, sides, sides, planes)
+    n = len(planes[0])
+    i16, f8 = [[np.zeros(n) for _ in range(16)] for _ in range(2)], [[np.zeros(n) for _ in range(8)] for _ in range(2)]
+    for d in (0, 1):
+        oracle.reconstruct(g, d, order, sides, G53, planes, i16[d])
+        oracle.face_flux(g, d, order, 0, sides, G53, i16[d], f8[d])
+    want = oracle.ct_emf(g, order, 0, sides, G53, planes, *i16)["ez"]
+    dev = [to_dev(x) for x in (planes, *i16, *f8)]
+    ez, sc = zeros_dev(n, 1)[0], scratch(qg)
+    call(lib.qmhd_ct_emf, C.byref(qg), order, flags(sides), G53, *[ptrs(x) for x in dev], C.c_void_p(ez.data_ptr()),
+         C.c_void_p(sc.data_ptr()), None)
+    m = flux_mask(nx, ny, ng)
+    got, ref = to_host([ez])[0][m], want[m]
+    assert np.isfinite(ref).all()
+    assert np.abs(got - ref).sum() <= 1e-13 * max(np.abs(ref).sum(), 1e-3 * len(ref))
