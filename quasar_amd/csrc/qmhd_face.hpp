@@ -264,6 +264,43 @@ __host__ __device__ __forceinline__ St<T> hlld_sides(const St<T>& L, const St<T>
   return f;
 }
 
+// HLL with Davis speeds of two states with one normal field, both sides
+// prepared, cf the larger of their fast speeds: F_L + w (F_R - F_L) + d (R - L),
+// so equal states give their own flux exactly.
+template <class T>
+__host__ __device__ __forceinline__ St<T> hll_sides(const St<T>& L, const St<T>& R, const Side<T>& l, const Side<T>& r,
+                                                    T cf) {
+#pragma clang fp contract(off)
+  const T sl = lo2(l.vx, r.vx) - cf, sr = hi2(l.vx, r.vx) + cf, width = sr - sl;
+  const bool fan = sl < T(0) && sr > T(0) && fin(width);
+  const T inv = rcp_near(fan ? width : T(1));
+  const T w = fan ? -sl * inv : !(sl >= T(0)) && sr <= T(0) ? T(1) : T(0), d = fan ? sl * sr * inv : T(0);
+  auto mix = [&](T a, T b, T x, T y) { return fm(d, y - x, fm(w, b - a, a)); };
+  const T bn = L.bx, ptl = fm(T(0.5), l.bt2, l.p), ptr = fm(T(0.5), r.bt2, r.p), hb = T(0.5) * l.bn2;
+  St<T> f;
+  f.rho = mix(L.mx, R.mx, L.rho, R.rho);
+  f.mx = mix(fm(L.mx, l.vx, ptl - hb), fm(R.mx, r.vx, ptr - hb), L.mx, R.mx);
+  f.my = mix(fm(L.mx, l.vy, -(bn * L.by)), fm(R.mx, r.vy, -(bn * R.by)), L.my, R.my);
+  f.mz = mix(fm(L.mx, l.vz, -(bn * L.bz)), fm(R.mx, r.vz, -(bn * R.bz)), L.mz, R.mz);
+  f.en = mix(fm(l.vx, (L.en - hb) + ptl, -(bn * fm(l.vy, L.by, l.vz * L.bz))),
+             fm(r.vx, (R.en - hb) + ptr, -(bn * fm(r.vy, R.by, r.vz * R.bz))), L.en, R.en);
+  f.bx = T(0);
+  f.by = mix(fm(L.by, l.vx, -(bn * l.vy)), fm(R.by, r.vx, -(bn * r.vy)), L.by, R.by);
+  f.bz = mix(fm(L.bz, l.vx, -(bn * l.vz)), fm(R.bz, r.vx, -(bn * r.vz)), L.bz, R.bz);
+  return f;
+}
+
+// The unlimited fifth-order face values of one component from the six cells
+// about the face (the MP5 interpolant's weights on its neighbour differences).
+template <class T>
+__host__ __device__ __forceinline__ void linear_pair(const T v[6], T& left, T& right) {
+#pragma clang fp contract(off)
+  const T d0 = v[1] - v[0], d1 = v[2] - v[1], d2 = v[3] - v[2], d3 = v[4] - v[3], d4 = v[5] - v[4];
+  constexpr T a = T(-2.0 / 60), b = T(11.0 / 60), c = T(24.0 / 60), e = T(-3.0 / 60);
+  left = fm(a, d0, fm(b, d1, fm(c, d2, fm(e, d3, v[2]))));
+  right = fm(-a, d4, fm(-b, d3, fm(-c, d2, fm(-e, d1, v[3]))));
+}
+
 // Flux of one pair of states (in the caller's frame), with the face's signal
 // speed folded into smax when RATE.
 template <bool LF, class T>

@@ -656,10 +656,17 @@ struct QueueTiles<counter_pair_reset_kernel_q> {
 // field.  Flagged faces, and cheap states that are not admissible, are listed
 // for the plain path (characteristic MP with its fallback chain).  The block
 // (64 x 4 faces) stages the cells its stencils read in LDS: 69 x 4 for x faces,
-// 64 x 9 for y faces.
-template <class T, int ORDER>
-__device__ __forceinline__ void cheap_face_flux(const St<T>& baseL, const St<T>& baseR, int dir, T gamma, St<T>& f,
-                                                T& smax);
+// 64 x 9 for y faces.  Bound by memory: 117 B per face in FP32, 380 us per 4096^2
+// launch at a copy's rate.  It was bound by instruction issue (1.2k VALU
+// instructions a face: 16 flag reads with their range tests for every face,
+// index quotients by a width not known in advance, finiteness and pressure
+// tests and speeds formed apart): where no flag is near the block none is
+// read per face, and each state's 1/rho, velocity and pressure serve its
+// admissibility, its speed and its flux.  x / y faces 533 / 527 -> 445 / 499 us,
+// and 404 / 450 with the blocks of one XCD adjacent (halo rows from its L2).
+template <class T>
+__device__ __forceinline__ void cheap_face_flux(const St<T>& L, const St<T>& R, const Side<T>& l, const Side<T>& r,
+                                                int dir, T gamma, bool rate, St<T>& f, T& smax);
 template <class T>
 __device__ __forceinline__ void store_face(const GridD& g, int dir, const FluxView<T>& flux, double* __restrict__ rate,
                                            std::size_t ko, const St<T>& f, T smax);
@@ -695,7 +702,7 @@ __global__ __launch_bounds__(256) void cheap_reconstruct_kernel(GridD g, int dir
                                                                 unsigned long long* __restrict__ fb_list,
                                                                 FluxView<T> flux, double* __restrict__ rate,
                                                                 int periodic_dir) {
-  [[maybe_unused]] const Blk qb = Blk::native();
+  [[maybe_unused]] const Blk qb = Blk::xcd_tiled();
 #include "tiles/cheap_reconstruct_kernel.inc"
 }
 
@@ -769,54 +776,17 @@ struct QueueTiles<cheap_reconstruct_kernel_q<T, TX, TY>> {
 // ---------------------------------------------------------------------------
 // Face flux with transverse Gauss quadrature and the CFL face rate.
 
-// |v_n| and c_fast of one face state (1/rho supplied) in the direction
-// `dir`; infinite when the state is not admissible.
-template <class T>
-__device__ __forceinline__ void speed_parts(const St<T>& s, T inv_rho, int dir, T gamma, T& vel, T& fast) {
-  const T gm1 = gamma - T(1);
-  const T p = pressure_ir(s, inv_rho, gm1);
-  if (!(fin(s.rho) && s.rho > T(0) && fin(s.mx) && fin(s.my) && fin(s.mz) && fin(s.en) && fin(s.bx) &&
-        fin(s.by) && fin(s.bz) && fin(p) && p > T(0))) {
-    vel = Lim<T>::inf();
-    fast = Lim<T>::inf();
-    return;
-  }
-  const T bn = dir == 0 ? s.bx : s.by;
-  const T bt = dir == 0 ? s.by : s.bx;
-  const T a2 = gamma * p * inv_rho;
-  const T b2 = (bn * bn + bt * bt + s.bz * s.bz) * inv_rho;
-  const T c2 = bn * bn * inv_rho;
-  const T sum = a2 + b2;
-  T disc = sum * sum - T(4) * a2 * c2;
-  disc = disc < T(0) ? T(0) : disc;
-  fast = fsqrt(T(0.5) * (sum + fsqrt(disc)));
-  vel = qabs(dir == 0 ? s.mx : s.my) * inv_rho;
-  if (!(fin(vel) && fin(fast))) {
-    vel = Lim<T>::inf();
-    fast = Lim<T>::inf();
-  }
-}
-
-template <class T>
-__device__ __forceinline__ T face_speed(const St<T>& L, T irL, const St<T>& R, T irR, int dir, int order,
-                                        T gamma) {
-  T vl, fl, vr, fr;
-  speed_parts(L, irL, dir, gamma, vl, fl);
-  speed_parts(R, irR, dir, gamma, vr, fr);
-  const T rate = order <= 1 ? fmax(vl + fl, vr + fr) : fmax(vl, vr) + fmax(fl, fr);
-  return fin(rate) ? rate : Lim<T>::inf();
-}
-
 // The learned form's flux of a face whose two cells the indicator left
-// unflagged: one HLL flux (Davis speeds) at its face-average states, the rate
-// from those states.  The plain list's flux and the cheap-face kernel share
-// it, so both give the same bits.
-template <class T, int ORDER>
-__device__ __forceinline__ void cheap_face_flux(const St<T>& baseL, const St<T>& baseR, int dir, T gamma, St<T>& f,
-                                                T& smax) {
-  const T irL = frcp(baseL.rho), irR = frcp(baseR.rho);
-  smax = face_speed(baseL, irL, baseR, irR, dir, ORDER, gamma);
-  f = rot(hll_davis_flux(rot(baseL, dir), rot(baseR, dir), irL, irR, gamma), dir);
+// unflagged: one HLL flux (Davis speeds) at its face-average states (in the
+// frame of the normal, both with the face's own normal field), the rate from
+// those states.  The plain list's flux and the cheap-face kernel share it, so
+// both give the same bits.
+template <class T>
+__device__ __forceinline__ void cheap_face_flux(const St<T>& L, const St<T>& R, const Side<T>& l, const Side<T>& r,
+                                                int dir, T gamma, bool rate, St<T>& f, T& smax) {
+  const T cl = fast_of(l, l.bn2, gamma), cr = fast_of(r, r.bn2, gamma);
+  smax = rate ? rate_of(l, cl, r, cr, 5) : T(0);
+  f = rot(hll_sides(L, R, l, r, hi2(cl, cr)), dir);
 }
 
 // Face flux and, with a rate plane, the face rate (0.5 * signal speed /
