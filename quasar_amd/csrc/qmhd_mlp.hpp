@@ -95,6 +95,27 @@ __host__ __device__ __forceinline__ CellQ cell_quantities(double rho, double mx,
   return c;
 }
 
+// The same quantities from one reciprocal of rho (each quotient corrected by
+// its exact residual, Markstein 1990) and unscaled square roots: equal to the
+// ones above but where an FP64 ulp falls on an FP32 rounding boundary.
+__device__ __forceinline__ CellQ cell_quantities_shared(double rho, double mx, double my, double mz, double en,
+                                                        double bx, double by, double bz, double gamma) {
+#pragma clang fp contract(off)
+  CellQ c;
+  const double m2 = (mx * mx + my * my) + mz * mz;
+  const double b2 = (bx * bx + by * by) + bz * bz;
+  const double r = frcp(rho);
+  auto over = [&](double a) {
+    const double t = a * r;
+    return __builtin_fma(__builtin_fma(-rho, t, a), r, t);
+  };
+  c.q[0] = static_cast<float>(rho);
+  c.q[1] = static_cast<float>((gamma - 1.0) * ((en - over(0.5 * m2)) - 0.5 * b2));
+  c.q[2] = static_cast<float>(fsqrt(b2));
+  c.q[3] = static_cast<float>(over(fsqrt(m2)));
+  return c;
+}
+
 // 1 / (|Q_c| + max_k |Q_k - Q_c| + tiny) over the 5x5 stencil of one quantity,
 // `at(dy, dx)` returning the stencil values.
 template <class F>
@@ -105,6 +126,13 @@ __host__ __device__ __forceinline__ float feature_scale(F at) {
   for (int dy = -kHalo; dy <= kHalo; ++dy)
     for (int dx = -kHalo; dx <= kHalo; ++dx) dev = fmaxf(dev, __builtin_fabsf(at(dy, dx) - c));
   return 1.f / ((__builtin_fabsf(c) + dev) + 1e-30f);
+}
+
+// As feature_scale from the stencil's extrema: rounding is monotone, so the
+// larger of the two rounded differences is the largest of all.
+__host__ __device__ __forceinline__ float feature_scale_of(float c, float lo, float hi) {
+#pragma clang fp contract(off)
+  return 1.f / ((__builtin_fabsf(c) + fmaxf(hi - c, c - lo)) + 1e-30f);
 }
 
 // Feature f = 25 q + 5 (dy + 2) + (dx + 2): (Q_q(dy,dx) - Q_q(0,0)) * scale_q.
@@ -144,6 +172,20 @@ __device__ __forceinline__ bf16x4 pack4(float a, float b, float c, float d) {
     short bits;
     __builtin_memcpy(&bits, &h, 2);
     v[k] = x[k] != x[k] ? static_cast<short>(0x7fc0) : bits;
+  }
+  return v;
+}
+
+// pack4 of values that are not NaN.
+__device__ __forceinline__ bf16x4 pack4_finite(float a, float b, float c, float d) {
+  const float x[4] = {a, b, c, d};
+  bf16x4 v;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const __bf16 h = static_cast<__bf16>(x[k]);
+    short bits;
+    __builtin_memcpy(&bits, &h, 2);
+    v[k] = bits;
   }
   return v;
 }
