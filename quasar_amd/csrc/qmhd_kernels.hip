@@ -276,9 +276,7 @@ __device__ __forceinline__ void list_faces(bool need, std::size_t k, unsigned lo
 
 // Face (i, j) of a reconstruction launch over dir 0 faces i in [0,nx],
 // j in [-ng, ny+ng) (dir 1 transposed); false outside.
-__device__ __forceinline__ bool recon_face_of(const Blk& qb, const GridD& g, int dir, int& i, int& j) {
-  const int li = qb.x * blockDim.x + threadIdx.x;
-  const int lj = qb.y * blockDim.y + threadIdx.y;
+__device__ __forceinline__ bool recon_face_of(const GridD& g, int dir, int li, int lj, int& i, int& j) {
   i = dir == 1 ? li - g.ng : li;
   j = dir == 0 ? lj - g.ng : lj;
   if (dir == 0) return li <= g.nx && lj < g.ny + 2 * g.ng;
@@ -318,17 +316,6 @@ __device__ __forceinline__ void reconstruct_kernel_tile(
 #include "tiles/reconstruct_kernel.inc"
 }
 
-template <class T, int ORDER>
-__global__ __launch_bounds__(256, kReconWaves<T>) void reconstruct_kernel(GridD g, int dir, T gamma, int side_lo, int side_hi,
-                                                          StateView u, const double* __restrict__ bxc,
-                                                          const double* __restrict__ byc, IfaceView<T> out,
-                                                          int* __restrict__ eq_flag,
-                                                          unsigned long long* __restrict__ fb_count,
-                                                          unsigned long long* __restrict__ fb_list) {
-  [[maybe_unused]] const Blk qb = Blk::xcd_tiled();
-#include "tiles/reconstruct_kernel.inc"
-}
-
 // Queue form of reconstruct_kernel (one launch over the tiles of many runs).
 template <class T, int ORDER>
 struct reconstruct_kernel_q {
@@ -352,10 +339,6 @@ struct reconstruct_kernel_q {
                                       queue_arg(a.out), queue_arg(a.eq_flag), queue_arg(a.fb_count),
                                       queue_arg(a.fb_list));
   }
-  static void launch(dim3 grid, dim3 block, hipStream_t s, const Args& a) {
-    hipLaunchKernelGGL((reconstruct_kernel<T, ORDER>), grid, block, 0, s, a.g, a.dir, a.gamma, a.side_lo, a.side_hi,
-                       a.u, a.bxc, a.byc, a.out, a.eq_flag, a.fb_count, a.fb_list);
-  }
   static const void* tag() {
     static const char t = 0;
     return &t;
@@ -367,10 +350,11 @@ struct reconstruct_kernel_q {
 template <class T, int ORDER>
 __global__ __launch_bounds__(256, kReconWaves<T>) void reconstruct_kernel_queue(
     const typename reconstruct_kernel_q<T, ORDER>::Args* __restrict__ qargs, const QueueRun* __restrict__ qruns,
-    int qnruns) {
-  const QueueTile qtile = queue_tile(qruns, qnruns);
+    int qnruns,
+    Pair<typename reconstruct_kernel_q<T, ORDER>::Args>) {
+  const auto qtile = tile_of(qargs, qruns, qnruns);
   [[maybe_unused]] const Blk qb = qtile.blk;
-  const typename reconstruct_kernel_q<T, ORDER>::Args& qa = qargs[qtile.run];
+  const auto& qa = qtile.args;
   GridD g = qa.g;
   int dir = qa.dir;
   T gamma = qa.gamma;
@@ -386,6 +370,11 @@ __global__ __launch_bounds__(256, kReconWaves<T>) void reconstruct_kernel_queue(
 #include "tiles/reconstruct_kernel.inc"
 }
 template <class T, int ORDER>
+struct Paired<reconstruct_kernel_q<T, ORDER>> {
+  static constexpr bool value = true;
+  static constexpr unsigned xcd = 1u;
+};
+template <class T, int ORDER>
 struct QueueTiles<reconstruct_kernel_q<T, ORDER>> {
   static constexpr auto kernel = &reconstruct_kernel_queue<T, ORDER>;
 };
@@ -400,20 +389,6 @@ __device__ __forceinline__ void reconstruct_list_kernel_tile(
     const unsigned long long* __restrict__ list_count, const unsigned long long* __restrict__ list,
     unsigned long long* __restrict__ fb_count, unsigned long long* __restrict__ fb_list,
     unsigned long long* __restrict__ plain_total) {
-#include "tiles/reconstruct_list_kernel.inc"
-}
-
-template <class T, int ORDER>
-__global__ __launch_bounds__(256) void reconstruct_list_kernel(GridD g, int dir, T gamma, StateView u,
-                                                               const double* __restrict__ bxc,
-                                                               const double* __restrict__ byc, IfaceView<T> out,
-                                                               int* __restrict__ eq_flag,
-                                                               const unsigned long long* __restrict__ list_count,
-                                                               const unsigned long long* __restrict__ list,
-                                                               unsigned long long* __restrict__ fb_count,
-                                                               unsigned long long* __restrict__ fb_list,
-                                                               unsigned long long* __restrict__ plain_total) {
-  [[maybe_unused]] const Blk qb = Blk::native();
 #include "tiles/reconstruct_list_kernel.inc"
 }
 
@@ -441,10 +416,6 @@ struct reconstruct_list_kernel_q {
                                            queue_arg(a.list_count), queue_arg(a.list), queue_arg(a.fb_count),
                                            queue_arg(a.fb_list), queue_arg(a.plain_total));
   }
-  static void launch(dim3 grid, dim3 block, hipStream_t s, const Args& a) {
-    hipLaunchKernelGGL((reconstruct_list_kernel<T, ORDER>), grid, block, 0, s, a.g, a.dir, a.gamma, a.u, a.bxc, a.byc,
-                       a.out, a.eq_flag, a.list_count, a.list, a.fb_count, a.fb_list, a.plain_total);
-  }
   static const void* tag() {
     static const char t = 0;
     return &t;
@@ -456,10 +427,11 @@ struct reconstruct_list_kernel_q {
 template <class T, int ORDER>
 __global__ __launch_bounds__(256) void reconstruct_list_kernel_queue(
     const typename reconstruct_list_kernel_q<T, ORDER>::Args* __restrict__ qargs, const QueueRun* __restrict__ qruns,
-    int qnruns) {
-  const QueueTile qtile = queue_tile(qruns, qnruns);
+    int qnruns,
+    Pair<typename reconstruct_list_kernel_q<T, ORDER>::Args>) {
+  const auto qtile = tile_of(qargs, qruns, qnruns);
   [[maybe_unused]] const Blk qb = qtile.blk;
-  const typename reconstruct_list_kernel_q<T, ORDER>::Args& qa = qargs[qtile.run];
+  const auto& qa = qtile.args;
   GridD g = qa.g;
   int dir = qa.dir;
   T gamma = qa.gamma;
@@ -476,6 +448,11 @@ __global__ __launch_bounds__(256) void reconstruct_list_kernel_queue(
 #include "tiles/reconstruct_list_kernel.inc"
 }
 template <class T, int ORDER>
+struct Paired<reconstruct_list_kernel_q<T, ORDER>> {
+  static constexpr bool value = true;
+  static constexpr unsigned xcd = 0u;
+};
+template <class T, int ORDER>
 struct QueueTiles<reconstruct_list_kernel_q<T, ORDER>> {
   static constexpr auto kernel = &reconstruct_list_kernel_queue<T, ORDER>;
 };
@@ -487,18 +464,6 @@ __device__ __forceinline__ void reconstruct_fallback_kernel_tile(
     const Blk& qb, const GridD& g, int dir, T gamma, int side_lo, int side_hi, const StateView& u,
     const double* __restrict__ bxc, const double* __restrict__ byc, const IfaceView<T>& out, int* __restrict__ eq_flag,
     const unsigned long long* __restrict__ fb_count, const unsigned long long* __restrict__ fb_list) {
-#include "tiles/reconstruct_fallback_kernel.inc"
-}
-
-template <class T, int ORDER>
-__global__ __launch_bounds__(256) void reconstruct_fallback_kernel(GridD g, int dir, T gamma, int side_lo,
-                                                                   int side_hi, StateView u,
-                                                                   const double* __restrict__ bxc,
-                                                                   const double* __restrict__ byc, IfaceView<T> out,
-                                                                   int* __restrict__ eq_flag,
-                                                                   const unsigned long long* __restrict__ fb_count,
-                                                                   const unsigned long long* __restrict__ fb_list) {
-  [[maybe_unused]] const Blk qb = Blk::native();
 #include "tiles/reconstruct_fallback_kernel.inc"
 }
 
@@ -525,10 +490,6 @@ struct reconstruct_fallback_kernel_q {
                                                queue_arg(a.bxc), queue_arg(a.byc), queue_arg(a.out),
                                                queue_arg(a.eq_flag), queue_arg(a.fb_count), queue_arg(a.fb_list));
   }
-  static void launch(dim3 grid, dim3 block, hipStream_t s, const Args& a) {
-    hipLaunchKernelGGL((reconstruct_fallback_kernel<T, ORDER>), grid, block, 0, s, a.g, a.dir, a.gamma, a.side_lo,
-                       a.side_hi, a.u, a.bxc, a.byc, a.out, a.eq_flag, a.fb_count, a.fb_list);
-  }
   static const void* tag() {
     static const char t = 0;
     return &t;
@@ -540,10 +501,11 @@ struct reconstruct_fallback_kernel_q {
 template <class T, int ORDER>
 __global__ __launch_bounds__(256) void reconstruct_fallback_kernel_queue(
     const typename reconstruct_fallback_kernel_q<T, ORDER>::Args* __restrict__ qargs,
-    const QueueRun* __restrict__ qruns, int qnruns) {
-  const QueueTile qtile = queue_tile(qruns, qnruns);
+    const QueueRun* __restrict__ qruns, int qnruns,
+    Pair<typename reconstruct_fallback_kernel_q<T, ORDER>::Args>) {
+  const auto qtile = tile_of(qargs, qruns, qnruns);
   [[maybe_unused]] const Blk qb = qtile.blk;
-  const typename reconstruct_fallback_kernel_q<T, ORDER>::Args& qa = qargs[qtile.run];
+  const auto& qa = qtile.args;
   GridD g = qa.g;
   int dir = qa.dir;
   T gamma = qa.gamma;
@@ -559,95 +521,18 @@ __global__ __launch_bounds__(256) void reconstruct_fallback_kernel_queue(
 #include "tiles/reconstruct_fallback_kernel.inc"
 }
 template <class T, int ORDER>
+struct Paired<reconstruct_fallback_kernel_q<T, ORDER>> {
+  static constexpr bool value = true;
+  static constexpr unsigned xcd = 0u;
+};
+template <class T, int ORDER>
 struct QueueTiles<reconstruct_fallback_kernel_q<T, ORDER>> {
   static constexpr auto kernel = &reconstruct_fallback_kernel_queue<T, ORDER>;
 };
-
-__device__ __forceinline__ void counter_reset_kernel_tile(const Blk& qb, unsigned long long* __restrict__ c) {
-#include "tiles/counter_reset_kernel.inc"
+// Zeroes face-list counters (the solver's own are zeroed by its prep launches).
+__global__ void counter_reset_kernel(unsigned long long* __restrict__ c, int n) {
+  if (static_cast<int>(threadIdx.x) < n) c[threadIdx.x] = 0ull;
 }
-
-__global__ void counter_reset_kernel(unsigned long long* __restrict__ c) {
-  [[maybe_unused]] const Blk qb = Blk::native();
-#include "tiles/counter_reset_kernel.inc"
-}
-
-// Queue form of counter_reset_kernel (one launch over the tiles of many runs).
-struct counter_reset_kernel_q {
-  struct Args {
-    unsigned long long* c;
-  };
-  static __device__ __forceinline__ void run(const Blk& qb, const Args& a) {
-    counter_reset_kernel_tile(qb, queue_arg(a.c));
-  }
-  static void launch(dim3 grid, dim3 block, hipStream_t s, const Args& a) {
-    hipLaunchKernelGGL((counter_reset_kernel), grid, block, 0, s, a.c);
-  }
-  static const void* tag() {
-    static const char t = 0;
-    return &t;
-  }
-};
-
-// counter_reset_kernel over the tile queue, one workgroup per tile: the same text, the
-// arguments read from the tile's run record.
-__global__ void counter_reset_kernel_queue(const counter_reset_kernel_q::Args* __restrict__ qargs,
-    const QueueRun* __restrict__ qruns, int qnruns) {
-  const QueueTile qtile = queue_tile(qruns, qnruns);
-  [[maybe_unused]] const Blk qb = qtile.blk;
-  const counter_reset_kernel_q::Args& qa = qargs[qtile.run];
-  unsigned long long* __restrict__ c = queue_arg(qa.c);
-#include "tiles/counter_reset_kernel.inc"
-}
-template <>
-struct QueueTiles<counter_reset_kernel_q> {
-  static constexpr auto kernel = &counter_reset_kernel_queue;
-};
-
-// Both list counters of a learned reconstruction launch, in one launch.
-__device__ __forceinline__ void counter_pair_reset_kernel_tile(const Blk& qb, unsigned long long* __restrict__ a,
-                                                               unsigned long long* __restrict__ b) {
-#include "tiles/counter_pair_reset_kernel.inc"
-}
-
-__global__ void counter_pair_reset_kernel(unsigned long long* __restrict__ a, unsigned long long* __restrict__ b) {
-  [[maybe_unused]] const Blk qb = Blk::native();
-#include "tiles/counter_pair_reset_kernel.inc"
-}
-
-// Queue form of counter_pair_reset_kernel (one launch over the tiles of many runs).
-struct counter_pair_reset_kernel_q {
-  struct Args {
-    unsigned long long* a;
-    unsigned long long* b;
-  };
-  static __device__ __forceinline__ void run(const Blk& qb, const Args& a) {
-    counter_pair_reset_kernel_tile(qb, queue_arg(a.a), queue_arg(a.b));
-  }
-  static void launch(dim3 grid, dim3 block, hipStream_t s, const Args& a) {
-    hipLaunchKernelGGL((counter_pair_reset_kernel), grid, block, 0, s, a.a, a.b);
-  }
-  static const void* tag() {
-    static const char t = 0;
-    return &t;
-  }
-};
-
-// counter_pair_reset_kernel over the tile queue, one workgroup per tile: the same text, the
-// arguments read from the tile's run record.
-__global__ void counter_pair_reset_kernel_queue(const counter_pair_reset_kernel_q::Args* __restrict__ qargs,
-    const QueueRun* __restrict__ qruns, int qnruns) {
-  const QueueTile qtile = queue_tile(qruns, qnruns);
-  [[maybe_unused]] const Blk qb = qtile.blk;
-  const counter_pair_reset_kernel_q::Args& qa = qargs[qtile.run];
-  unsigned long long* __restrict__ a = queue_arg(qa.a);
-  unsigned long long* __restrict__ b = queue_arg(qa.b);
-#include "tiles/counter_pair_reset_kernel.inc"
-}
-template <>
-struct QueueTiles<counter_pair_reset_kernel_q> {
-  static constexpr auto kernel = &counter_pair_reset_kernel_queue;
-};
 
 // Learned form, one thread per face: a face whose two cells the indicator
 // left unflagged takes the linear fifth-order upwind-biased face values (the
@@ -816,28 +701,30 @@ __device__ __forceinline__ void store_face(const GridD& g, int dir, const FluxVi
 // / 795 us.  In the hardware's tile order the x faces take 565 us.
 constexpr int kFluxTiles[2][2] = {{16, 16}, {32, 8}};
 constexpr int kFluxListBlock = 64;
+// Waves per SIMD of the face flux: both directions in one kernel take 147
+// registers in FP32 (119 / 127 apart), past four waves.
+template <class T>
+constexpr int kFluxWaves = sizeof(T) == 4 ? 4 : 2;
+template <int ORDER>
+constexpr int flux_tile_values() {
+  constexpr int more = ORDER == 5 ? 3 : 5;
+  constexpr int x = kFluxTiles[0][0] * (kFluxTiles[0][1] + more), y = (kFluxTiles[1][0] + more) * kFluxTiles[1][1];
+  return 16 * (x > y ? x : y);
+}
 
-// One instantiation per direction: the direction's component swaps and
-// stencil stride fold at compile time.
-template <class T, int ORDER, bool LF, int DIR>
+template <class T, int ORDER, bool LF>
 __device__ __forceinline__ void flux_kernel_tile(
-    const Blk& qb, const GridD& g, int periodic_dir, T gamma, const IfaceView<T>& in, const FluxView<T>& flux,
+    const Blk& qb, const GridD& g, int dir, int periodic_dir, T gamma, const IfaceView<T>& in, const FluxView<T>& flux,
     double* __restrict__ rate) {
 #include "tiles/flux_kernel.inc"
 }
 
-template <class T, int ORDER, bool LF, int DIR>
-__global__ __launch_bounds__(256) void flux_kernel(GridD g, int periodic_dir, T gamma, IfaceView<T> in,
-                                                   FluxView<T> flux, double* __restrict__ rate) {
-  [[maybe_unused]] const Blk qb = ORDER >= 5 ? Blk::xcd_tiled() : Blk::native();
-#include "tiles/flux_kernel.inc"
-}
-
 // Queue form of flux_kernel (one launch over the tiles of many runs).
-template <class T, int ORDER, bool LF, int DIR>
+template <class T, int ORDER, bool LF>
 struct flux_kernel_q {
   struct Args {
     GridD g;
+    int dir;
     int periodic_dir;
     T gamma;
     IfaceView<T> in;
@@ -845,12 +732,8 @@ struct flux_kernel_q {
     double* rate;
   };
   static __device__ __forceinline__ void run(const Blk& qb, const Args& a) {
-    flux_kernel_tile<T, ORDER, LF, DIR>(qb, queue_arg(a.g), queue_arg(a.periodic_dir), queue_arg(a.gamma),
+    flux_kernel_tile<T, ORDER, LF>(qb, queue_arg(a.g), queue_arg(a.dir), queue_arg(a.periodic_dir), queue_arg(a.gamma),
                                         queue_arg(a.in), queue_arg(a.flux), queue_arg(a.rate));
-  }
-  static void launch(dim3 grid, dim3 block, hipStream_t s, const Args& a) {
-    hipLaunchKernelGGL((flux_kernel<T, ORDER, LF, DIR>), grid, block, 0, s, a.g, a.periodic_dir, a.gamma, a.in, a.flux,
-                       a.rate);
   }
   static const void* tag() {
     static const char t = 0;
@@ -860,14 +743,16 @@ struct flux_kernel_q {
 
 // flux_kernel over the tile queue, one workgroup per tile: the same text, the
 // arguments read from the tile's run record.
-template <class T, int ORDER, bool LF, int DIR>
-__global__ __launch_bounds__(256) void flux_kernel_queue(
-    const typename flux_kernel_q<T, ORDER, LF, DIR>::Args* __restrict__ qargs, const QueueRun* __restrict__ qruns,
-    int qnruns) {
-  const QueueTile qtile = queue_tile(qruns, qnruns);
+template <class T, int ORDER, bool LF>
+__global__ __launch_bounds__(256, kFluxWaves<T>) void flux_kernel_queue(
+    const typename flux_kernel_q<T, ORDER, LF>::Args* __restrict__ qargs, const QueueRun* __restrict__ qruns,
+    int qnruns,
+    Pair<typename flux_kernel_q<T, ORDER, LF>::Args>) {
+  const auto qtile = tile_of(qargs, qruns, qnruns);
   [[maybe_unused]] const Blk qb = qtile.blk;
-  const typename flux_kernel_q<T, ORDER, LF, DIR>::Args& qa = qargs[qtile.run];
+  const auto& qa = qtile.args;
   GridD g = qa.g;
+  const int dir = qa.dir;
   int periodic_dir = qa.periodic_dir;
   T gamma = qa.gamma;
   IfaceView<T> in = queue_arg(qa.in);
@@ -875,9 +760,14 @@ __global__ __launch_bounds__(256) void flux_kernel_queue(
   double* __restrict__ rate = queue_arg(qa.rate);
 #include "tiles/flux_kernel.inc"
 }
-template <class T, int ORDER, bool LF, int DIR>
-struct QueueTiles<flux_kernel_q<T, ORDER, LF, DIR>> {
-  static constexpr auto kernel = &flux_kernel_queue<T, ORDER, LF, DIR>;
+template <class T, int ORDER, bool LF>
+struct Paired<flux_kernel_q<T, ORDER, LF>> {
+  static constexpr bool value = true;
+  static constexpr unsigned xcd = 1u;
+};
+template <class T, int ORDER, bool LF>
+struct QueueTiles<flux_kernel_q<T, ORDER, LF>> {
+  static constexpr auto kernel = &flux_kernel_queue<T, ORDER, LF>;
 };
 
 // Learned form: the flux of the faces on the plain reconstruction's list,
@@ -888,8 +778,8 @@ struct QueueTiles<flux_kernel_q<T, ORDER, LF, DIR>> {
 // skipped; a periodic high face takes its low partner's flux.  A bounded grid
 // strides over the list; one wave per block, its lanes' neighbour differences
 // in LDS (24 KB in FP32).
-template <class T, int ORDER, int DIR>
-__device__ __forceinline__ void flux_plain_list_kernel_tile(const Blk& qb, const GridD& g, int periodic_dir, T gamma,
+template <class T, int ORDER>
+__device__ __forceinline__ void flux_plain_list_kernel_tile(const Blk& qb, const GridD& g, int dir, int periodic_dir, T gamma,
                                                               const IfaceView<T>& in, const FluxView<T>& flux,
                                                               double* __restrict__ rate,
                                                               const uint8_t* __restrict__ cell_flags,
@@ -898,22 +788,12 @@ __device__ __forceinline__ void flux_plain_list_kernel_tile(const Blk& qb, const
 #include "tiles/flux_plain_list_kernel.inc"
 }
 
-template <class T, int ORDER, int DIR>
-__global__ __launch_bounds__(kFluxListBlock) void flux_plain_list_kernel(GridD g, int periodic_dir, T gamma,
-                                                              IfaceView<T> in, FluxView<T> flux,
-                                                              double* __restrict__ rate,
-                                                              const uint8_t* __restrict__ cell_flags,
-                                                              const unsigned long long* __restrict__ fb_count,
-                                                              const unsigned long long* __restrict__ fb_list) {
-  [[maybe_unused]] const Blk qb = Blk::native();
-#include "tiles/flux_plain_list_kernel.inc"
-}
-
 // Queue form of flux_plain_list_kernel (one launch over the tiles of many runs).
-template <class T, int ORDER, int DIR>
+template <class T, int ORDER>
 struct flux_plain_list_kernel_q {
   struct Args {
     GridD g;
+    int dir;
     int periodic_dir;
     T gamma;
     IfaceView<T> in;
@@ -924,13 +804,9 @@ struct flux_plain_list_kernel_q {
     const unsigned long long* fb_list;
   };
   static __device__ __forceinline__ void run(const Blk& qb, const Args& a) {
-    flux_plain_list_kernel_tile<T, ORDER, DIR>(qb, queue_arg(a.g), queue_arg(a.periodic_dir), queue_arg(a.gamma),
+    flux_plain_list_kernel_tile<T, ORDER>(qb, queue_arg(a.g), queue_arg(a.dir), queue_arg(a.periodic_dir), queue_arg(a.gamma),
                                                queue_arg(a.in), queue_arg(a.flux), queue_arg(a.rate),
                                                queue_arg(a.cell_flags), queue_arg(a.fb_count), queue_arg(a.fb_list));
-  }
-  static void launch(dim3 grid, dim3 block, hipStream_t s, const Args& a) {
-    hipLaunchKernelGGL((flux_plain_list_kernel<T, ORDER, DIR>), grid, block, 0, s, a.g, a.periodic_dir, a.gamma, a.in,
-                       a.flux, a.rate, a.cell_flags, a.fb_count, a.fb_list);
   }
   static const void* tag() {
     static const char t = 0;
@@ -940,14 +816,16 @@ struct flux_plain_list_kernel_q {
 
 // flux_plain_list_kernel over the tile queue, one workgroup per tile: the same text, the
 // arguments read from the tile's run record.
-template <class T, int ORDER, int DIR>
+template <class T, int ORDER>
 __global__ __launch_bounds__(kFluxListBlock) void flux_plain_list_kernel_queue(
-    const typename flux_plain_list_kernel_q<T, ORDER, DIR>::Args* __restrict__ qargs,
-    const QueueRun* __restrict__ qruns, int qnruns) {
-  const QueueTile qtile = queue_tile(qruns, qnruns);
+    const typename flux_plain_list_kernel_q<T, ORDER>::Args* __restrict__ qargs,
+    const QueueRun* __restrict__ qruns, int qnruns,
+    Pair<typename flux_plain_list_kernel_q<T, ORDER>::Args>) {
+  const auto qtile = tile_of(qargs, qruns, qnruns);
   [[maybe_unused]] const Blk qb = qtile.blk;
-  const typename flux_plain_list_kernel_q<T, ORDER, DIR>::Args& qa = qargs[qtile.run];
+  const auto& qa = qtile.args;
   GridD g = qa.g;
+  const int dir = qa.dir;
   int periodic_dir = qa.periodic_dir;
   T gamma = qa.gamma;
   IfaceView<T> in = queue_arg(qa.in);
@@ -958,9 +836,14 @@ __global__ __launch_bounds__(kFluxListBlock) void flux_plain_list_kernel_queue(
   const unsigned long long* __restrict__ fb_list = queue_arg(qa.fb_list);
 #include "tiles/flux_plain_list_kernel.inc"
 }
-template <class T, int ORDER, int DIR>
-struct QueueTiles<flux_plain_list_kernel_q<T, ORDER, DIR>> {
-  static constexpr auto kernel = &flux_plain_list_kernel_queue<T, ORDER, DIR>;
+template <class T, int ORDER>
+struct Paired<flux_plain_list_kernel_q<T, ORDER>> {
+  static constexpr bool value = true;
+  static constexpr unsigned xcd = 0u;
+};
+template <class T, int ORDER>
+struct QueueTiles<flux_plain_list_kernel_q<T, ORDER>> {
+  static constexpr auto kernel = &flux_plain_list_kernel_queue<T, ORDER>;
 };
 
 // Additive cell CFL rate from the incident face rates, reduced to the maximum.
@@ -2074,156 +1957,155 @@ void launch_collocate(const GridD& g, int axis, int co, const double* face, doub
                      cell);
 }
 
+void launch_counter_reset(unsigned long long* counters, int n, hipStream_t stream) {
+  hipLaunchKernelGGL(counter_reset_kernel, dim3(1), dim3(64), 0, stream, counters, n);
+}
+
+// Faces of a reconstruction launch along x and y.
+static dim3 recon_faces(const GridD& g, int dir) {
+  return dir == 0 ? dim3(g.nx + 1, g.ny + 2 * g.ng) : dim3(g.nx + 2 * g.ng, g.ny + 1);
+}
+// Blocks over a face list: no more than it can fill (a queue batch launches
+// every run's).
+static dim3 list_blocks_of(const GridD& g, int dir, std::size_t most) {
+  const dim3 l = recon_faces(g, dir);
+  return dim3(static_cast<unsigned>(std::min<std::size_t>(most, (static_cast<std::size_t>(l.x) * l.y + 255) / 256)));
+}
+static int periodic_of(const Flags4& flags, int dir) {
+  return flags.side[2 * dir] == 0 && flags.side[2 * dir + 1] == 0;
+}
+
 template <class T>
-void launch_reconstruct(const GridD& g, int dir, int order, double gamma, const Flags4& flags, const StateView& u,
-                        const double* bxc, const double* byc, const IfaceView<T>& out, int* eq,
-                        unsigned long long* fb_count, unsigned long long* fb_list, hipStream_t stream) {
-  const dim3 b = order >= 5 ? dim3(kReconTiles[dir][0], kReconTiles[dir][1]) : dim3(64, 4);
-  const int lx = dir == 0 ? g.nx + 1 : g.nx + 2 * g.ng;
-  const int ly = dir == 0 ? g.ny + 2 * g.ng : g.ny + 1;
-  const int slo = dir == 0 ? flags.side[0] : flags.side[2];
-  const int shi = dir == 0 ? flags.side[1] : flags.side[3];
-  const dim3 grid = blocks2d(lx, ly, b);
-  // No more blocks than the list can fill: a queue batch launches every run's.
-  const std::size_t slots = (static_cast<std::size_t>(lx) * ly + 255) / 256;
-  const dim3 fb_block(256), fb_grid(static_cast<unsigned>(std::min<std::size_t>(64, slots)));
+void launch_reconstruct(const GridD& g, int order, double gamma, const Flags4& flags, const StateView& u,
+                        const double* bxc, const double* byc, const FaceOut<T>* out, int first, int count,
+                        hipStream_t stream) {
   const T gamma_t = T(gamma);
-  auto faces = [&](auto q) {
-    go<decltype(q)>(grid, b, stream, g, dir, gamma_t, slo, shi, u, bxc, byc, out, eq, fb_count, fb_list);
-  };
-  auto fallback = [&](auto q) {
-    go<decltype(q)>(fb_grid, fb_block, stream, g, dir, gamma_t, slo, shi, u, bxc, byc, out, eq,
-                    static_cast<const unsigned long long*>(fb_count), static_cast<const unsigned long long*>(fb_list));
+  auto launch = [&](auto faces, auto fallback) {
+    using F = decltype(faces);
+    using B = decltype(fallback);
+    dim3 grid[2]{dim3(0, 0), dim3(0, 0)}, fb_grid[2]{dim3(0, 0), dim3(0, 0)};
+    typename F::Args a[2];
+    typename B::Args b[2];
+    for (int k = 0; k < 2; ++k) {
+      const int dir = k < count ? first + k : first;
+      const FaceOut<T>& o = out[k < count ? k : 0];
+      const int slo = flags.side[2 * dir], shi = flags.side[2 * dir + 1];
+      a[k] = {g, dir, gamma_t, slo, shi, u, bxc, byc, o.states, o.eq, o.list.count, o.list.faces};
+      b[k] = {g, dir, gamma_t, slo, shi, u, bxc, byc, o.states, o.eq, o.list.count, o.list.faces};
+      if (k >= count) continue;
+      const dim3 l = recon_faces(g, dir);
+      grid[k] = blocks2d(l.x, l.y, dim3(kReconTiles[dir][0], kReconTiles[dir][1]));
+      fb_grid[k] = list_blocks_of(g, dir, 64);
+    }
+    go_pair<F>(grid[0], a[0], grid[1], a[1], dim3(256), stream);
+    if (order >= 5) go_pair<B>(fb_grid[0], b[0], fb_grid[1], b[1], dim3(256), stream);
   };
   switch (order) {
-    case 1:
-      faces(reconstruct_kernel_q<T, 1>{});
-      break;
-    case 2:
-      faces(reconstruct_kernel_q<T, 2>{});
-      break;
-    case 5:
-      go<counter_reset_kernel_q>(dim3(1), dim3(64), stream, fb_count);
-      faces(reconstruct_kernel_q<T, 5>{});
-      fallback(reconstruct_fallback_kernel_q<T, 5>{});
-      break;
-    default:
-      go<counter_reset_kernel_q>(dim3(1), dim3(64), stream, fb_count);
-      faces(reconstruct_kernel_q<T, 7>{});
-      fallback(reconstruct_fallback_kernel_q<T, 7>{});
-      break;
+    case 1: launch(reconstruct_kernel_q<T, 1>{}, reconstruct_fallback_kernel_q<T, 5>{}); break;
+    case 2: launch(reconstruct_kernel_q<T, 2>{}, reconstruct_fallback_kernel_q<T, 5>{}); break;
+    case 5: launch(reconstruct_kernel_q<T, 5>{}, reconstruct_fallback_kernel_q<T, 5>{}); break;
+    default: launch(reconstruct_kernel_q<T, 7>{}, reconstruct_fallback_kernel_q<T, 7>{}); break;
   }
 }
 
 template <class T>
-void launch_reconstruct_learned(const GridD& g, int dir, int order, double gamma, const Flags4& flags,
-                                const StateView& u, const double* bxc, const double* byc, const uint8_t* cell_flags,
-                                const IfaceView<T>& out, int* eq, unsigned long long* fb_count,
-                                unsigned long long* fb_list, unsigned long long* fb2_count,
-                                unsigned long long* fb2_list, unsigned long long* plain_total,
-                                const FluxView<T>& flux, double* rate, hipStream_t stream, int list_blocks,
-                                int cheap_tile) {
-  if (cheap_tile < 0 || cheap_tile >= kCheapTileCount)
-    throw std::invalid_argument("reconstruct launch: cheap tile choice is 0..4");
-  const int periodic = dir == 0 ? (flags.side[0] == 0 && flags.side[1] == 0) : (flags.side[2] == 0 && flags.side[3] == 0);
-  const int lx = dir == 0 ? g.nx + 1 : g.nx + 2 * g.ng;
-  const int ly = dir == 0 ? g.ny + 2 * g.ng : g.ny + 1;
-  const int slo = dir == 0 ? flags.side[0] : flags.side[2];
-  const int shi = dir == 0 ? flags.side[1] : flags.side[3];
+void launch_reconstruct_learned(const GridD& g, int order, double gamma, const Flags4& flags, const StateView& u,
+                                const double* bxc, const double* byc, const uint8_t* cell_flags,
+                                const FaceOut<T>* out, unsigned long long* plain_total, hipStream_t stream,
+                                int list_blocks, const int* cheap_tile) {
   const T gamma_t = T(gamma);
+  for (int dir = 0; dir < 2; ++dir) {
+    if (cheap_tile[dir] < 0 || cheap_tile[dir] >= kCheapTileCount)
+      throw std::invalid_argument("reconstruct launch: cheap tile choice is 0..4");
+  }
+  for (int dir = 0; dir < 2; ++dir) {
+    const dim3 l = recon_faces(g, dir), cb(kCheapTiles[cheap_tile[dir]][0], kCheapTiles[cheap_tile[dir]][1]);
+    const FaceOut<T>& o = out[dir];
+    auto cheap = [&](auto q) {
+      go<decltype(q)>(blocks2d(l.x, l.y, cb), cb, stream, g, dir, gamma_t, u, bxc, byc, cell_flags, o.states, o.eq,
+                      o.list.count, o.list.faces, o.flux, o.rate, periodic_of(flags, dir));
+    };
+    switch (cheap_tile[dir]) {
+      case 0: cheap(cheap_reconstruct_kernel_q<T, kCheapTiles[0][0], kCheapTiles[0][1]>{}); break;
+      case 1: cheap(cheap_reconstruct_kernel_q<T, kCheapTiles[1][0], kCheapTiles[1][1]>{}); break;
+      case 2: cheap(cheap_reconstruct_kernel_q<T, kCheapTiles[2][0], kCheapTiles[2][1]>{}); break;
+      case 3: cheap(cheap_reconstruct_kernel_q<T, kCheapTiles[3][0], kCheapTiles[3][1]>{}); break;
+      default: cheap(cheap_reconstruct_kernel_q<T, kCheapTiles[4][0], kCheapTiles[4][1]>{}); break;
+    }
+  }
   // Enough blocks to fill the device at the MP kernel's occupancy (the plain
   // list can hold a large share of the faces), no more than the list can fill:
   // one block per possible slot spent 25 us at 4096^2 on blocks without work.
-  const std::size_t slots = (static_cast<std::size_t>(lx) * ly + 255) / 256;
-  const dim3 list_block(256), list_grid(static_cast<unsigned>(std::min<std::size_t>(list_blocks, slots)));
-  go<counter_pair_reset_kernel_q>(dim3(1), dim3(64), stream, fb_count, fb2_count);
-  const dim3 cb(kCheapTiles[cheap_tile][0], kCheapTiles[cheap_tile][1]);
-  auto cheap = [&](auto q) {
-    go<decltype(q)>(blocks2d(lx, ly, cb), cb, stream, g, dir, gamma_t, u, bxc, byc, cell_flags, out, eq, fb_count,
-                    fb_list, flux, rate, periodic);
-  };
-  switch (cheap_tile) {
-    case 0: cheap(cheap_reconstruct_kernel_q<T, kCheapTiles[0][0], kCheapTiles[0][1]>{}); break;
-    case 1: cheap(cheap_reconstruct_kernel_q<T, kCheapTiles[1][0], kCheapTiles[1][1]>{}); break;
-    case 2: cheap(cheap_reconstruct_kernel_q<T, kCheapTiles[2][0], kCheapTiles[2][1]>{}); break;
-    case 3: cheap(cheap_reconstruct_kernel_q<T, kCheapTiles[3][0], kCheapTiles[3][1]>{}); break;
-    default: cheap(cheap_reconstruct_kernel_q<T, kCheapTiles[4][0], kCheapTiles[4][1]>{}); break;
-  }
-  const unsigned long long* list_count = fb_count;
-  const unsigned long long* list = fb_list;
-  auto listed = [&](auto q) {
-    go<decltype(q)>(list_grid, list_block, stream, g, dir, gamma_t, u, bxc, byc, out, eq, list_count, list, fb2_count,
-                    fb2_list, plain_total);
-  };
-  const unsigned long long* fb2c = fb2_count;
-  const unsigned long long* fb2l = fb2_list;
-  auto fallback = [&](auto q) {
-    go<decltype(q)>(list_grid, list_block, stream, g, dir, gamma_t, slo, shi, u, bxc, byc, out, eq, fb2c, fb2l);
-  };
-  if (order == 5) {
-    listed(reconstruct_list_kernel_q<T, 5>{});
-    fallback(reconstruct_fallback_kernel_q<T, 5>{});
-  } else {
-    listed(reconstruct_list_kernel_q<T, 7>{});
-    fallback(reconstruct_fallback_kernel_q<T, 7>{});
-  }
-}
-
-template <class T>
-void launch_flux(const GridD& g, int dir, int order, int hll_only, const Flags4& flags, double gamma,
-                 const IfaceView<T>& in, const FluxView<T>& flux, double* rate, hipStream_t stream,
-                 dim3 b) {
-  const T gm = T(gamma);
-  if (order == 5 || order == 7) b = dim3(kFluxTiles[dir][0], kFluxTiles[dir][1]);
-  const dim3 grid = blocks2d(g.nx + 1, g.ny + 1, b);
-  const int periodic = dir == 0 ? (flags.side[0] == 0 && flags.side[1] == 0) : (flags.side[2] == 0 && flags.side[3] == 0);
-  auto one_lane = [&](auto qx, auto qy) {
-    if (dir == 0)
-      go<decltype(qx)>(grid, b, stream, g, periodic, gm, in, flux, rate);
-    else
-      go<decltype(qy)>(grid, b, stream, g, periodic, gm, in, flux, rate);
-  };
-  switch (order) {
-    case 1:
-      hll_only ? one_lane(flux_kernel_q<T, 1, true, 0>{}, flux_kernel_q<T, 1, true, 1>{})
-               : one_lane(flux_kernel_q<T, 1, false, 0>{}, flux_kernel_q<T, 1, false, 1>{});
-      break;
-    case 2:
-      hll_only ? one_lane(flux_kernel_q<T, 2, true, 0>{}, flux_kernel_q<T, 2, true, 1>{})
-               : one_lane(flux_kernel_q<T, 2, false, 0>{}, flux_kernel_q<T, 2, false, 1>{});
-      break;
-    case 5:
-      hll_only ? one_lane(flux_kernel_q<T, 5, true, 0>{}, flux_kernel_q<T, 5, true, 1>{})
-               : one_lane(flux_kernel_q<T, 5, false, 0>{}, flux_kernel_q<T, 5, false, 1>{});
-      break;
-    default:
-      hll_only ? one_lane(flux_kernel_q<T, 7, true, 0>{}, flux_kernel_q<T, 7, true, 1>{})
-               : one_lane(flux_kernel_q<T, 7, false, 0>{}, flux_kernel_q<T, 7, false, 1>{});
-      break;
-  }
-}
-
-template <class T>
-void launch_flux_learned(const GridD& g, int dir, int order, const Flags4& flags, double gamma,
-                         const IfaceView<T>& in, const FluxView<T>& flux, double* rate, const uint8_t* cell_flags,
-                         const unsigned long long* fb_count, const unsigned long long* fb_list, hipStream_t stream,
-                         int list_blocks) {
-  if (order != 5 && order != 7) throw std::invalid_argument("flux launch: the learned form runs MP5/MP7");
-  const T gm = T(gamma);
-  const int periodic = dir == 0 ? (flags.side[0] == 0 && flags.side[1] == 0) : (flags.side[2] == 0 && flags.side[3] == 0);
-  // The list holds at most the reconstruction launch's faces.
-  const std::size_t max_list = dir == 0 ? static_cast<std::size_t>(g.nx + 1) * (g.ny + 2 * g.ng)
-                                        : static_cast<std::size_t>(g.nx + 2 * g.ng) * (g.ny + 1);
-  const std::size_t fill = static_cast<std::size_t>(list_blocks) * 256 / kFluxListBlock;
-  const dim3 list_block(kFluxListBlock),
-      list_grid(static_cast<unsigned>(std::min(fill, (max_list + kFluxListBlock - 1) / kFluxListBlock)));
-  auto listed = [&](auto q) {
-    go<decltype(q)>(list_grid, list_block, stream, g, periodic, gm, in, flux, rate, cell_flags, fb_count, fb_list);
+  auto launch = [&](auto listed, auto fallback) {
+    using F = decltype(listed);
+    using B = decltype(fallback);
+    dim3 grid[2];
+    typename F::Args a[2];
+    typename B::Args b[2];
+    for (int dir = 0; dir < 2; ++dir) {
+      const FaceOut<T>& o = out[dir];
+      grid[dir] = list_blocks_of(g, dir, list_blocks);
+      a[dir] = {g, dir, gamma_t, u, bxc, byc, o.states, o.eq, o.list.count, o.list.faces, o.redo.count, o.redo.faces,
+                plain_total};
+      b[dir] = {g, dir, gamma_t, flags.side[2 * dir], flags.side[2 * dir + 1], u, bxc, byc, o.states, o.eq,
+                o.redo.count, o.redo.faces};
+    }
+    go_pair<F>(grid[0], a[0], grid[1], a[1], dim3(256), stream);
+    go_pair<B>(grid[0], b[0], grid[1], b[1], dim3(256), stream);
   };
   if (order == 5)
-    dir == 0 ? listed(flux_plain_list_kernel_q<T, 5, 0>{}) : listed(flux_plain_list_kernel_q<T, 5, 1>{});
+    launch(reconstruct_list_kernel_q<T, 5>{}, reconstruct_fallback_kernel_q<T, 5>{});
   else
-    dir == 0 ? listed(flux_plain_list_kernel_q<T, 7, 0>{}) : listed(flux_plain_list_kernel_q<T, 7, 1>{});
+    launch(reconstruct_list_kernel_q<T, 7>{}, reconstruct_fallback_kernel_q<T, 7>{});
+}
+
+template <class T>
+void launch_flux(const GridD& g, int order, int hll_only, const Flags4& flags, double gamma, const FaceOut<T>* face,
+                 int first, int count, hipStream_t stream, dim3 b) {
+  const bool mp = order != 1 && order != 2;
+  auto launch = [&](auto q) {
+    using F = decltype(q);
+    dim3 grid[2]{dim3(0, 0), dim3(0, 0)};
+    typename F::Args a[2];
+    for (int k = 0; k < 2; ++k) {
+      const int dir = k < count ? first + k : first;
+      const FaceOut<T>& o = face[k < count ? k : 0];
+      a[k] = {g, dir, periodic_of(flags, dir), T(gamma), o.states, o.flux, o.rate};
+      if (k < count)
+        grid[k] = blocks2d(g.nx + 1, g.ny + 1, mp ? dim3(kFluxTiles[dir][0], kFluxTiles[dir][1]) : b);
+    }
+    go_pair<F>(grid[0], a[0], grid[1], a[1], mp ? dim3(256) : b, stream);
+  };
+  switch (order) {
+    case 1: hll_only ? launch(flux_kernel_q<T, 1, true>{}) : launch(flux_kernel_q<T, 1, false>{}); break;
+    case 2: hll_only ? launch(flux_kernel_q<T, 2, true>{}) : launch(flux_kernel_q<T, 2, false>{}); break;
+    case 5: hll_only ? launch(flux_kernel_q<T, 5, true>{}) : launch(flux_kernel_q<T, 5, false>{}); break;
+    default: hll_only ? launch(flux_kernel_q<T, 7, true>{}) : launch(flux_kernel_q<T, 7, false>{}); break;
+  }
+}
+
+template <class T>
+void launch_flux_learned(const GridD& g, int order, const Flags4& flags, double gamma, const FaceOut<T>* face,
+                         const uint8_t* cell_flags, hipStream_t stream, int list_blocks) {
+  if (order != 5 && order != 7) throw std::invalid_argument("flux launch: the learned form runs MP5/MP7");
+  auto launch = [&](auto q) {
+    using F = decltype(q);
+    dim3 grid[2];
+    typename F::Args a[2];
+    for (int dir = 0; dir < 2; ++dir) {
+      const FaceOut<T>& o = face[dir];
+      const dim3 l = recon_faces(g, dir);
+      const std::size_t most = (static_cast<std::size_t>(l.x) * l.y + kFluxListBlock - 1) / kFluxListBlock;
+      grid[dir] = dim3(static_cast<unsigned>(std::min(static_cast<std::size_t>(list_blocks) * 256 / kFluxListBlock, most)));
+      a[dir] = {g, dir, periodic_of(flags, dir), T(gamma), o.states, o.flux, o.rate, cell_flags, o.list.count,
+                o.list.faces};
+    }
+    go_pair<F>(grid[0], a[0], grid[1], a[1], dim3(kFluxListBlock), stream);
+  };
+  if (order == 5)
+    launch(flux_plain_list_kernel_q<T, 5>{});
+  else
+    launch(flux_plain_list_kernel_q<T, 7>{});
 }
 
 void launch_cfl_reduce(const GridD& g, const double* rate_x, const double* rate_y, unsigned long long* max_rate,
@@ -2350,11 +2232,10 @@ hipError_t upload_quad_rows(const QuadRows& rows) {
 
 // FP64 and FP32 forms of the face-level launchers.
 #define QMHD_INSTANTIATE(T)                                                                                        \
-  template void launch_reconstruct<T>(const GridD&, int, int, double, const Flags4&, const StateView&,            \
-                                      const double*, const double*, const IfaceView<T>&, int*, unsigned long long*, \
-                                      unsigned long long*, hipStream_t);                                          \
-  template void launch_flux<T>(const GridD&, int, int, int, const Flags4&, double, const IfaceView<T>&,            \
-                               const FluxView<T>&, double*, hipStream_t, dim3);                                   \
+  template void launch_reconstruct<T>(const GridD&, int, double, const Flags4&, const StateView&, const double*,     \
+                                      const double*, const FaceOut<T>*, int, int, hipStream_t);                     \
+  template void launch_flux<T>(const GridD&, int, int, const Flags4&, double, const FaceOut<T>*, int, int,          \
+                               hipStream_t, dim3);                                                                 \
   template void launch_cell_emf<T>(const GridD&, int, const Flags4&, double, const StateView&, const double*,     \
                                    const double*, double*, hipStream_t, const uint8_t*, int);                     \
   template void launch_corner<T>(const GridD&, int, const Flags4&, const FluxView<T>&, const FluxView<T>&,        \
@@ -2363,14 +2244,11 @@ hipError_t upload_quad_rows(const QuadRows& rows) {
                                  const StateView&, const FluxView<T>&, const FluxView<T>&, const double*,         \
                                  const StateOut&, hipStream_t, dim3);
 #define QMHD_INSTANTIATE_LEARNED(T)                                                                                \
-  template void launch_flux_learned<T>(const GridD&, int, int, const Flags4&, double, const IfaceView<T>&,         \
-                                       const FluxView<T>&, double*, const uint8_t*, const unsigned long long*,      \
-                                       const unsigned long long*, hipStream_t, int);                               \
-  template void launch_reconstruct_learned<T>(const GridD&, int, int, double, const Flags4&, const StateView&,     \
-                                              const double*, const double*, const uint8_t*, const IfaceView<T>&,  \
-                                              int*, unsigned long long*, unsigned long long*, unsigned long long*, \
-                                              unsigned long long*, unsigned long long*, const FluxView<T>&,       \
-                                              double*, hipStream_t, int, int);
+  template void launch_flux_learned<T>(const GridD&, int, const Flags4&, double, const FaceOut<T>*,                \
+                                       const uint8_t*, hipStream_t, int);                                         \
+  template void launch_reconstruct_learned<T>(const GridD&, int, double, const Flags4&, const StateView&,           \
+                                              const double*, const double*, const uint8_t*, const FaceOut<T>*,     \
+                                              unsigned long long*, hipStream_t, int, const int*);
 QMHD_INSTANTIATE_LEARNED(double)
 QMHD_INSTANTIATE_LEARNED(float)
 #undef QMHD_INSTANTIATE_LEARNED

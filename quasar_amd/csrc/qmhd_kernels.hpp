@@ -45,7 +45,8 @@ struct StepStatus {
   unsigned long long max_rate;       // CFL additive rate (max)
   double dt;                         // device-side dt of the auto-dt loop
   double time;                       // accumulated simulated time
-  double pad[5];
+  unsigned long long lists[4];       // faces listed for the general path (x, y), and again (x, y); see FaceOut
+  double pad[1];
 };
 
 struct IcSpecD {
@@ -74,34 +75,48 @@ void launch_collocate(const GridD& g, int axis, int co, const double* face, doub
 // The face-level launchers are instantiated for T = double (the FP64 form)
 // and T = float (the FP32 form: interface states, fluxes and their arithmetic
 // in FP32; state, collocation, cell/corner E_z, rates and the update in FP64).
+// A counted face list; the count is zero before the launch that fills it.
+struct FaceList {
+  unsigned long long* count;
+  unsigned long long* faces;
+};
+// One face direction's planes: interface states, L == R flags, fluxes and rates
+// (null: no signal speeds wanted), the faces left to the general path and, in
+// the learned form, the listed faces left to it.
 template <class T>
-void launch_reconstruct(const GridD& g, int dir, int order, double gamma, const Flags4& flags, const StateView& u,
-                        const double* bxc, const double* byc, const IfaceView<T>& out, int* eq,
-                        unsigned long long* fb_count, unsigned long long* fb_list, hipStream_t stream);
-// Learned form (orders 5 and 7): cheap faces where the indicator left both
-// cells unflagged, the plain path over the list of the others; adds the
-// listed count to *plain_total when given.
-// Learned form: the flux of the faces on the plain reconstruction's list (the
-// cheap reconstruction stores every other face's flux and rate itself).
+struct FaceOut {
+  IfaceView<T> states;
+  int* eq;
+  FluxView<T> flux;
+  double* rate;
+  FaceList list, redo;
+};
+// Both directions (first 0, count 2) or one (count 1) in one launch each of the
+// faces and of the fallback.
 template <class T>
-void launch_flux_learned(const GridD& g, int dir, int order, const Flags4& flags, double gamma,
-                         const IfaceView<T>& in, const FluxView<T>& flux, double* rate, const uint8_t* cell_flags,
-                         const unsigned long long* fb_count, const unsigned long long* fb_list, hipStream_t stream,
-                         int list_blocks);
+void launch_reconstruct(const GridD& g, int order, double gamma, const Flags4& flags, const StateView& u,
+                        const double* bxc, const double* byc, const FaceOut<T>* out, int first, int count,
+                        hipStream_t stream);
+// Zeroes `n` counters (at most 64).
+void launch_counter_reset(unsigned long long* counters, int n, hipStream_t stream);
+// Learned form (orders 5 and 7), both directions: cheap faces where the
+// indicator left both cells unflagged, the plain path over the lists of the
+// others; adds the listed counts to *plain_total when given.  The flux launch
+// takes the listed faces (the cheap reconstruction stores every other face's
+// flux and rate itself).
 template <class T>
-void launch_reconstruct_learned(const GridD& g, int dir, int order, double gamma, const Flags4& flags,
-                                const StateView& u, const double* bxc, const double* byc, const uint8_t* cell_flags,
-                                const IfaceView<T>& out, int* eq, unsigned long long* fb_count,
-                                unsigned long long* fb_list, unsigned long long* fb2_count,
-                                unsigned long long* fb2_list, unsigned long long* plain_total,
-                                const FluxView<T>& flux, double* rate, hipStream_t stream, int list_blocks = 1024,
-                                int cheap_tile = 0);
-// `rate` may be null (no signal speeds wanted); `block` shapes the orders
-// without transverse quadrature (MP5/MP7 take their LDS tile).
+void launch_flux_learned(const GridD& g, int order, const Flags4& flags, double gamma, const FaceOut<T>* face,
+                         const uint8_t* cell_flags, hipStream_t stream, int list_blocks);
 template <class T>
-void launch_flux(const GridD& g, int dir, int order, int hll_only, const Flags4& flags, double gamma,
-                 const IfaceView<T>& in, const FluxView<T>& flux, double* rate, hipStream_t stream,
-                 dim3 block = dim3(64, 4));
+void launch_reconstruct_learned(const GridD& g, int order, double gamma, const Flags4& flags, const StateView& u,
+                                const double* bxc, const double* byc, const uint8_t* cell_flags,
+                                const FaceOut<T>* out, unsigned long long* plain_total, hipStream_t stream,
+                                int list_blocks, const int* cheap_tile);
+// `block` shapes the orders without transverse quadrature (MP5/MP7 take their
+// LDS tile).
+template <class T>
+void launch_flux(const GridD& g, int order, int hll_only, const Flags4& flags, double gamma, const FaceOut<T>* face,
+                 int first, int count, hipStream_t stream, dim3 block = dim3(64, 4));
 void launch_cfl_reduce(const GridD& g, const double* rate_x, const double* rate_y, unsigned long long* max_rate,
                        hipStream_t stream);
 // MP5/MP7 cell E_z: `tile` selects the LDS tile, 0: 16x16, 1: 32x8, 2: 8x32

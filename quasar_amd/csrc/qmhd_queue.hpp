@@ -61,9 +61,10 @@ __device__ __forceinline__ Blk Blk::xcd_tiled() {
   return Blk{t % gx, t / gx, gx, gy};
 }
 
-// Run r owns the queue's tiles [first, next run's first); its own grid is gx x gy.
+// Run r owns the queue's tiles [first, next run's first); its own grid is gx x
+// gy.  xcd: a Pair's half takes its tiles in the XCD-aware order.
 struct QueueRun {
-  unsigned first, gx, gy, pad;
+  unsigned first, gx, gy, xcd;
 };
 
 // Arguments as a tile function receives them from an argument record.  A
@@ -112,10 +113,62 @@ struct QueueTile {
   Blk blk;
 };
 __device__ __forceinline__ QueueTile queue_tile(const QueueRun* __restrict__ runs, int nruns) {
-  const int r = queue_run_of(runs, nruns, blockIdx.x);
+  // The last run whose first tile is not past this one, 64 runs per read (the
+  // binary search is five reads one after another for 24 runs, 4 us in front of
+  // every launch; a block of less than a wave keeps it).
+  int r = -1;
+  if (blockDim.x * blockDim.y < 64) {
+    r = queue_run_of(runs, nruns, blockIdx.x);
+  } else {
+    for (int base = 0; base < nruns; base += 64) {
+      const int k = base + static_cast<int>(__lane_id());
+      r += __popcll(__ballot(k < nruns && runs[k < nruns ? k : 0].first <= blockIdx.x));
+    }
+  }
+  r = __builtin_amdgcn_readfirstlane(r);
   const QueueRun run = runs[r];
   const unsigned local = blockIdx.x - run.first;
   return QueueTile{r, Blk{local % run.gx, local / run.gx, run.gx, run.gy}};
+}
+
+// Two launches of one kernel taken as one: the records and tile ranges of both
+// (r[1].first is the first tile of the second), passed by value.  A kernel that
+// can run so takes a Pair behind its queue arguments and is launched with null
+// ones.  Small grids spend most of a step on launches that fill a fraction of
+// the device; a pair costs one of them, and its halves run side by side: 64^2
+// FP64, x and y faces, reconstruction 9.6 + 9.6 -> 9.4 us, flux 14 + 14 -> 14,
+// fallback 2.9 + 2.9 -> 4.1; learned rotor 768^2 lists 16.6 + 16.6 -> 22.6, their
+// fluxes 17.6 + 14.2 -> 21.4; large grids within 2 %.
+template <class A>
+struct Pair {
+  A a[2];
+  QueueRun r[2];
+};
+template <class A>
+struct TileOf {
+  const A& args;
+  Blk blk;
+};
+// Records are read through the constant address space: scalar loads, and no
+// private copy of the by-value ones.
+template <class A>
+__device__ __forceinline__ const A* constant_space(const A* p) {
+  return (const A*)(const __attribute__((address_space(4))) A*)(__UINTPTR_TYPE__)p;
+}
+template <class A>
+__device__ __forceinline__ TileOf<A> tile_of(const A* __restrict__ args, const QueueRun* __restrict__ runs, int nruns) {
+  if (runs) {
+    const QueueTile t = queue_tile(runs, nruns);
+    return TileOf<A>{*constant_space(args + t.run), t.blk};
+  }
+  // The Pair follows two pointers and an int in the kernel's arguments.
+  static_assert(alignof(Pair<A>) == 8, "the pair's offset in the kernel arguments");
+  const Pair<A>* own = constant_space(
+      (const Pair<A>*)((__UINTPTR_TYPE__)__builtin_amdgcn_kernarg_segment_ptr() + 24));
+  const int second = blockIdx.x >= own->r[1].first ? 1 : 0;
+  const QueueRun run = own->r[second];
+  const unsigned b = blockIdx.x - run.first, t = run.xcd ? xcd_tile(b, run.gx * run.gy) : b;
+  return TileOf<A>{own->a[second], Blk{t % run.gx, t / run.gx, run.gx, run.gy}};
 }
 
 // QueueTiles<Q>::kernel: the kernel <name>_queue, which includes the step
@@ -124,6 +177,11 @@ __device__ __forceinline__ QueueTile queue_tile(const QueueRun* __restrict__ run
 // one tile per workgroup.
 template <class Q>
 struct QueueTiles;
+// Whether that kernel takes a Pair.
+template <class Q>
+struct Paired {
+  static constexpr bool value = false;
+};
 
 // Persistent form: `cap` workgroups, each taking tiles blockIdx.x,
 // blockIdx.x + gridDim.x, ...  The loop around the tile function costs
@@ -152,9 +210,13 @@ void queue_launch(const void* dev_args, const QueueRun* dev_runs, int nruns, uns
                   hipStream_t stream) {
   if (total == 0) return;
   const auto* args = static_cast<const typename Q::Args*>(dev_args);
-  if (cap == 0 || cap >= total)
-    hipLaunchKernelGGL(QueueTiles<Q>::kernel, dim3(total), block, 0, stream, args, dev_runs, nruns);
-  else
+  if (cap == 0 || cap >= total) {
+    if constexpr (Paired<Q>::value)
+      hipLaunchKernelGGL(QueueTiles<Q>::kernel, dim3(total), block, 0, stream, args, dev_runs, nruns,
+                         Pair<typename Q::Args>{});
+    else
+      hipLaunchKernelGGL(QueueTiles<Q>::kernel, dim3(total), block, 0, stream, args, dev_runs, nruns);
+  } else
     hipLaunchKernelGGL((queue_kernel<Q>), dim3(cap), block, 0, stream, args, dev_runs, nruns, total);
 }
 
@@ -165,11 +227,12 @@ struct Recorder {
     dim3 grid, block;
     std::vector<unsigned char> args;
     QueueLaunch launch;
+    bool joins;  // runs beside the entry before it, in one launch
   };
   std::vector<Entry> entries;
 
   template <class Q>
-  void add(dim3 grid, dim3 block, const typename Q::Args& a) {
+  void add(dim3 grid, dim3 block, const typename Q::Args& a, bool joins = false) {
     Entry e;
     e.tag = Q::tag();
     e.grid = grid;
@@ -177,11 +240,31 @@ struct Recorder {
     e.args.resize(sizeof a);
     std::memcpy(e.args.data(), &a, sizeof a);
     e.launch = &queue_launch<Q>;
+    e.joins = joins;
     entries.push_back(std::move(e));
   }
 };
 
 inline thread_local Recorder* g_recorder = nullptr;
+
+// One launch over the tiles of both grids (the second may be empty).  Q's tiles
+// go out in the XCD-aware order when neighbours share cells; a face list, whose
+// first tiles hold all its work, in the hardware's, which deals them over the
+// XCDs (in the other order the 1024-block launches of the learned rotor 768^2
+// had their faces on one XCD: 59 against 21 us).
+template <class Q>
+void go_pair(dim3 grid0, const typename Q::Args& a0, dim3 grid1, const typename Q::Args& a1, dim3 block,
+             hipStream_t stream) {
+  if (g_recorder) {
+    g_recorder->add<Q>(grid0, block, a0);
+    g_recorder->add<Q>(grid1, block, a1, true);
+    return;
+  }
+  const unsigned n0 = grid0.x * grid0.y, n1 = grid1.x * grid1.y;
+  hipLaunchKernelGGL(QueueTiles<Q>::kernel, dim3(n0 + n1), block, 0, stream, nullptr, nullptr, 0,
+                     Pair<typename Q::Args>{{a0, a1},
+                                            {{0u, grid0.x, grid0.y, Paired<Q>::xcd}, {n0, grid1.x, grid1.y, Paired<Q>::xcd}}});
+}
 
 // Launch of a step kernel through its queue functor.
 template <class Q, class... A>
@@ -189,6 +272,8 @@ void go(dim3 grid, dim3 block, hipStream_t stream, A... a) {
   const typename Q::Args args{a...};
   if (g_recorder)
     g_recorder->add<Q>(grid, block, args);
+  else if constexpr (Paired<Q>::value)
+    go_pair<Q>(grid, args, dim3(0, 0), args, block, stream);
   else
     Q::launch(grid, block, stream, args);
 }

@@ -325,7 +325,8 @@ class Solver {
     QMHD_HIP(hipStreamCreate(&stream_));
     const std::size_t n = storage(g_);
     for (auto& r : reg_) r.allocate(n);
-    for (auto& p : iface_) p = DBuf(n);
+    for (auto& d : iface_)
+      for (auto& p : d) p = DBuf(n);
     for (auto& p : fx_) p = DBuf(n);
     for (auto& p : fy_) p = DBuf(n);
     rate_x_ = DBuf(n);
@@ -334,11 +335,9 @@ class Solver {
     eqy_ = DBuf(n);
     cell_ez_ = DBuf(n);
     ez_ = DBuf(n);
-    fb_list_ = DBuf(n);
-    fb_count_ = DBuf(1);
-    if (learned_) {
-      fb2_list_ = DBuf(n);
-      fb2_count_ = DBuf(1);
+    for (int dir = 0; dir < 2; ++dir) {
+      fb_list_[dir] = DBuf(n);
+      if (learned_) fb2_list_[dir] = DBuf(n);
     }
     if (learned_) {
       mlp_params_ = DBuf((mlp::kParams + 1) / 2);
@@ -463,14 +462,6 @@ class Solver {
   void issue_faces(int slot, int order, bool want_rates) {
     const int hll = order <= 1 ? 1 : 0;
     Register& r = reg_[slot];
-    double* ip[16];
-    for (int c = 0; c < 16; ++c) ip[c] = iface_[c].p;
-    double* fxp[8];
-    double* fyp[8];
-    for (int c = 0; c < 8; ++c) {
-      fxp[c] = fx_[c].p;
-      fyp[c] = fy_[c].p;
-    }
     if (learned_ && order == order_) {
       if (!indicator_set_)
         throw std::invalid_argument("MhdSolver2D: indicator 'mlp' needs its network (set_indicator) before stepping");
@@ -485,48 +476,44 @@ class Solver {
       faces_issued_ += static_cast<long long>(g_.nx + 1) * (g_.ny + 2 * g_.ng) +
                        static_cast<long long>(g_.nx + 2 * g_.ng) * (g_.ny + 1);
     }
-    // Only the live state's face rates are reduced to a timestep.
-    double* rx = want_rates ? rate_x_.p : nullptr;
-    double* ry = want_rates ? rate_y_.p : nullptr;
     if (fp32_)
-      issue_faces_as<float>(r, order, hll, ip, fxp, fyp, rx, ry);
+      issue_faces_as<float>(r, order, hll, want_rates);
     else
-      issue_faces_as<double>(r, order, hll, ip, fxp, fyp, rx, ry);
+      issue_faces_as<double>(r, order, hll, want_rates);
   }
 
+  // Reconstruction and fluxes of both directions, each in one launch (the
+  // lists' counters were zeroed by the register's prep launch).
   template <class T>
-  void issue_reconstruct(Register& r, int dir, int order, double* const* ip, int* eq, double* const* fp,
-                         double* rate) {
-    if (learned_ && order == order_)
-      launch_reconstruct_learned<T>(g_, dir, order, gamma_, field_, r.view(), r.bxc.p, r.byc.p, flags(),
-                                    iface_as<T>(ip), eq, fb_count(), fb_list(), fb2_count(), fb2_list(), plain_total(),
-                                    flux_as<T>(fp), rate, stream_, tuning_.list_blocks,
-                                    dir == 0 ? tuning_.cheap_tile : tuning_.cheap_tile_y);
-    else
-      launch_reconstruct<T>(g_, dir, order, gamma_, field_, r.view(), r.bxc.p, r.byc.p, iface_as<T>(ip), eq,
-                            fb_count(), fb_list(), stream_);
-  }
-
-  template <class T>
-  void issue_faces_as(Register& r, int order, int hll, double* const* ip, double* const* fxp, double* const* fyp,
-                      double* rx, double* ry) {
-    const uint8_t* cf = learned_ && order == order_ ? flags() : nullptr;
-    clock_.timed(QMHD_KERNEL_RECONSTRUCT, stream_,
-                 [&] { issue_reconstruct<T>(r, 0, order, ip, reinterpret_cast<int*>(eqx_.p), fxp, rx); });
-    auto flux = [&](int dir, double* const* fp, double* rate) {
-      clock_.timed(QMHD_KERNEL_FLUX, stream_, [&] {
-        if (cf)
-          launch_flux_learned<T>(g_, dir, order, field_, gamma_, iface_as<T>(ip), flux_as<T>(fp), rate, cf,
-                                 fb_count(), fb_list(), stream_, tuning_.list_blocks);
-        else
-          launch_flux<T>(g_, dir, order, hll, field_, gamma_, iface_as<T>(ip), flux_as<T>(fp), rate, stream_,
-                         tuning_.flux);
-      });
-    };
-    flux(0, fxp, rx);
-    clock_.timed(QMHD_KERNEL_RECONSTRUCT, stream_,
-                 [&] { issue_reconstruct<T>(r, 1, order, ip, reinterpret_cast<int*>(eqy_.p), fyp, ry); });
-    flux(1, fyp, ry);
+  void issue_faces_as(Register& r, int order, int hll, bool want_rates) {
+    const bool learned = learned_ && order == order_;
+    FaceOut<T> out[2];
+    for (int dir = 0; dir < 2; ++dir) {
+      double* ip[16];
+      double* fp[8];
+      for (int c = 0; c < 16; ++c) ip[c] = iface_[dir][c].p;
+      for (int c = 0; c < 8; ++c) fp[c] = (dir == 0 ? fx_ : fy_)[c].p;
+      unsigned long long* lists = status_->lists;
+      out[dir] = FaceOut<T>{iface_as<T>(ip), reinterpret_cast<int*>((dir == 0 ? eqx_ : eqy_).p), flux_as<T>(fp),
+                            // Only the live state's face rates are reduced to a timestep.
+                            want_rates ? (dir == 0 ? rate_x_ : rate_y_).p : nullptr,
+                            FaceList{lists + dir, reinterpret_cast<unsigned long long*>(fb_list_[dir].p)},
+                            FaceList{lists + 2 + dir, reinterpret_cast<unsigned long long*>(fb2_list_[dir].p)}};
+    }
+    const int cheap[2] = {tuning_.cheap_tile, tuning_.cheap_tile_y};
+    clock_.timed(QMHD_KERNEL_RECONSTRUCT, stream_, [&] {
+      if (learned)
+        launch_reconstruct_learned<T>(g_, order, gamma_, field_, r.view(), r.bxc.p, r.byc.p, flags(), out, plain_total(),
+                                      stream_, tuning_.list_blocks, cheap);
+      else
+        launch_reconstruct<T>(g_, order, gamma_, field_, r.view(), r.bxc.p, r.byc.p, out, 0, 2, stream_);
+    });
+    clock_.timed(QMHD_KERNEL_FLUX, stream_, [&] {
+      if (learned)
+        launch_flux_learned<T>(g_, order, field_, gamma_, out, flags(), stream_, tuning_.list_blocks);
+      else
+        launch_flux<T>(g_, order, hll, field_, gamma_, out, 0, 2, stream_, tuning_.flux);
+    });
   }
 
   // Cell E_z, corner E_z and the fused update of one stage.
@@ -1054,14 +1041,10 @@ class Solver {
   std::unique_ptr<Register> snap_;  // batch autotuning snapshot
   double snap_acc_[8]{};
   int snap_live_{0};
-  DBuf iface_[16], fx_[8], fy_[8];
+  DBuf iface_[2][16], fx_[8], fy_[8];
   DBuf rate_x_, rate_y_, eqx_, eqy_, cell_ez_, ez_;
   // Faces whose MP states need the fallback chain (list + count).
-  DBuf fb_list_, fb_count_, fb2_list_, fb2_count_;
-  unsigned long long* fb_list() { return reinterpret_cast<unsigned long long*>(fb_list_.p); }
-  unsigned long long* fb2_list() { return reinterpret_cast<unsigned long long*>(fb2_list_.p); }
-  unsigned long long* fb2_count() { return reinterpret_cast<unsigned long long*>(fb2_count_.p); }
-  unsigned long long* fb_count() { return reinterpret_cast<unsigned long long*>(fb_count_.p); }
+  DBuf fb_list_[2], fb2_list_[2];
   StepStatus* status_{nullptr};
   StepStatus* host_status_{nullptr};
   int cache_order_{-1};
@@ -1232,6 +1215,13 @@ void set_bits(unsigned long long* dev, double v, hipStream_t stream) {
   qmhd::hip_check(hipMemcpyAsync(dev, &b, sizeof b, hipMemcpyHostToDevice, stream), "hipMemcpyAsync");
 }
 
+// One direction's face fluxes (and rates, when given) from its interface states.
+void face_flux(const qmhd::GridD& d, int dir, int order, int hll_only, const qmhd::Flags4& f, double gamma,
+               const double* const* if16, double* const* flux8, double* rate, hipStream_t stream) {
+  const qmhd::FaceOut<double> o{qmhd::iface(const_cast<double* const*>(if16)), nullptr, qmhd::fluxv(flux8), rate, {}, {}};
+  qmhd::launch_flux<double>(d, order, hll_only, f, gamma, &o, dir, 1, stream);
+}
+
 // The EMF tables of the CT corner (cell E_z, face fluxes, no-jump flags)
 // from u and both directions' interface states.  Work planes: scratch 0..7.
 void prepare_emf_tables(const qmhd::GridD& d, int order, bool hll_only, const qmhd::Flags4& f, double gamma,
@@ -1246,11 +1236,9 @@ void prepare_emf_tables(const qmhd::GridD& d, int order, bool hll_only, const qm
   // By (x faces) and Bx (y faces) components go to the tables, the rest to
   // work planes (two components share a plane; only the table is read).
   double* fx[8] = {s.plane(0), s.plane(1), s.plane(2), s.plane(3), s.plane(4), s.plane(5), t.xface_flux_by, s.plane(6)};
-  qmhd::launch_flux(d, 0, order, hll_only ? 1 : 0, f, gamma, qmhd::iface(const_cast<double* const*>(ifx16)),
-                    qmhd::fluxv(fx), nullptr, stream);
+  face_flux(d, 0, order, hll_only ? 1 : 0, f, gamma, ifx16, fx, nullptr, stream);
   double* fy[8] = {s.plane(0), s.plane(1), s.plane(2), s.plane(3), s.plane(4), t.yface_flux_bx, s.plane(5), s.plane(6)};
-  qmhd::launch_flux(d, 1, order, hll_only ? 1 : 0, f, gamma, qmhd::iface(const_cast<double* const*>(ify16)),
-                    qmhd::fluxv(fy), nullptr, stream);
+  face_flux(d, 1, order, hll_only ? 1 : 0, f, gamma, ify16, fy, nullptr, stream);
 }
 
 // Corner E_z from prepared tables: the corner reads only the By flux of the
@@ -1296,10 +1284,12 @@ int qmhd_reconstruct(const qmhd_grid* g, int dir, int order, const int32_t* flag
     const qmhd::StateView u = qmhd::view(u8);
     qmhd::launch_collocate(d, 0, 0, u8[5], s.plane(0), st(stream));
     qmhd::launch_collocate(d, 1, 0, u8[6], s.plane(1), st(stream));
-    qmhd::launch_reconstruct(d, dir, order, gamma, qmhd::flags_of(flags4), u, s.plane(0), s.plane(1),
-                             qmhd::iface(out16), reinterpret_cast<int*>(s.plane(2)),
-                             reinterpret_cast<unsigned long long*>(s.tail()),
-                             reinterpret_cast<unsigned long long*>(s.plane(3)), st(stream));
+    const qmhd::FaceList list{reinterpret_cast<unsigned long long*>(s.tail()),
+                              reinterpret_cast<unsigned long long*>(s.plane(3))};
+    const qmhd::FaceOut<double> o{qmhd::iface(out16), reinterpret_cast<int*>(s.plane(2)), {}, nullptr, list, {}};
+    if (order >= 5) qmhd::launch_counter_reset(list.count, 1, st(stream));
+    qmhd::launch_reconstruct<double>(d, order, gamma, qmhd::flags_of(flags4), u, s.plane(0), s.plane(1), &o,
+                                     dir == 0 ? 0 : 1, 1, st(stream));
     qmhd::hip_check(hipGetLastError(), "reconstruct");
   });
 }
@@ -1310,8 +1300,7 @@ int qmhd_hlld_flux(const qmhd_grid* g, int dir, int order, int hll_only, const i
     const qmhd::GridD d = qmhd::to_grid(*g);
     qmhd::ensure_quad_rows();
     (void)scratch_of(g, scratch);  // a missing workspace stays refused
-    qmhd::launch_flux(d, dir, order, hll_only, qmhd::flags_of(flags4), gamma,
-                      qmhd::iface(const_cast<double* const*>(in16)), qmhd::fluxv(flux8), nullptr, st(stream));
+    face_flux(d, dir == 0 ? 0 : 1, order, hll_only, qmhd::flags_of(flags4), gamma, in16, flux8, nullptr, st(stream));
     qmhd::hip_check(hipGetLastError(), "hlld_flux");
   });
 }
@@ -1426,10 +1415,8 @@ int qmhd_cfl_max_rate(const qmhd_grid* g, int order, const int32_t* flags4, doub
     // The face kernels write fluxes too; route them to scratch planes 2..7 and
     // the two rate planes to 0..1 (flux planes 6,7 share scratch tail-free).
     double* fl[8] = {s.plane(2), s.plane(3), s.plane(4), s.plane(5), s.plane(6), s.plane(7), s.plane(6), s.plane(7)};
-    qmhd::launch_flux(d, 0, order, order <= 1, f, gamma, qmhd::iface(const_cast<double* const*>(ifx16)),
-                      qmhd::fluxv(fl), s.plane(0), st(stream));
-    qmhd::launch_flux(d, 1, order, order <= 1, f, gamma, qmhd::iface(const_cast<double* const*>(ify16)),
-                      qmhd::fluxv(fl), s.plane(1), st(stream));
+    face_flux(d, 0, order, order <= 1, f, gamma, ifx16, fl, s.plane(0), st(stream));
+    face_flux(d, 1, order, order <= 1, f, gamma, ify16, fl, s.plane(1), st(stream));
     auto* slot = reinterpret_cast<unsigned long long*>(s.tail());
     set_bits(slot, 0.0, st(stream));
     qmhd::launch_cfl_reduce(d, s.plane(0), s.plane(1), slot, st(stream));
@@ -1764,6 +1751,7 @@ struct qmhd_batch {
     qmhd::QueueLaunch launch;
     dim3 block;
     std::size_t args_off, runs_off;
+    int nruns;
     unsigned total;
   };
   std::vector<Slot> slots[2];
@@ -1861,8 +1849,8 @@ struct qmhd_batch {
         const qmhd::Recorder::Entry& e0 = rec[0][i];
         for (std::size_t k = 1; k < runs.size(); ++k) {
           const qmhd::Recorder::Entry& e = rec[k][i];
-          if (e.tag != e0.tag || e.block.x != e0.block.x || e.block.y != e0.block.y || e.block.z != e0.block.z ||
-              e.args.size() != e0.args.size())
+          if (e.tag != e0.tag || e.joins != e0.joins || e.block.x != e0.block.x || e.block.y != e0.block.y ||
+              e.block.z != e0.block.z || e.args.size() != e0.args.size())
             throw std::invalid_argument(
                 "qmhd_batch: queue mode needs runs with the same scheme, form and launch shapes");
         }
@@ -1871,22 +1859,29 @@ struct qmhd_batch {
         s.block = e0.block;
         align(256);
         s.args_off = blob.size();
-        for (std::size_t k = 0; k < runs.size(); ++k)
-          blob.insert(blob.end(), rec[k][i].args.begin(), rec[k][i].args.end());
+        // A joining entry's tiles follow its predecessor's in one launch.
+        const std::size_t last = i + 1 < n && rec[0][i + 1].joins ? i + 1 : i;
+        for (std::size_t q = i; q <= last; ++q)
+          for (std::size_t k = 0; k < runs.size(); ++k)
+            blob.insert(blob.end(), rec[k][q].args.begin(), rec[k][q].args.end());
         align(16);
         s.runs_off = blob.size();
+        s.nruns = static_cast<int>((last - i + 1) * runs.size());
         unsigned long long total = 0;
-        for (std::size_t k = 0; k < runs.size(); ++k) {
-          const dim3 gr = rec[k][i].grid;
-          if (gr.z != 1 || gr.x == 0 || gr.y == 0) throw std::logic_error("qmhd_batch: queue slot with an empty or 3-D grid");
-          const qmhd::QueueRun qr{static_cast<unsigned>(total), gr.x, gr.y, 0u};
-          const unsigned char* b = reinterpret_cast<const unsigned char*>(&qr);
-          blob.insert(blob.end(), b, b + sizeof qr);
-          total += static_cast<unsigned long long>(gr.x) * gr.y;
-        }
+        for (std::size_t q = i; q <= last; ++q)
+          for (std::size_t k = 0; k < runs.size(); ++k) {
+            const dim3 gr = rec[k][q].grid;
+            if (gr.z != 1 || gr.x == 0 || gr.y == 0)
+              throw std::logic_error("qmhd_batch: queue slot with an empty or 3-D grid");
+            const qmhd::QueueRun qr{static_cast<unsigned>(total), gr.x, gr.y, 0u};
+            const unsigned char* b = reinterpret_cast<const unsigned char*>(&qr);
+            blob.insert(blob.end(), b, b + sizeof qr);
+            total += static_cast<unsigned long long>(gr.x) * gr.y;
+          }
         if (total > 0xFFFFFFFFull) throw std::invalid_argument("qmhd_batch: too many tiles in one queue launch");
         s.total = static_cast<unsigned>(total);
         slots[p].push_back(s);
+        i = last;
       }
       (void)nruns;
     }
@@ -1906,7 +1901,7 @@ struct qmhd_batch {
       qmhd::hip_check(hipStreamBeginCapture(master, hipStreamCaptureModeRelaxed), "hipStreamBeginCapture");
       for (const Slot& s : slots[p]) {
         s.launch(queue_mem + s.args_off, reinterpret_cast<const qmhd::QueueRun*>(queue_mem + s.runs_off),
-                 static_cast<int>(runs.size()), s.total, queue_blocks, s.block, master);
+                 s.nruns, s.total, queue_blocks, s.block, master);
       }
       hipGraph_t g = nullptr;
       const hipError_t e = hipStreamEndCapture(master, &g);
