@@ -148,6 +148,17 @@ __device__ __forceinline__ double ok_or_zero(double v) { return fin(v) ? v : 0.0
 // reading the candidate and its base (16 planes) and bisecting with divisions
 // in every cell, took 262 us; now 106 us.  A division-free sign test decides
 // all but the cells at the edge of the admissible set; those read the base.
+// The one-sided closures of the outer ghost cells, a serial chain of some 600
+// instructions each, have blocks of their own, a thread per closure: taken by
+// the wave that holds the cell, nearly every wave of a small grid ran one per
+// axis behind its centred sums (64^2 FP64 16 -> 6.3 us per launch, learned rotor
+// 768^2 21 -> 17, a queue of 24 runs 24 -> 18).
+// Blocks of the closures' part of a prep launch.
+template <int W>
+__host__ __device__ __forceinline__ int prep_strip_blocks(const GridD& g) {
+  return ((W - 1) * (g.nx + g.ny + 4 * g.ng) + 255) / 256;
+}
+
 template <bool EXACT, int W>
 __device__ __forceinline__ void prep_kernel_tile(
     const Blk& qb, const GridD& g, const StateView& u, double* __restrict__ bxc, double* __restrict__ byc,
@@ -170,6 +181,7 @@ __global__ __launch_bounds__(256) void prep_kernel(GridD g, StateView u, double*
 // Queue form of prep_kernel (one launch over the tiles of many runs).
 template <bool EXACT, int W>
 struct prep_kernel_q {
+  static constexpr int kWindow = W;
   struct Args {
     GridD g;
     StateView u;
@@ -1934,9 +1946,10 @@ void launch_prep(const GridD& g, const StateView& u, double* bxc, double* byc, c
                  const double* base_bxc, const double* base_byc, int theta_slot, int theta_co, int theta_both,
                  int live_checks, int solver_owned, StepStatus* status, hipStream_t stream, bool exact) {
   const dim3 b(64, 4);
-  const dim3 grid = blocks2d(g.nx + 2 * g.ng, g.ny + 2 * g.ng, b);
+  const dim3 cells = blocks2d(g.nx + 2 * g.ng, g.ny + 2 * g.ng, b);
   auto prep = [&](auto q) {
-    go<decltype(q)>(grid, b, stream, g, u, bxc, byc, base, base_bxc, base_byc, theta_slot, theta_co, theta_both,
+    const int strips = prep_strip_blocks<decltype(q)::kWindow>(g);
+    go<decltype(q)>(dim3(strips + cells.x * cells.y), b, stream, g, u, bxc, byc, base, base_bxc, base_byc, theta_slot, theta_co, theta_both,
                     live_checks, solver_owned, status);
   };
   // The padded extents hold the halo's full window (2 ng + 1 cells at least).

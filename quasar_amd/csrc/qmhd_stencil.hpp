@@ -328,12 +328,17 @@ __host__ __device__ __forceinline__ int colloc_start(int cell, int lo, int hi) {
   return start + W - 1 > hi ? hi - W + 1 : start;
 }
 
+// The centred rule in the form's arithmetic.
+template <int W, bool EXACT>
+__host__ __device__ __forceinline__ double colloc_centred_as(const double* s) {
+  return EXACT ? colloc_centred<W>(s) : colloc_centred_fma<W>(s);
+}
+
 // Cell average from the window's faces s, the cell `rel` faces after its first
 // face: the centred rule, or the one-sided closure where the window was moved.
 template <int W, bool EXACT>
 __host__ __device__ __forceinline__ double colloc_window(const double* s, int rel) {
-  if (rel == W / 2 - 1) return EXACT ? colloc_centred<W>(s) : colloc_centred_fma<W>(s);
-  return one_sided<W>(s, rel);
+  return rel == W / 2 - 1 ? colloc_centred_as<W, EXACT>(s) : one_sided<W>(s, rel);
 }
 
 // Learned form: a face normal to `dir` (x faces dir 0, y faces dir 1) is
