@@ -153,6 +153,7 @@ __device__ __forceinline__ double ok_or_zero(double v) { return fin(v) ? v : 0.0
 // the wave that holds the cell, nearly every wave of a small grid ran one per
 // axis behind its centred sums (64^2 FP64 16 -> 6.3 us per launch, learned rotor
 // 768^2 21 -> 17, a queue of 24 runs 24 -> 18).
+
 // Blocks of the closures' part of a prep launch.
 template <int W>
 __host__ __device__ __forceinline__ int prep_strip_blocks(const GridD& g) {
