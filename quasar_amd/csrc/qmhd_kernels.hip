@@ -309,7 +309,7 @@ constexpr int kReconWaves = sizeof(T) == 4 ? 4 : 2;
 constexpr int kReconTiles[2][2] = {{64, 4}, {32, 8}};
 template <int ORDER>
 constexpr int recon_tile_cells() {
-  constexpr int more = ORDER == 5 ? 5 : 7;
+  constexpr int more = ORDER == 2 ? 3 : ORDER == 5 ? 5 : 7;
   constexpr int x = (kReconTiles[0][0] + more) * kReconTiles[0][1], y = kReconTiles[1][0] * (kReconTiles[1][1] + more);
   return x > y ? x : y;
 }
@@ -2012,11 +2012,11 @@ void launch_reconstruct(const GridD& g, int order, double gamma, const Flags4& f
       fb_grid[k] = list_blocks_of(g, dir, 64);
     }
     go_pair<F>(grid[0], a[0], grid[1], a[1], dim3(256), stream);
-    if (order >= 5) go_pair<B>(fb_grid[0], b[0], fb_grid[1], b[1], dim3(256), stream);
+    if (order >= 2) go_pair<B>(fb_grid[0], b[0], fb_grid[1], b[1], dim3(256), stream);
   };
   switch (order) {
     case 1: launch(reconstruct_kernel_q<T, 1>{}, reconstruct_fallback_kernel_q<T, 5>{}); break;
-    case 2: launch(reconstruct_kernel_q<T, 2>{}, reconstruct_fallback_kernel_q<T, 5>{}); break;
+    case 2: launch(reconstruct_kernel_q<T, 2>{}, reconstruct_fallback_kernel_q<T, 2>{}); break;
     case 5: launch(reconstruct_kernel_q<T, 5>{}, reconstruct_fallback_kernel_q<T, 5>{}); break;
     default: launch(reconstruct_kernel_q<T, 7>{}, reconstruct_fallback_kernel_q<T, 7>{}); break;
   }

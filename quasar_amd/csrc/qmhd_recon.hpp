@@ -302,6 +302,29 @@ __host__ __device__ __forceinline__ bool settle_state(St<T>& s, T v) {
   return ok;
 }
 
+// set_normal_b to the bit (frame of the normal); false when the state is not
+// certainly admissible after it, or (FP64) the energy's three-term sum takes
+// more than one rounding.
+template <class T>
+__host__ __device__ __forceinline__ bool settle_exact(St<T>& s, T v, T gamma) {
+#pragma clang fp contract(off)
+  bool ok = true;
+  const T add = v * (T(0.5) * v), sub = s.bx * (T(0.5) * s.bx);
+  if constexpr (sizeof(T) == 4) {
+    s.en = (s.en + add) - sub;
+  } else {
+    double t, e1, e2, e, rest;
+    two_sum(s.en, add, t, e1);
+    two_sum(t, -sub, t, e2);
+    two_sum(e1, e2, e, rest);
+    ok = rest == 0.0;
+    s.en = t + e;
+  }
+  s.bx = v;
+  Side<T> o;
+  return ok & side_of(s, gamma, o);
+}
+
 // Interface states of a face in the frame of its normal; cell(c, q) is
 // component c (rho, mn, mt1, mt2, E, bn, bt1, bt2) of cell q of its union
 // stencil, bn its own normal field.  False leaves the face to

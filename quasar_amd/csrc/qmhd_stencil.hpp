@@ -474,17 +474,11 @@ __host__ __device__ __forceinline__ int slope_drop(int c, int n, int lo, int hi)
 
 // Second-order MUSCL-minmod in primitive variables (also the MP fallback),
 // mhd_reconstruct.hip:96-120, 375-414, in the reference's arithmetic.
+// Both states of a face from the primitive cells around it.
 template <class T>
-__host__ __device__ __noinline__ void muscl_face(const GridD& g, int dir, int i, int j, T gamma, int side_lo,
-                                                 int side_hi, const StateView& u, const double* bxc, const double* byc,
-                                                 St<T>& ul, St<T>& ur) {
+__host__ __device__ __forceinline__ void muscl_pair(const Prim<T>* w, int drop_m, int drop_p, T gamma, St<T>& ul,
+                                                    St<T>& ur) {
 #pragma clang fp contract(off)
-  const int di = dir == 0 ? 1 : 0, dj = dir == 0 ? 0 : 1;
-  Prim<T> w[4];
-  for (int s = 0; s < 4; ++s) w[s] = to_prim(load_cell<T>(g, u, bxc, byc, i + (s - 2) * di, j + (s - 2) * dj), gamma);
-  const int n_dir = dir == 0 ? g.nx : g.ny;
-  const int drop_m = slope_drop((dir == 0 ? i : j) - 1, n_dir, side_lo, side_hi);
-  const int drop_p = slope_drop(dir == 0 ? i : j, n_dir, side_lo, side_hi);
   auto face = [&](const Prim<T>& wm, const Prim<T>& wc, const Prim<T>& wp, T sign, int drop) {
     const T h = T(0.5) * sign;
     Prim<T> f;
@@ -502,8 +496,20 @@ __host__ __device__ __noinline__ void muscl_face(const GridD& g, int dir, int i,
   ur = to_cons(face(w[1], w[2], w[3], T(-1), drop_p), gamma);
 }
 
-// `clip_rel` (optional) receives the largest change any of the 14 limiter
-// calls made, relative to the largest component of the reference state.
+template <class T>
+__host__ __device__ __noinline__ void muscl_face(const GridD& g, int dir, int i, int j, T gamma, int side_lo,
+                                                 int side_hi, const StateView& u, const double* bxc, const double* byc,
+                                                 St<T>& ul, St<T>& ur) {
+#pragma clang fp contract(off)
+  const int di = dir == 0 ? 1 : 0, dj = dir == 0 ? 0 : 1;
+  Prim<T> w[4];
+  for (int s = 0; s < 4; ++s) w[s] = to_prim(load_cell<T>(g, u, bxc, byc, i + (s - 2) * di, j + (s - 2) * dj), gamma);
+  const int n_dir = dir == 0 ? g.nx : g.ny;
+  const int drop_m = slope_drop((dir == 0 ? i : j) - 1, n_dir, side_lo, side_hi);
+  const int drop_p = slope_drop(dir == 0 ? i : j, n_dir, side_lo, side_hi);
+  muscl_pair(w, drop_m, drop_p, gamma, ul, ur);
+}
+
 template <class T, int ORDER>
 __host__ __device__ __forceinline__ void mp_char_face(const GridD& g, int dir, int i, int j, T gamma, const StateView& u,
                                              const double* bxc, const double* byc, St<T>& ul, St<T>& ur,

@@ -79,6 +79,33 @@ def test_faces_at_tile_edges(oracle, order, ng, nx, ny, state):
 
 
 @pytest.mark.parametrize("state", ["smooth", "at_rest", "supersonic", "dense", "thin"])
+@pytest.mark.parametrize("ng,nx,ny,sides", [(2, 63, 5, (0, 0, 0, 0)), (2, 33, 17, (1, 1, 1, 1)), (4, 65, 8, (2, 2, 0, 0)),
+                                            (3, 5, 31, (1, 2, 2, 1))])
+def test_muscl_faces_at_tile_edges(oracle, ng, nx, ny, sides, state):
+    """`thin` holds states whose pressure is near or below zero: the faces there
+    take the fallback chain, which the oracle's NaN pattern and values show."""
+    from quasar_amd import _lib
+    lib = _lib.load()
+    g, qg = oracle.grid(nx, ny, ng), qgrid(nx, ny, ng)
+    planes = planes_of("smooth" if state == "thin" else state, nx, ny, ng)
+    if state == "thin":
+        kinetic = sum(planes[c] ** 2 for c in (1, 2, 3)) / (2 * planes[0])
+        rng = np.random.default_rng(3)
+        planes[4] = kinetic + 0.5 * sum(planes[c] ** 2 for c in (5, 6, 7)) + 0.1 * rng.random(len(kinetic))
+    oracle.fill_ghosts(g, sides, sides, planes)
+    n = len(planes[0])
+    sc = scratch(qg)
+    for d in (0, 1):
+        ref16 = [np.zeros(n) for _ in range(16)]
+        oracle.reconstruct(g, d, 2, sides, G53, planes, ref16)
+        dev, out = to_dev(planes), zeros_dev(n, 16)
+        call(lib.qmhd_reconstruct, C.byref(qg), d, 2, flags(sides), G53, ptrs(dev), ptrs(out), C.c_void_p(sc.data_ptr()),
+             None)
+        m = face_mask(nx, ny, ng, d)
+        compare([q[m] for q in to_host(out)], [q[m] for q in ref16], (0, 8), ("muscl", d))
+
+
+@pytest.mark.parametrize("state", ["smooth", "at_rest", "supersonic", "dense", "thin"])
 @pytest.mark.parametrize("order,ng,nx,ny,sides", [(7, 4, 15, 17, 0), (7, 4, 16, 3, 1), (7, 4, 33, 64, 0), (5, 3, 31, 9, 1),
                                                   (5, 3, 17, 16, 0), (7, 4, 18, 5, 1), (7, 4, 5, 8, 0)])
 def test_cell_ez_at_tile_edges(oracle, order, ng, nx, ny, sides, state):
