@@ -335,16 +335,17 @@ int qmhd_solver_set_indicator(qmhd_solver* s, const float* host_params, float th
 /* Faces sent to the plain path and faces reconstructed since the last call. */
 int qmhd_solver_plain_faces(qmhd_solver* s, int64_t* plain, int64_t* total);
 /* ---- launch tuning and batched runs (no reference counterpart) --------
- * Tuning vector (QMHD_TUNING_INTS x int32): [0,1] flux block x, y; [2,3]
+ * Tuning vector (QMHD_TUNING_INTS x int32): [0,1] flux block x, y (MUSCL and
+ * first order; MP5/MP7 take their LDS tile); [2,3]
  * corner block x, y; [4,5] update block x, y (64..256 threads, multiples of
- * 64); [6] blocks of the persistent list launches of the learned form's plain
- * path; [7] cell E_z LDS tile (0: 16x16, 1: 32x8, 2: 8x32 cells; the learned
+ * 64); [6] most blocks of a face-list launch of the learned form's plain
+ * path; [7] cell E_z tile (0: 16x16, 1: 32x8, 2: 8x32 cells; the learned
  * form takes the full quadrature in whole tiles that hold a flagged cell, so
  * there the tile changes results and the autotuner leaves it at 0); [8] the
- * learned form's cheap-face tile for x faces (0: 64x4, 1: 32x8, 2: 128x2,
- * 3: 16x16, 4: 8x32 faces); [9] MP5/MP7 corner kernel (1: 16x16 LDS tile,
- * 0: one thread per corner in the [2,3] block); [10] the cheap-face tile for
- * y faces (as [8]); [11] reserved (0).  qmhd_solver_autotune times every
+ * learned form's cheap-face tile, both directions (0: 64x4, 1: 32x8, 2: 128x2,
+ * 3: 16x16, 4: 8x32 cells); [9] MP5/MP7 corner kernel (1: 16x16 LDS tile,
+ * 0: one thread per corner in the [2,3] block); [10] accepted as [8], without
+ * effect (the y faces of a cell are taken with its x faces); [11] reserved (0).  qmhd_solver_autotune times every
  * candidate of each knob over `trial_steps` steps (the live state is restored
  * afterwards) and keeps the fastest. */
 #define QMHD_TUNING_INTS 12

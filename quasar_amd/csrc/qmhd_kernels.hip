@@ -552,16 +552,17 @@ __global__ void counter_reset_kernel(unsigned long long* __restrict__ c, int n) 
 // unlimited MP5 interpolant, include/quasar/numerics/mp_limiter.hpp:182-191)
 // of the conserved cell averages, component by component, and the face normal
 // field.  Flagged faces, and cheap states that are not admissible, are listed
-// for the plain path (characteristic MP with its fallback chain).  The block
-// (64 x 4 faces) stages the cells its stencils read in LDS: 69 x 4 for x faces,
-// 64 x 9 for y faces.  Bound by memory: 117 B per face in FP32, 380 us per 4096^2
-// launch at a copy's rate.  It was bound by instruction issue (1.2k VALU
-// instructions a face: 16 flag reads with their range tests for every face,
-// index quotients by a width not known in advance, finiteness and pressure
-// tests and speeds formed apart): where no flag is near the block none is
-// read per face, and each state's 1/rho, velocity and pressure serve its
-// admissibility, its speed and its flux.  x / y faces 533 / 527 -> 445 / 499 us,
-// and 404 / 450 with the blocks of one XCD adjacent (halo rows from its L2).
+// for the plain path (characteristic MP with its fallback chain).  A block takes
+// a tile of cells and the low x and low y face of each from one staged set of
+// cells (32 x 8: 37 x 13).  Bound by memory: 64 B of state and 80 B of outputs
+// per cell in FP32, about 470 us per 4096^2 launch at a copy's rate.  Where no
+// flag is near the block none is read per face, and each state's 1/rho,
+// velocity and pressure serve its admissibility, its speed and its flux.
+// 4096^2, both directions: 1060 us with a launch per direction at 1.2k VALU
+// instructions a face (16 flag reads with range tests, index quotients by a
+// run-time width, tests, speeds and fluxes formed apart); 944 with the
+// instructions cut, 854 with the blocks of one XCD adjacent, 741 in one
+// launch.
 template <class T>
 __device__ __forceinline__ void cheap_face_flux(const St<T>& L, const St<T>& R, const Side<T>& l, const Side<T>& r,
                                                 int dir, T gamma, bool rate, St<T>& f, T& smax);
@@ -569,37 +570,44 @@ template <class T>
 __device__ __forceinline__ void store_face(const GridD& g, int dir, const FluxView<T>& flux, double* __restrict__ rate,
                                            std::size_t ko, const St<T>& f, T smax);
 
-// Cheap-reconstruction tiles (faces per block, TX x TY = 256 threads): the
-// autotuner picks one of kCheapTiles per face direction.  The tile stages the
-// 6-cell stencils along the face normal, so a wide tile suits x faces (64x4:
-// 69x4 cells) and a tall one y faces (16x16: 16x21, 8x32: 8x37 cells, where
-// 64x4 stages 64x9).
+// One direction's outputs of the cheap faces.
+template <class T>
+struct CheapFace {
+  IfaceView<T> out;
+  int* eq;
+  unsigned long long* count;
+  unsigned long long* list;
+  FluxView<T> flux;
+  double* rate;
+  int periodic;
+};
+template <class T>
+__device__ __forceinline__ CheapFace<T> queue_arg(const CheapFace<T>& f) {
+  return CheapFace<T>{queue_arg(f.out), queue_arg(f.eq), queue_arg(f.count), queue_arg(f.list), queue_arg(f.flux),
+                      queue_arg(f.rate), f.periodic};
+}
+
+// Cheap-reconstruction tiles (cells per block, TX x TY = 256 threads): the
+// autotuner picks one of kCheapTiles.  The tile stages TX + 5 by TY + 5 cells:
+// the squarer ones stage fewest (4096^2, reconstruction of a stage: 32 x 8 773 us,
+// 16 x 16 817, 64 x 4 834, 128 x 2 878, 8 x 32 947).
 constexpr int kCheapTileCount = 5;
 constexpr int kCheapTiles[kCheapTileCount][2] = {{64, 4}, {32, 8}, {128, 2}, {16, 16}, {8, 32}};
-template <int TX, int TY>
-constexpr int cheap_tile_cells() {
-  return (TX + 5) * TY > TX * (TY + 5) ? (TX + 5) * TY : TX * (TY + 5);
-}
 
 template <class T, int TX, int TY>
 __device__ __forceinline__ void cheap_reconstruct_kernel_tile(
-    const Blk& qb, const GridD& g, int dir, T gamma, const StateView& u, const double* __restrict__ bxc,
-    const double* __restrict__ byc, const uint8_t* __restrict__ cell_flags, const IfaceView<T>& out,
-    int* __restrict__ eq_flag, unsigned long long* __restrict__ fb_count, unsigned long long* __restrict__ fb_list,
-    const FluxView<T>& flux, double* __restrict__ rate, int periodic_dir) {
+    const Blk& qb, const GridD& g, T gamma, const StateView& u, const double* __restrict__ bxc,
+    const double* __restrict__ byc, const uint8_t* __restrict__ cell_flags, const CheapFace<T>& cheap_x,
+    const CheapFace<T>& cheap_y) {
 #include "tiles/cheap_reconstruct_kernel.inc"
 }
 
 template <class T, int TX, int TY>
-__global__ __launch_bounds__(256) void cheap_reconstruct_kernel(GridD g, int dir, T gamma, StateView u,
+__global__ __launch_bounds__(256) void cheap_reconstruct_kernel(GridD g, T gamma, StateView u,
                                                                 const double* __restrict__ bxc,
                                                                 const double* __restrict__ byc,
                                                                 const uint8_t* __restrict__ cell_flags,
-                                                                IfaceView<T> out, int* __restrict__ eq_flag,
-                                                                unsigned long long* __restrict__ fb_count,
-                                                                unsigned long long* __restrict__ fb_list,
-                                                                FluxView<T> flux, double* __restrict__ rate,
-                                                                int periodic_dir) {
+                                                                CheapFace<T> cheap_x, CheapFace<T> cheap_y) {
   [[maybe_unused]] const Blk qb = Blk::xcd_tiled();
 #include "tiles/cheap_reconstruct_kernel.inc"
 }
@@ -609,30 +617,22 @@ template <class T, int TX, int TY>
 struct cheap_reconstruct_kernel_q {
   struct Args {
     GridD g;
-    int dir;
     T gamma;
     StateView u;
     const double* bxc;
     const double* byc;
     const uint8_t* cell_flags;
-    IfaceView<T> out;
-    int* eq_flag;
-    unsigned long long* fb_count;
-    unsigned long long* fb_list;
-    FluxView<T> flux;
-    double* rate;
-    int periodic_dir;
+    CheapFace<T> cheap_x;
+    CheapFace<T> cheap_y;
   };
   static __device__ __forceinline__ void run(const Blk& qb, const Args& a) {
-    cheap_reconstruct_kernel_tile<T, TX, TY>(qb, queue_arg(a.g), queue_arg(a.dir), queue_arg(a.gamma), queue_arg(a.u),
-                                             queue_arg(a.bxc), queue_arg(a.byc), queue_arg(a.cell_flags),
-                                             queue_arg(a.out), queue_arg(a.eq_flag), queue_arg(a.fb_count),
-                                             queue_arg(a.fb_list), queue_arg(a.flux), queue_arg(a.rate),
-                                             queue_arg(a.periodic_dir));
+    cheap_reconstruct_kernel_tile<T, TX, TY>(qb, queue_arg(a.g), queue_arg(a.gamma), queue_arg(a.u), queue_arg(a.bxc),
+                                             queue_arg(a.byc), queue_arg(a.cell_flags), queue_arg(a.cheap_x),
+                                             queue_arg(a.cheap_y));
   }
   static void launch(dim3 grid, dim3 block, hipStream_t s, const Args& a) {
-    hipLaunchKernelGGL((cheap_reconstruct_kernel<T, TX, TY>), grid, block, 0, s, a.g, a.dir, a.gamma, a.u, a.bxc, a.byc,
-                       a.cell_flags, a.out, a.eq_flag, a.fb_count, a.fb_list, a.flux, a.rate, a.periodic_dir);
+    hipLaunchKernelGGL((cheap_reconstruct_kernel<T, TX, TY>), grid, block, 0, s, a.g, a.gamma, a.u, a.bxc, a.byc,
+                       a.cell_flags, a.cheap_x, a.cheap_y);
   }
   static const void* tag() {
     static const char t = 0;
@@ -650,19 +650,12 @@ __global__ __launch_bounds__(256) void cheap_reconstruct_kernel_queue(
   [[maybe_unused]] const Blk qb = qtile.blk;
   const typename cheap_reconstruct_kernel_q<T, TX, TY>::Args& qa = qargs[qtile.run];
   GridD g = qa.g;
-  int dir = qa.dir;
   T gamma = qa.gamma;
   StateView u = queue_arg(qa.u);
   const double* __restrict__ bxc = queue_arg(qa.bxc);
   const double* __restrict__ byc = queue_arg(qa.byc);
   const uint8_t* __restrict__ cell_flags = queue_arg(qa.cell_flags);
-  IfaceView<T> out = queue_arg(qa.out);
-  int* __restrict__ eq_flag = queue_arg(qa.eq_flag);
-  unsigned long long* __restrict__ fb_count = queue_arg(qa.fb_count);
-  unsigned long long* __restrict__ fb_list = queue_arg(qa.fb_list);
-  FluxView<T> flux = queue_arg(qa.flux);
-  double* __restrict__ rate = queue_arg(qa.rate);
-  int periodic_dir = qa.periodic_dir;
+  const CheapFace<T> cheap_x = queue_arg(qa.cheap_x), cheap_y = queue_arg(qa.cheap_y);
 #include "tiles/cheap_reconstruct_kernel.inc"
 }
 template <class T, int TX, int TY>
@@ -2026,26 +2019,25 @@ template <class T>
 void launch_reconstruct_learned(const GridD& g, int order, double gamma, const Flags4& flags, const StateView& u,
                                 const double* bxc, const double* byc, const uint8_t* cell_flags,
                                 const FaceOut<T>* out, unsigned long long* plain_total, hipStream_t stream,
-                                int list_blocks, const int* cheap_tile) {
+                                int list_blocks, int cheap_tile) {
   const T gamma_t = T(gamma);
-  for (int dir = 0; dir < 2; ++dir) {
-    if (cheap_tile[dir] < 0 || cheap_tile[dir] >= kCheapTileCount)
-      throw std::invalid_argument("reconstruct launch: cheap tile choice is 0..4");
-  }
-  for (int dir = 0; dir < 2; ++dir) {
-    const dim3 l = recon_faces(g, dir), cb(kCheapTiles[cheap_tile[dir]][0], kCheapTiles[cheap_tile[dir]][1]);
+  if (cheap_tile < 0 || cheap_tile >= kCheapTileCount)
+    throw std::invalid_argument("reconstruct launch: cheap tile choice is 0..4");
+  const dim3 cb(kCheapTiles[cheap_tile][0], kCheapTiles[cheap_tile][1]);
+  auto side = [&](int dir) {
     const FaceOut<T>& o = out[dir];
-    auto cheap = [&](auto q) {
-      go<decltype(q)>(blocks2d(l.x, l.y, cb), cb, stream, g, dir, gamma_t, u, bxc, byc, cell_flags, o.states, o.eq,
-                      o.list.count, o.list.faces, o.flux, o.rate, periodic_of(flags, dir));
-    };
-    switch (cheap_tile[dir]) {
-      case 0: cheap(cheap_reconstruct_kernel_q<T, kCheapTiles[0][0], kCheapTiles[0][1]>{}); break;
-      case 1: cheap(cheap_reconstruct_kernel_q<T, kCheapTiles[1][0], kCheapTiles[1][1]>{}); break;
-      case 2: cheap(cheap_reconstruct_kernel_q<T, kCheapTiles[2][0], kCheapTiles[2][1]>{}); break;
-      case 3: cheap(cheap_reconstruct_kernel_q<T, kCheapTiles[3][0], kCheapTiles[3][1]>{}); break;
-      default: cheap(cheap_reconstruct_kernel_q<T, kCheapTiles[4][0], kCheapTiles[4][1]>{}); break;
-    }
+    return CheapFace<T>{o.states, o.eq, o.list.count, o.list.faces, o.flux, o.rate, periodic_of(flags, dir)};
+  };
+  auto cheap = [&](auto q) {
+    go<decltype(q)>(blocks2d(g.nx + 2 * g.ng, g.ny + 2 * g.ng, cb), cb, stream, g, gamma_t, u, bxc, byc, cell_flags,
+                    side(0), side(1));
+  };
+  switch (cheap_tile) {
+    case 0: cheap(cheap_reconstruct_kernel_q<T, kCheapTiles[0][0], kCheapTiles[0][1]>{}); break;
+    case 1: cheap(cheap_reconstruct_kernel_q<T, kCheapTiles[1][0], kCheapTiles[1][1]>{}); break;
+    case 2: cheap(cheap_reconstruct_kernel_q<T, kCheapTiles[2][0], kCheapTiles[2][1]>{}); break;
+    case 3: cheap(cheap_reconstruct_kernel_q<T, kCheapTiles[3][0], kCheapTiles[3][1]>{}); break;
+    default: cheap(cheap_reconstruct_kernel_q<T, kCheapTiles[4][0], kCheapTiles[4][1]>{}); break;
   }
   // Enough blocks to fill the device at the MP kernel's occupancy (the plain
   // list can hold a large share of the faces), no more than the list can fill:
@@ -2262,7 +2254,7 @@ hipError_t upload_quad_rows(const QuadRows& rows) {
                                        const uint8_t*, hipStream_t, int);                                         \
   template void launch_reconstruct_learned<T>(const GridD&, int, double, const Flags4&, const StateView&,           \
                                               const double*, const double*, const uint8_t*, const FaceOut<T>*,     \
-                                              unsigned long long*, hipStream_t, int, const int*);
+                                              unsigned long long*, hipStream_t, int, int);
 QMHD_INSTANTIATE_LEARNED(double)
 QMHD_INSTANTIATE_LEARNED(float)
 #undef QMHD_INSTANTIATE_LEARNED

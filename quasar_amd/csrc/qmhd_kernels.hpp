@@ -111,7 +111,7 @@ template <class T>
 void launch_reconstruct_learned(const GridD& g, int order, double gamma, const Flags4& flags, const StateView& u,
                                 const double* bxc, const double* byc, const uint8_t* cell_flags,
                                 const FaceOut<T>* out, unsigned long long* plain_total, hipStream_t stream,
-                                int list_blocks, const int* cheap_tile);
+                                int list_blocks, int cheap_tile);
 // `block` shapes the orders without transverse quadrature (MP5/MP7 take their
 // LDS tile).
 template <class T>
@@ -123,7 +123,7 @@ void launch_cfl_reduce(const GridD& g, const double* rate_x, const double* rate_
 // cells per block.  MP5/MP7 corners: `tiled` selects the 16x16 LDS-tile kernel,
 // otherwise one thread per corner in `block`-shaped blocks.  Learned
 // reconstruction: `cheap_tile` selects the cheap faces' tile, 0: 64x4, 1: 32x8,
-// 2: 128x2, 3: 16x16, 4: 8x32 faces per block.
+// 2: 128x2, 3: 16x16, 4: 8x32 cells per block.
 template <class T>
 void launch_cell_emf(const GridD& g, int order, const Flags4& flags, double gamma, const StateView& u,
                      const double* bxc, const double* byc, double* cell_ez, hipStream_t stream,

@@ -503,11 +503,10 @@ class Solver {
                             FaceList{lists + dir, reinterpret_cast<unsigned long long*>(fb_list_[dir].p)},
                             FaceList{lists + 2 + dir, reinterpret_cast<unsigned long long*>(fb2_list_[dir].p)}};
     }
-    const int cheap[2] = {tuning_.cheap_tile, tuning_.cheap_tile_y};
     clock_.timed(QMHD_KERNEL_RECONSTRUCT, stream_, [&] {
       if (learned)
         launch_reconstruct_learned<T>(g_, order, gamma_, field_, r.view(), r.bxc.p, r.byc.p, flags(), out, plain_total(),
-                                      stream_, tuning_.list_blocks, cheap);
+                                      stream_, tuning_.list_blocks, tuning_.cheap_tile);
       else
         launch_reconstruct<T>(g_, order, gamma_, field_, r.view(), r.bxc.p, r.byc.p, out, 0, 2, stream_);
     });
@@ -662,8 +661,8 @@ class Solver {
     dim3 flux{64, 4}, corner{64, 4}, update{64, 4};
     int list_blocks{1024};
     int emf_tile{0};      // cell E_z LDS tile: 16x16, 32x8, 8x32
-    int cheap_tile{0};    // learned form's cheap-face tile, x faces: 64x4, 32x8, 128x2, 16x16, 8x32
-    int cheap_tile_y{1};  // the same for y faces
+    int cheap_tile{1};    // learned form's cheap-face tile: 64x4, 32x8, 128x2, 16x16, 8x32
+    int cheap_tile_y{1};  // kept and validated; both directions run in cheap_tile's tile
     int corner_tiled{1};  // MP5/MP7 corners: LDS tile (1) or one thread per corner in `corner` blocks (0)
   };
   static bool valid_block(int bx, int by) {
@@ -753,7 +752,6 @@ class Solver {
     // tile is a knob of the plain method only.
     if (order_ >= 5 && !learned_) choose(tuning_.emf_tile, {0, 1, 2}, QMHD_KERNEL_CELL_EMF);
     if (learned_) choose(tuning_.cheap_tile, {0, 1, 2, 3, 4}, QMHD_KERNEL_RECONSTRUCT);
-    if (learned_) choose(tuning_.cheap_tile_y, {0, 1, 2, 3, 4}, QMHD_KERNEL_RECONSTRUCT);
     if (learned_) {
       const int grids[] = {256, 512, 1024, 2048, 4096};
       int best = tuning_.list_blocks;
