@@ -35,10 +35,10 @@ PEAK_HBM_GBS = 8000.0
 PEAK_FP64_TFLOPS = 78.6
 
 # Algorithmic cost per unit of each launch kind, FP64 MP7.  Units per launch
-# are given by `units()`: reconstruct covers the (n+1)(n+2ng) faces of its
-# direction (the transverse quadrature needs the ghost rows), flux and corner
-# the (n+1)^2 faces/corners, cell_emf and update the n^2 cells, prep the
-# (n+2ng)^2 padded cells.
+# are given by `units()`: one reconstruct launch covers the (n+1)(n+2ng) faces
+# of each direction (the transverse quadrature needs the ghost rows), one flux
+# launch the (n+1)^2 faces of each, corner the (n+1)^2 corners, cell_emf and
+# update the n^2 cells, prep the (n+2ng)^2 padded cells.
 #   bytes: every plane the kernel must read once and write once (8 B words),
 #   flops: the arithmetic the algorithm needs for one unit (add, mul, div and
 #          sqrt count 1, fma 2): the reference's operation sequence for that
@@ -60,9 +60,9 @@ UNIT_COST = {
     # flux difference, curl, Shu-Osher combine; 8 base + 8 stage + 2x8 flux +
     # E_z planes in, 8 planes out
     "update": {"bytes": 8 * (8 + 8 + 16 + 1 + 8), "flops": 90},
-    # two correctly rounded 8-tap collocations, theta and checks; 8 candidate +
-    # 8 base + 2 base collocated field planes in, 2 collocated field planes out
-    "prep": {"bytes": 8 * (8 + 8 + 2 + 2), "flops": 1000},
+    # two correctly rounded 8-tap collocations, theta and checks; 8 candidate
+    # planes in (the base only where a check is close), 2 collocated planes out
+    "prep": {"bytes": 8 * (8 + 2), "flops": 1000},
 }
 NG = 4
 
@@ -339,8 +339,10 @@ def _interior(solver, n: int):
 
 def units(kind: str, n: int) -> int:
     if kind == "reconstruct":
-        return (n + 1) * (n + 2 * NG)
-    if kind in ("flux", "corner"):
+        return 2 * (n + 1) * (n + 2 * NG)
+    if kind == "flux":
+        return 2 * (n + 1) * (n + 1)
+    if kind == "corner":
         return (n + 1) * (n + 1)
     if kind == "prep":
         return (n + 2 * NG) * (n + 2 * NG)
@@ -413,12 +415,11 @@ def measured_traffic(kind: str, n: int):
 
 # Kernels of each timed kind of the FP64 MP7 step (one dispatch of each per
 # launch of the kind).  A symbol matches every instantiation whose name
-# contains it (the flux kernel has one per direction); their per-dispatch
-# values are averaged.
+# contains it; their per-dispatch values are averaged.
 KERNEL_SYMBOLS = {
     "prep": ("prep_kernel<true, 8>",),
-    "reconstruct": ("reconstruct_kernel<double, 7>", "reconstruct_fallback_kernel<double, 7>"),
-    "flux": ("flux_kernel<double, 7, false, ",),
+    "reconstruct": ("reconstruct_kernel_queue<double, 7>", "reconstruct_fallback_kernel_queue<double, 7>"),
+    "flux": ("flux_kernel_queue<double, 7, false>",),
     "cell_emf": ("cell_emf_kernel<double, 7, false, 16, 16>",),
     "corner": ("corner_tiled_kernel<double, 7>",),
     "update": ("update_kernel<double>",),
