@@ -35,8 +35,11 @@ struct FluxView {
 };
 
 // Device-resident per-step status, reduced with order-independent atomics on
-// the bit patterns of non-negative doubles.
-struct StepStatus {
+// the bit patterns of non-negative doubles.  The first 128 bytes (one cache
+// line of the L2) are what the checks and reductions of a launch update; the
+// face-list counters, which a launch's first block clears with plain stores,
+// have the next line to themselves.
+struct alignas(128) StepStatus {
   unsigned long long theta[4];     // per-stage admissible fraction (min); [3] = stage 2, second collocation
   unsigned long long live_theta0;  // live state, high-order collocation (min)
   unsigned long long live_theta1;  // live state, two-face collocation (min)
@@ -45,8 +48,8 @@ struct StepStatus {
   unsigned long long max_rate;       // CFL additive rate (max)
   double dt;                         // device-side dt of the auto-dt loop
   double time;                       // accumulated simulated time
-  unsigned long long lists[4];       // faces listed for the general path (x, y), and again (x, y); see FaceOut
-  double pad[1];
+  // Faces listed for the general path (x, y), and again (x, y); see FaceOut.
+  alignas(128) unsigned long long lists[4];
 };
 
 struct IcSpecD {
