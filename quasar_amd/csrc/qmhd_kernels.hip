@@ -1804,12 +1804,12 @@ struct QueueTiles<status_reset_kernel_q> {
 // step is rejected and the run is held: its later attempts in the same batch
 // call commit nothing, and the host's positivity controller finishes its
 // steps after the graph launches).
-__device__ __forceinline__ void batch_commit_kernel_tile(const Blk& qb, const StepStatus* __restrict__ st,
+__device__ __forceinline__ void batch_commit_kernel_tile(const Blk& qb, StepStatus* __restrict__ st,
                                                          double* __restrict__ acc) {
 #include "tiles/batch_commit_kernel.inc"
 }
 
-__global__ void batch_commit_kernel(const StepStatus* __restrict__ st, double* __restrict__ acc) {
+__global__ void batch_commit_kernel(StepStatus* __restrict__ st, double* __restrict__ acc) {
   [[maybe_unused]] const Blk qb = Blk::native();
 #include "tiles/batch_commit_kernel.inc"
 }
@@ -1817,7 +1817,7 @@ __global__ void batch_commit_kernel(const StepStatus* __restrict__ st, double* _
 // Queue form of batch_commit_kernel (one launch over the tiles of many runs).
 struct batch_commit_kernel_q {
   struct Args {
-    const StepStatus* st;
+    StepStatus* st;
     double* acc;
   };
   static __device__ __forceinline__ void run(const Blk& qb, const Args& a) {
@@ -1839,7 +1839,7 @@ __global__ void batch_commit_kernel_queue(const batch_commit_kernel_q::Args* __r
   const QueueTile qtile = queue_tile(qruns, qnruns);
   [[maybe_unused]] const Blk qb = qtile.blk;
   const batch_commit_kernel_q::Args& qa = qargs[qtile.run];
-  const StepStatus* __restrict__ st = queue_arg(qa.st);
+  StepStatus* __restrict__ st = queue_arg(qa.st);
   double* __restrict__ acc = queue_arg(qa.acc);
 #include "tiles/batch_commit_kernel.inc"
 }
@@ -1900,7 +1900,7 @@ struct QueueTiles<batch_restore_kernel_q> {
 // ---------------------------------------------------------------------------
 // Host launchers.
 
-void launch_batch_commit(const StepStatus* status, double* acc, hipStream_t stream) {
+void launch_batch_commit(StepStatus* status, double* acc, hipStream_t stream) {
   go<batch_commit_kernel_q>(dim3(1), dim3(64), stream, status, acc);
 }
 

@@ -48,6 +48,7 @@ struct alignas(128) StepStatus {
   unsigned long long max_rate;       // CFL additive rate (max)
   double dt;                         // device-side dt of the auto-dt loop
   double time;                       // accumulated simulated time
+  unsigned long long owned;          // batched steps: the live state is one the solver made (see prep_kernel)
   // Faces listed for the general path (x, y), and again (x, y); see FaceOut.
   alignas(128) unsigned long long lists[4];
 };
@@ -66,6 +67,11 @@ struct IcSpecD {
   unsigned long long noise_seed;
   double blob_half;
 };
+
+// launch_prep's solver_owned: the solver made the live state (1), a caller
+// seeded it (0), or status.owned says which: a captured step is replayed on
+// states of both kinds.
+constexpr int kOwnedByStatus = -1;
 
 hipError_t upload_quad_rows(const QuadRows& rows);
 void build_quad_rows(QuadRows& rows);
@@ -162,7 +168,7 @@ void launch_status_reset(StepStatus* s, hipStream_t stream);
 // Unless the step was accepted, the restore launch copies the live state over
 // the candidate, so the next step (which reads the candidate register) starts
 // again from the same state.
-void launch_batch_commit(const StepStatus* status, double* acc, hipStream_t stream);
+void launch_batch_commit(StepStatus* status, double* acc, hipStream_t stream);
 void launch_batch_restore(const GridD& g, const double* acc, const StateView& live, const StateOut& cand,
                           hipStream_t stream);
 

@@ -541,9 +541,10 @@ class Solver {
   // Ghost fill, collocation + live checks, reconstruction and fluxes of the live
   // register at `order`, additive CFL rate reduction.  Leaves the flux cache
   // valid for `order`.
-  void issue_rate_phase(int order) {
+  void issue_rate_phase(int order) { issue_rate_phase(order, solver_owned_ ? 1 : 0); }
+  void issue_rate_phase(int order, int owned) {
     launch_status_reset(status_, stream_);
-    issue_live_prep();
+    issue_live_prep(owned);
     issue_faces(L_, order, true);
     clock_.timed(QMHD_KERNEL_REDUCE, stream_,
                  [&] { launch_cfl_reduce(g_, rate_x_.p, rate_y_.p, &status_->max_rate, stream_); });
@@ -593,11 +594,12 @@ class Solver {
   }
 
   // Ghost fill and live-state preparation of the live register.
-  void issue_live_prep() {
+  void issue_live_prep() { issue_live_prep(solver_owned_ ? 1 : 0); }
+  void issue_live_prep(int owned) {
     clock_.timed(QMHD_KERNEL_GHOSTS, stream_, [&] { launch_ghosts(g_, fluid_, field_, reg_[L_].out(), stream_); });
     clock_.timed(QMHD_KERNEL_PREP, stream_, [&] {
       launch_prep(g_, reg_[L_].view(), reg_[L_].bxc.p, reg_[L_].byc.p, reg_[L_].view(), reg_[L_].bxc.p,
-                  reg_[L_].byc.p, -1, 0, 0, 1, solver_owned_ ? 1 : 0, status_, stream_, !fp32_);
+                  reg_[L_].byc.p, -1, 0, 0, 1, owned, status_, stream_, !fp32_);
     });
   }
 
@@ -785,7 +787,7 @@ class Solver {
       throw std::invalid_argument("MhdSolver2D: indicator 'mlp' needs its network (set_indicator) before stepping");
     double* acc = batch_acc();
     const double eff = order_ >= 5 ? std::min(cfl_, 0.2) : cfl_;
-    issue_rate_phase(order_);
+    issue_rate_phase(order_, kOwnedByStatus);
     launch_dt(&status_->max_rate, eff, g_.dx, g_.dy, &status_->dt, nullptr, stream_);
     issue_attempt(0.0, &status_->dt, 0, false);
     launch_batch_commit(status_, acc, stream_);
@@ -796,7 +798,15 @@ class Solver {
   void swap_roles() {
     std::swap(L_, C_);
     cache_order_ = -1;
-    solver_owned_ = true;
+  }
+  // Whether the live state is one the solver made: the host's word for it, and
+  // the batched step's (status.owned, which an accepted step sets).
+  bool owned() const { return solver_owned_; }
+  void set_owned(bool v) { solver_owned_ = v; }
+  void set_status_owned(bool v) {
+    const unsigned long long word = v ? 1ull : 0ull;
+    QMHD_HIP(hipMemcpyAsync(&status_->owned, &word, sizeof word, hipMemcpyHostToDevice, stream_));
+    QMHD_HIP(hipStreamSynchronize(stream_));
   }
   void batch_status(long long* accepted, long long* rejected, int* fatal, double* sim_time) {
     double h[8];
@@ -1741,6 +1751,10 @@ struct qmhd_batch {
   // positivity controller after a rejected step held it.
   std::vector<long long> requested, host_accepted;
   std::vector<double> host_time;
+  // Steps the device had accepted when last looked at, and what status.owned
+  // of a run holds.
+  std::vector<double> seen;
+  std::vector<char> status_owned;
   int parity{0};           // parity of the next step
   int solver_parity{0};    // parity the runs' register roles reflect
   // Tile work-queue mode: the recorded launch slots of each parity (one
@@ -1776,6 +1790,12 @@ struct qmhd_batch {
     solver_parity = want;
   }
 
+  // Brings status.owned of run k in line with the run's own word.
+  void tell_owned(std::size_t k) {
+    runs[k]->set_status_owned(runs[k]->owned());
+    status_owned[k] = runs[k]->owned() ? 1 : 0;
+  }
+
   // Streams mode: the step of every run, each on its own stream, forked from
   // and joined back to the master stream, captured as one graph per register
   // parity.  Queue mode: every run's step recorded, and each launch slot
@@ -1795,6 +1815,9 @@ struct qmhd_batch {
     requested.assign(runs.size(), 0);
     host_accepted.assign(runs.size(), 0);
     host_time.assign(runs.size(), 0.0);
+    seen.assign(runs.size(), 0.0);
+    status_owned.assign(runs.size(), 0);
+    for (std::size_t k = 0; k < runs.size(); ++k) tell_owned(k);
     if (queued) {
       record_queue();
       capture_queue();
@@ -1970,6 +1993,7 @@ struct qmhd_batch {
     requested = req0;
     host_accepted = acc0;
     host_time = time0;
+    for (std::size_t k = 0; k < runs.size(); ++k) tell_owned(k);
     queue_blocks = best;
     capture_queue();
     return best;
@@ -1982,6 +2006,7 @@ struct qmhd_batch {
       const int expect = parity == 0 ? live0[k] : cand0[k];
       if (runs[k]->live_index() != expect)
         throw std::invalid_argument("qmhd_batch_run: a run was stepped outside the batch");
+      if (runs[k]->owned() != (status_owned[k] != 0)) tell_owned(k);
     }
     // Segments of at most kSegment graph launches: a run held by a rejected
     // step waits at most one segment before its own loop finishes that
@@ -2011,6 +2036,11 @@ struct qmhd_batch {
     qmhd::Solver* r = runs[k];
     double acc[8];
     r->batch_counters(acc);
+    if (acc[0] > seen[k]) {
+      seen[k] = acc[0];
+      r->set_owned(true);
+      status_owned[k] = 1;
+    }
     if (acc[2] != 0.0 || acc[5] == 0.0) return;
     const long long remaining = requested[k] - static_cast<long long>(acc[0]) - host_accepted[k];
     if (remaining > 0) {
@@ -2025,6 +2055,7 @@ struct qmhd_batch {
       }
       host_accepted[k] += done;
       host_time[k] += t;
+      if (!status_owned[k]) tell_owned(k);
     }
     r->batch_set_counter(5, 0.0);
     r->set_live_register(parity == 0 ? live0[k] : cand0[k]);
