@@ -386,6 +386,11 @@ int qmhd_batch_create_queued(qmhd_solver* const* runs, int count, int queue_bloc
 int qmhd_batch_autotune(qmhd_batch* b, int trial_steps, int* queue_blocks);
 void qmhd_batch_destroy(qmhd_batch* b);
 int qmhd_batch_run(qmhd_batch* b, int steps);
+/* Runs found fatal by the calls so far, and why (and after how many accepted
+ * steps) run `run` stopped: "" for a run that has not (text owned by the
+ * batch, valid until it is destroyed). */
+int qmhd_batch_fatal_runs(const qmhd_batch* b);
+const char* qmhd_batch_run_failure(const qmhd_batch* b, int run);
 int qmhd_batch_run_status(qmhd_batch* b, int run, int64_t* accepted, int64_t* rejected, int* fatal,
                           double* sim_time);
 

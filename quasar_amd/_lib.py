@@ -69,7 +69,7 @@ EXPORTS = [
     "qmhd_solver_set_indicator", "qmhd_solver_plain_faces", "qmhd_solver_cell_features",
     "qmhd_solver_cell_labels", "qmhd_solver_autotune", "qmhd_solver_set_tuning", "qmhd_solver_get_tuning",
     "qmhd_batch_create", "qmhd_batch_create_queued", "qmhd_batch_autotune", "qmhd_batch_destroy", "qmhd_batch_run",
-    "qmhd_batch_run_status",
+    "qmhd_batch_run_status", "qmhd_batch_fatal_runs", "qmhd_batch_run_failure",
 ]
 
 MLP_FEATURES = 100
@@ -165,6 +165,9 @@ def load() -> C.CDLL:
     L.qmhd_batch_destroy.argtypes = [VP]
     L.qmhd_batch_destroy.restype = None
     L.qmhd_batch_run.argtypes = [VP, C.c_int]
+    L.qmhd_batch_fatal_runs.argtypes = [VP]
+    L.qmhd_batch_run_failure.argtypes = [VP, C.c_int]
+    L.qmhd_batch_run_failure.restype = C.c_char_p
     L.qmhd_batch_run_status.argtypes = [VP, C.c_int, C.POINTER(I64), C.POINTER(I64), C.POINTER(C.c_int), DP]
     _lib = L
     return L

@@ -13,6 +13,7 @@ from __future__ import annotations
 
 import ctypes as C
 import math
+import warnings
 from typing import Dict, List, Sequence
 
 import numpy as np
@@ -36,6 +37,7 @@ class Batch:
         self._lib = _lib.load()
         self._solvers = list(solvers)
         self.queue = bool(queue)
+        self._told = set()
         arr = (C.c_void_p * len(self._solvers))(*[s._h.value for s in self._solvers])
         h = C.c_void_p()
         if self.queue:
@@ -58,7 +60,20 @@ class Batch:
             self._h = None
 
     def run(self, steps: int) -> None:
+        """Advance every run by `steps`; a run that stops on the way is told
+        in a RuntimeWarning (the other runs take their steps)."""
+        before = self._lib.qmhd_batch_fatal_runs(self._h)
         _lib.check(self._lib.qmhd_batch_run(self._h, int(steps)))
+        if self._lib.qmhd_batch_fatal_runs(self._h) != before:
+            for k in range(len(self._solvers)):
+                why = self.failure(k)
+                if why and k not in self._told:
+                    self._told.add(k)
+                    warnings.warn(f"batch run {k} stopped {why}", RuntimeWarning, stacklevel=2)
+
+    def failure(self, run: int) -> str:
+        """Why run `run` stopped, or "" where it has not."""
+        return self._lib.qmhd_batch_run_failure(self._h, int(run)).decode()
 
     def status(self, run: int) -> Dict:
         a, r = C.c_int64(), C.c_int64()

@@ -73,6 +73,10 @@ struct IcSpecD {
 // states of both kinds.
 constexpr int kOwnedByStatus = -1;
 
+// Why a batched run stopped (acc[6] of launch_batch_commit; acc[7] the value
+// that failed).
+enum BatchStop { kStopNone, kStopDivergence, kStopInadmissible, kStopRate };
+
 hipError_t upload_quad_rows(const QuadRows& rows);
 void build_quad_rows(QuadRows& rows);
 

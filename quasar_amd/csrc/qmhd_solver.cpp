@@ -19,6 +19,7 @@
 #include <cstring>
 #include <limits>
 #include <memory>
+#include <sstream>
 #include <stdexcept>
 #include <string>
 #include <vector>
@@ -1751,10 +1752,12 @@ struct qmhd_batch {
   // positivity controller after a rejected step held it.
   std::vector<long long> requested, host_accepted;
   std::vector<double> host_time;
-  // Steps the device had accepted when last looked at, and what status.owned
-  // of a run holds.
+  // Steps the device had accepted when last looked at, what status.owned of a
+  // run holds, and why a run stopped.
   std::vector<double> seen;
   std::vector<char> status_owned;
+  std::vector<std::string> failure;
+  int fatal_runs{0};
   int parity{0};           // parity of the next step
   int solver_parity{0};    // parity the runs' register roles reflect
   // Tile work-queue mode: the recorded launch slots of each parity (one
@@ -1816,6 +1819,7 @@ struct qmhd_batch {
     host_accepted.assign(runs.size(), 0);
     host_time.assign(runs.size(), 0.0);
     seen.assign(runs.size(), 0.0);
+    failure.assign(runs.size(), std::string());
     status_owned.assign(runs.size(), 0);
     for (std::size_t k = 0; k < runs.size(); ++k) tell_owned(k);
     if (queued) {
@@ -2028,6 +2032,23 @@ struct qmhd_batch {
     }
   }
 
+  // Keeps what stopped run k (told once).
+  void stopped(std::size_t k, const double acc[8], const char* controller = nullptr) {
+    if (!failure[k].empty()) return;
+    ++fatal_runs;
+    std::ostringstream why;
+    why << "after " << static_cast<long long>(acc[0]) + host_accepted[k] << " accepted steps: ";
+    switch (static_cast<int>(acc[6])) {
+      case qmhd::kStopDivergence:
+        why << "live magnetic field is not discretely divergence-free (relative residual " << acc[7] << ")";
+        break;
+      case qmhd::kStopInadmissible: why << "live state is not admissible (fraction " << acc[7] << ")"; break;
+      case qmhd::kStopRate: why << "non-finite CFL rate (" << acc[7] << ")"; break;
+      default: why << (controller ? controller : "stopped before this batch"); break;
+    }
+    failure[k] = why.str();
+  }
+
   // A run held by a rejected step finishes its requested steps through its
   // own auto-dt loop, whose positivity controller takes the retries
   // (mhd_solver.cpp:965-1143), and rejoins the batch on the register the
@@ -2041,6 +2062,7 @@ struct qmhd_batch {
       r->set_owned(true);
       status_owned[k] = 1;
     }
+    if (acc[2] != 0.0) stopped(k, acc);
     if (acc[2] != 0.0 || acc[5] == 0.0) return;
     const long long remaining = requested[k] - static_cast<long long>(acc[0]) - host_accepted[k];
     if (remaining > 0) {
@@ -2048,8 +2070,11 @@ struct qmhd_batch {
       double t = 0.0;
       try {
         r->run(static_cast<int>(remaining), 0.0, &done, &t);
-      } catch (const std::exception&) {
+      } catch (const std::exception& e) {
         r->batch_set_counter(2, 1.0);
+        acc[2] = 1.0;
+        acc[6] = qmhd::kStopNone;
+        stopped(k, acc, e.what());
         r->set_live_register(parity == 0 ? live0[k] : cand0[k]);
         return;
       }
@@ -2101,6 +2126,13 @@ void qmhd_batch_destroy(qmhd_batch* b) { delete b; }
 
 int qmhd_batch_run(qmhd_batch* b, int steps) {
   return guarded([&] { b->run(steps); });
+}
+
+int qmhd_batch_fatal_runs(const qmhd_batch* b) { return b->fatal_runs; }
+
+const char* qmhd_batch_run_failure(const qmhd_batch* b, int run) {
+  if (run < 0 || run >= static_cast<int>(b->runs.size())) return "";
+  return b->failure[run].c_str();
 }
 
 int qmhd_batch_run_status(qmhd_batch* b, int run, int64_t* accepted, int64_t* rejected, int* fatal,
