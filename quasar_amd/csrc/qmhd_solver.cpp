@@ -1876,20 +1876,21 @@ struct qmhd_batch {
           throw std::invalid_argument("qmhd_batch: queue mode needs runs with the same scheme, form and launch shapes");
       for (std::size_t i = 0; i < n; ++i) {
         const qmhd::Recorder::Entry& e0 = rec[0][i];
-        for (std::size_t k = 1; k < runs.size(); ++k) {
-          const qmhd::Recorder::Entry& e = rec[k][i];
-          if (e.tag != e0.tag || e.joins != e0.joins || e.block.x != e0.block.x || e.block.y != e0.block.y ||
-              e.block.z != e0.block.z || e.args.size() != e0.args.size())
-            throw std::invalid_argument(
-                "qmhd_batch: queue mode needs runs with the same scheme, form and launch shapes");
-        }
+        // A joining entry's tiles follow its predecessor's in one launch.
+        const std::size_t last = i + 1 < n && rec[0][i + 1].joins ? i + 1 : i;
+        for (std::size_t q = i; q <= last; ++q)
+          for (std::size_t k = 0; k < runs.size(); ++k) {
+            const qmhd::Recorder::Entry& e = rec[k][q];
+            if (e.tag != e0.tag || e.joins != (q > i) || e.block.x != e0.block.x || e.block.y != e0.block.y ||
+                e.block.z != e0.block.z || e.args.size() != e0.args.size())
+              throw std::invalid_argument(
+                  "qmhd_batch: queue mode needs runs with the same scheme, form and launch shapes");
+          }
         Slot s;
         s.launch = e0.launch;
         s.block = e0.block;
         align(256);
         s.args_off = blob.size();
-        // A joining entry's tiles follow its predecessor's in one launch.
-        const std::size_t last = i + 1 < n && rec[0][i + 1].joins ? i + 1 : i;
         for (std::size_t q = i; q <= last; ++q)
           for (std::size_t k = 0; k < runs.size(); ++k)
             blob.insert(blob.end(), rec[k][q].args.begin(), rec[k][q].args.end());
