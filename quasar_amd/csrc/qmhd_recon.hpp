@@ -231,7 +231,9 @@ __host__ __device__ __forceinline__ bool mp_keeps(T vl, T v0, T em, T ep) {
 
 // Both face values of one wave: v[0 .. 2H+1] its union stencil, the left value
 // from cell H, the right one from cell H + 1 (mp_limit's operations; the
-// second differences, the median bound and the pair's extrema are shared).
+// second differences, the median bound and the pair's extrema are shared).  The
+// unlimited value, a sum over its stencil, is not finite where a cell's is not;
+// it stands then, since the median's minima and maxima would drop a NaN.
 template <class T, int ORDER>
 __host__ __device__ __forceinline__ void mp_pair(const T* v, T& left, T& right) {
 #pragma clang fp contract(off)
@@ -262,13 +264,13 @@ __host__ __device__ __forceinline__ void mp_pair(const T* v, T& left, T& right) 
     const T ul = fm(T(4), e1, m[2]), lc = fm(T(4.0 / 3.0), minmod_m4(d2, d1), fm(T(0.5), e1, m[2]));
     const T lo = hi2(alo, lo2(lo2(m[2], ul), lc)), hi = lo2(ahi, hi2(hi2(m[2], ul), lc));
     const T med = hi2(lo2(lo, hi), lo2(hi2(lo, hi), vl));
-    left = kl ? vl : med;
+    left = kl || !fin(vl) ? vl : med;
   }
   {
     const T ul = fm(T(-4), e3, m[3]), lc = fm(T(4.0 / 3.0), minmod_m4(d3, d4), fm(T(-0.5), e3, m[3]));
     const T lo = hi2(alo, lo2(lo2(m[3], ul), lc)), hi = lo2(ahi, hi2(hi2(m[3], ul), lc));
     const T med = hi2(lo2(lo, hi), lo2(hi2(lo, hi), vr));
-    right = kr ? vr : med;
+    right = kr || !fin(vr) ? vr : med;
   }
 }
 
