@@ -34,7 +34,10 @@ __host__ __device__ __forceinline__ float lo2(float a, float b) { return __built
 __host__ __device__ __forceinline__ float hi2(float a, float b) { return __builtin_fmaxf(a, b); }
 
 // sqrt(x) and 1 / (2 sqrt(x)) of a positive normal x (Goldschmidt from the
-// hardware's reciprocal square root).
+// hardware's reciprocal square root).  One Goldschmidt step leaves the inverse
+// 19 epsilon off in FP64, so where it is asked for it takes one more against
+// the rounded root: within 2 epsilon, as a quotient of the rounded root is (the
+// wave basis and the Alfven speeds divide by roots).
 __host__ __device__ __forceinline__ double sqrt_pos(double x, double& half_inv) {
 #if defined(__HIP_DEVICE_COMPILE__)
   const double y = __builtin_amdgcn_rsq(x);
@@ -42,8 +45,9 @@ __host__ __device__ __forceinline__ double sqrt_pos(double x, double& half_inv) 
   const double r = __builtin_fma(-g, h, 0.5);
   g = __builtin_fma(g, r, g);
   h = __builtin_fma(h, r, h);
-  half_inv = h;
-  return __builtin_fma(__builtin_fma(-g, g, x), h, g);
+  g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
+  half_inv = __builtin_fma(h + h, __builtin_fma(-g, h, 0.5), h);
+  return g;
 #else
   const double g = __builtin_sqrt(x);
   half_inv = 0.5 / g;
@@ -53,9 +57,11 @@ __host__ __device__ __forceinline__ double sqrt_pos(double x, double& half_inv) 
 __host__ __device__ __forceinline__ float sqrt_pos(float x, float& half_inv) {
 #if defined(__HIP_DEVICE_COMPILE__)
   const float y = __builtin_amdgcn_rsqf(x);
-  const float g = x * y, h = 0.5f * y;
-  half_inv = h;
-  return __builtin_fmaf(__builtin_fmaf(-g, g, x), h, g);
+  const float h = 0.5f * y;
+  float g = x * y;
+  g = __builtin_fmaf(__builtin_fmaf(-g, g, x), h, g);
+  half_inv = __builtin_fmaf(h + h, __builtin_fmaf(-g, h, 0.5f), h);
+  return g;
 #else
   const float g = __builtin_sqrtf(x);
   half_inv = 0.5f / g;
