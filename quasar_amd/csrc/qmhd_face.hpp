@@ -88,6 +88,15 @@ __host__ __device__ __forceinline__ void schedule_fence() {
 #endif
 }
 
+// Whether any lane of the wave has `b` (the host runs one lane).
+__host__ __device__ __forceinline__ bool any_lane(bool b) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __any(b);
+#else
+  return b;
+#endif
+}
+
 // What the solver needs of one state, in the frame of the face normal.
 template <class T>
 struct Side {
@@ -389,13 +398,24 @@ struct NodeRows<float, 5> {
   static __host__ __device__ __forceinline__ float mean(const QuadRows& t, int q) { return t.mp5_mean_f[q]; }
 };
 
+// side_of of a state u (s: u in the frame of the normal) where it may be within
+// rounding of zero pressure: the reference decides, and its pressure serves the
+// rate, which asks for its sign again (side_of's, rounded otherwise, is at or
+// below zero for some 8 % of the admissible states within 4 ulp of zero: an
+// infinite rate, which stops a run).
+template <class T>
+__host__ __device__ __forceinline__ bool decided_side(const St<T>& u, const St<T>& s, T gamma, Side<T>& o) {
+  bool good = side_of(s, gamma, o);
+  if (!good) good = admissible_state_p(u, gamma, o.p);
+  return good;
+}
+
 // Signal speed of a face's averages (infinite when one is not admissible).
 template <class T>
-__host__ __device__ __forceinline__ T base_rate(const St<T>& L, const Side<T>& l, bool good_l, const St<T>& R,
-                                                const Side<T>& r, bool good_r, int order, T gamma) {
-  const bool good = (good_l && good_r) || (fin(L.rho) && L.rho > T(0) && fin(R.rho) && R.rho > T(0));
+__host__ __device__ __forceinline__ T base_rate(const Side<T>& l, bool good_l, const Side<T>& r, bool good_r, int order,
+                                                T gamma) {
   const T v = rate_of(l, fast_of(l, l.bn2, gamma), r, fast_of(r, r.bn2, gamma), order);
-  return good ? v : Lim<T>::inf();
+  return good_l && good_r ? v : Lim<T>::inf();
 }
 
 // Flux (and signal speed, when `rate`) of a face at its averages: the orders
@@ -405,8 +425,8 @@ __host__ __device__ __forceinline__ St<T> average_flux(const St<T>& bL, const St
                                                        bool rate, T& smax) {
   const St<T> a = rot(bL, dir), b = rot(bR, dir);
   Side<T> l, r;
-  const bool good_l = side_of(a, gamma, l), good_r = side_of(b, gamma, r);
-  smax = rate ? base_rate(a, l, good_l, b, r, good_r, order, gamma) : T(0);
+  const bool good_l = decided_side(bL, a, gamma, l), good_r = decided_side(bR, b, gamma, r);
+  smax = rate ? base_rate(l, good_l, r, good_r, order, gamma) : T(0);
   T unused = T(0);
   return solve_face<LF>(a, b, l, r, dir, order, gamma, false, unused);
 }
@@ -417,7 +437,7 @@ __host__ __device__ __forceinline__ St<T> average_flux(const St<T>& bL, const St
 // flux of its averages: one more pass of the same loop, taken by waves that
 // hold such a face.
 template <class T, int ORDER, bool LF>
-__device__ __forceinline__ St<T> node_flux(const QuadRows& rows, const T* diff, int cs, int ms, const St<T>& bL,
+__host__ __device__ __forceinline__ St<T> node_flux(const QuadRows& rows, const T* diff, int cs, int ms, const St<T>& bL,
                                            const St<T>& bR, int dir, T gamma, bool rate, T& smax) {
 #pragma clang fp contract(off)
   using R = NodeRows<T, ORDER>;
@@ -425,14 +445,14 @@ __device__ __forceinline__ St<T> node_flux(const QuadRows& rows, const T* diff, 
   if (rate) {
     const St<T> a = rot(bL, dir), b = rot(bR, dir);
     Side<T> l, r;
-    const bool good_l = side_of(a, gamma, l), good_r = side_of(b, gamma, r);
-    smax = base_rate(a, l, good_l, b, r, good_r, ORDER, gamma);
+    const bool good_l = decided_side(bL, a, gamma, l), good_r = decided_side(bR, b, gamma, r);
+    smax = base_rate(l, good_l, r, good_r, ORDER, gamma);
   }
   St<T> acc;
   bool ok = true;
 #pragma nounroll
   for (int q = 0; q <= R::NQ; ++q) {
-    if (q == R::NQ && !__any(!ok)) break;
+    if (q == R::NQ && !any_lane(!ok)) break;
     St<T> a = bL, b = bR;
     if (q < R::NQ) {
 #pragma unroll
@@ -453,9 +473,15 @@ __device__ __forceinline__ St<T> node_flux(const QuadRows& rows, const T* diff, 
     if (q < R::NQ && !(cl && cr)) {
 #pragma nounroll
       for (int side = 0; side < 2; ++side) {
+        const bool sure = side == 0 ? cl : cr;
         St<T> x = a;
         if (side == 1) x = b;
-        ok = ok && admissible_state_ir(x, rcp_near(x.rho), gamma);
+        T p = side == 0 ? l.p : r.p;
+        ok = ok && (sure || admissible_state_p(x, gamma, p));
+        if (side == 0)
+          l.p = p;
+        else
+          r.p = p;
       }
     }
     T speed = T(0);

@@ -363,22 +363,6 @@ __host__ __device__ __forceinline__ bool finite_ratio(T m, T rho) {
   return fin(m / rho);
 }
 
-// As pressure_positive below with the state's 1/rho supplied: the fast value
-// takes the kinetic energy as a product with it; the margin covers that
-// rounding as it covers the rest.
-template <class T>
-__host__ __device__ __forceinline__ bool pressure_positive_ir(const St<T>& u, T inv_rho, T gamma) {
-  const T kin = T(0.5) * (u.mx * u.mx + u.my * u.my + u.mz * u.mz) * inv_rho;
-  const T mag = T(0.5) * (u.bx * u.bx + u.by * u.by + u.bz * u.bz);
-  const T gm1 = gamma - T(1);
-  const T pf = gm1 * ((u.en - kin) - mag);
-  const T margin = T(32) * Lim<T>::eps * gm1 * (qabs(u.en) + kin + mag);
-  if (fin(pf) && fin(margin) && pf > margin) return true;
-  if (fin(pf) && fin(margin) && pf < -margin) return false;
-  const T p = ref_pressure(u, gamma);
-  return fin(p) && p > T(0);
-}
-
 template <class T>
 __host__ __device__ __forceinline__ bool pressure_positive(const St<T>& u, T gamma) {
   const T kin = fdiv(T(0.5) * (u.mx * u.mx + u.my * u.my + u.mz * u.mz), u.rho);

@@ -424,22 +424,25 @@ __host__ __device__ __forceinline__ St<T> load_cell_lo(const GridD& g, const Sta
 
 // Reconstructed-state admissibility (mhd_reconstruct.hip:433-446): finite
 // components and primitive velocities, rho > 0, reference pressure > 0.
-// admissible_state with the state's 1/rho supplied (for finite rho > 0 the
-// same decisions; the pressure sign test keeps its margin and exact fallback).
-template <class T>
-__host__ __device__ __forceinline__ bool admissible_state_ir(const St<T>& s, T inv_rho, T gamma) {
-  if (!(fin(s.rho) && s.rho > T(0))) return false;
-  if (!(fin(s.mx) && fin(s.my) && fin(s.mz) && fin(s.en) && fin(s.bx) && fin(s.by) && fin(s.bz))) return false;
-  if (!(finite_ratio(s.mx, s.rho) && finite_ratio(s.my, s.rho) && finite_ratio(s.mz, s.rho))) return false;
-  return pressure_positive_ir(s, inv_rho, gamma);
-}
-
 template <class T>
 __host__ __device__ __forceinline__ bool admissible_state(const St<T>& s, T gamma) {
   if (!(fin(s.rho) && s.rho > T(0))) return false;
   if (!(fin(s.mx) && fin(s.my) && fin(s.mz) && fin(s.en) && fin(s.bx) && fin(s.by) && fin(s.bz))) return false;
   if (!(finite_ratio(s.mx, s.rho) && finite_ratio(s.my, s.rho) && finite_ratio(s.mz, s.rho))) return false;
   return pressure_positive(s, gamma);
+}
+
+// The reference's decision with its pressure, in p where the state is
+// admissible.
+template <class T>
+__host__ __device__ __forceinline__ bool admissible_state_p(const St<T>& s, T gamma, T& p) {
+  if (!(fin(s.rho) && s.rho > T(0))) return false;
+  if (!(fin(s.mx) && fin(s.my) && fin(s.mz) && fin(s.en) && fin(s.bx) && fin(s.by) && fin(s.bz))) return false;
+  if (!(finite_ratio(s.mx, s.rho) && finite_ratio(s.my, s.rho) && finite_ratio(s.mz, s.rho))) return false;
+  const T v = ref_pressure(s, gamma);
+  if (!(fin(v) && v > T(0))) return false;
+  p = v;
+  return true;
 }
 
 // Replace the normal field of a face state keeping its pressure: the energy

@@ -1,6 +1,6 @@
-// Host build of the face functions of the MP5/MP7 path (quasar_amd/csrc/
-// qmhd_recon.hpp): its basis decisions and whole faces, state by state on the
-// CPU.
+// Host build of the face functions of the step kernels (quasar_amd/csrc/
+// qmhd_recon.hpp, qmhd_face.hpp): basis decisions, whole reconstructed faces,
+// face fluxes and rates, state by state on the CPU.
 #include "../../quasar_amd/csrc/qmhd_recon.hpp"
 
 using namespace qmhd;
@@ -22,7 +22,52 @@ static void decisions(long n, const double* s8, double gamma, int32_t* out) {
   }
 }
 
+// Fluxes and signal speeds of n faces: s holds 16 planes (L, R) by the 2 H + 1
+// face averages along the face line (one average for orders without nodes).
+template <class T, int ORDER, bool LF>
+static void fluxes(long n, const double* s, int dir, T gamma, double* flux, double* rate) {
+  constexpr int H = ORDER == 7 ? 3 : ORDER == 5 ? 2 : 0, W = 2 * H + 1;
+  QuadRows rows;
+  build_quad_rows(rows);
+  for (long t = 0; t < n; ++t) {
+    const double* v = s + static_cast<std::size_t>(t) * 16 * W;
+    T diff[16][W] = {};
+    St<T> l, r;
+    for (int c = 0; c < 16; ++c) {
+      for (int m = 0; m + 1 < W; ++m) diff[c][m] = T(v[c * W + m + 1]) - T(v[c * W + m]);
+      set_comp(c < 8 ? l : r, c % 8, T(v[c * W + H]));
+    }
+    T speed;
+    St<T> f;
+    if constexpr (H > 0)
+      f = node_flux<T, ORDER, LF>(rows, &diff[0][0], W, 1, l, r, dir, gamma, true, speed);
+    else
+      f = average_flux<T, LF>(l, r, dir, ORDER, gamma, true, speed);
+    for (int c = 0; c < 8; ++c) flux[8 * t + c] = comp(f, c);
+    rate[t] = speed;
+  }
+}
+
+template <class T>
+static void fluxes_of(int order, int lf, long n, const double* s, int dir, double gamma, double* flux, double* rate) {
+  if (order == 1)
+    lf ? fluxes<T, 1, true>(n, s, dir, T(gamma), flux, rate) : fluxes<T, 1, false>(n, s, dir, T(gamma), flux, rate);
+  else if (order == 2)
+    fluxes<T, 2, false>(n, s, dir, T(gamma), flux, rate);
+  else if (order == 5)
+    fluxes<T, 5, false>(n, s, dir, T(gamma), flux, rate);
+  else
+    fluxes<T, 7, false>(n, s, dir, T(gamma), flux, rate);
+}
+
 extern "C" {
+
+void fk_fluxes(int fp32, int order, int lf, long n, const double* s, int dir, double gamma, double* flux, double* rate) {
+  if (fp32)
+    fluxes_of<float>(order, lf, n, s, dir, gamma, flux, rate);
+  else
+    fluxes_of<double>(order, lf, n, s, dir, gamma, flux, rate);
+}
 
 void fk_basis_decisions(int fp32, long n, const double* s8, double gamma, int32_t* out) {
   if (fp32)
