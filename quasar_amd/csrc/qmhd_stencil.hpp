@@ -105,28 +105,67 @@ __host__ __device__ __forceinline__ void two_sum(double a, double b, double& s, 
   e = (a - (s - bv)) + (b - bv);
 }
 
-// Correctly rounded sum of the finite terms that each(f) hands to f, in four
-// chained accumulators: every two-sum error moves one accumulator down, so
-// only the last one rounds, 2^-159 of the running magnitude and below, and the
-// four are rounded from the top with cr_sum's half-even correction.  The rare
-// path behind certified_sum; its registers (cr_sum<16> keeps 16 partials) do
-// not grow with the number of terms.
+// A zero that the compiler does not know: what is computed from it in a loop
+// stays in the loop (all terms hoisted out of cr_sum_each's take 20 registers of
+// the preparation kernel, past three waves per SIMD).
+__host__ __device__ __forceinline__ double opaque_zero() {
+  double z = 0.0;
+#if defined(__HIP_DEVICE_COMPILE__)
+  asm volatile("" : "+v"(z));
+#endif
+  return z;
+}
+
+// Correctly rounded sum of the terms that each(f) hands to f (at most 32; NaN
+// where one or the sum is not finite, as the expansion arithmetic gives).
+// Error-free extraction (Rump, Ogita and Oishi 2008): against a power of two
+// above all partial sums every term splits into a multiple of that power's last
+// bit, which add exactly, and a rest for the next, 2^46 smaller power.  Four
+// chained accumulators take the exact sums of the slices, from the top, and are
+// rounded with cr_sum's half-even correction; what they lose lies 159 bits and
+// more under a leading part that no later slice reaches.  The rare path behind
+// certified_sum: the terms are formed again for every slice, so its registers
+// do not grow with their number (cr_sum<16> keeps 16 partials).
 template <class E>
-__host__ __device__ __forceinline__ double cr_sum_chain(E each) {
+__host__ __device__ __forceinline__ double cr_sum_each(E each) {
 #pragma clang fp contract(off)
-  double c[4] = {0.0, 0.0, 0.0, 0.0};
+  double top = 0.0, bad = 0.0;
   each([&](double t) {
-    two_sum(c[0], t, c[0], t);
-    two_sum(c[1], t, c[1], t);
-    two_sum(c[2], t, c[2], t);
-    c[3] += t;
+    bad = bad + (t - t);
+    top = __builtin_fmax(top, __builtin_fabs(t));
   });
+  if (bad != 0.0) return bad;
+  if (top == 0.0) return 0.0;
+  int e;
+  (void)__builtin_frexp(top, &e);
+  // Sums of terms next to the largest number are taken 2^60 smaller.
+  const double unit = e > 1000 ? 0x1p-60 : 1.0, first = __builtin_ldexp(1.0, (e > 1000 ? e - 60 : e) + 6);
+  double c[4] = {0.0, 0.0, 0.0, 0.0};
+  bool more = true;
+#pragma nounroll
+  for (double sigma = first; more; sigma = sigma * 0x1p-46) {
+    double slice = 0.0;
+    more = false;
+    each([&](double t) {
+      double rest = t * unit;
+#pragma nounroll
+      for (double s = first; s > sigma; s = s * 0x1p-46) rest = rest - ((s + rest) - s);
+      const double part = (sigma + rest) - sigma;
+      slice = slice + part;
+      more = more || rest != part;
+    });
+    two_sum(c[0], slice, c[0], slice);
+    two_sum(c[1], slice, c[1], slice);
+    two_sum(c[2], slice, c[2], slice);
+    c[3] = c[3] + slice;
+  }
 #pragma unroll
   for (int pass = 0; pass < 3; ++pass)
 #pragma unroll
     for (int q = 2; q >= 0; --q) two_sum(c[q], c[q + 1], c[q], c[q + 1]);
   const double t[4] = {c[3], c[2], c[1], c[0]};
-  return cr_sum<4>(t);
+  const double r = cr_sum<4>(t) * (1.0 / unit);
+  return __builtin_isfinite(r) ? r : r - r;
 }
 
 // Whether s + e, within `bound` of the exact sum of terms whose magnitudes add
@@ -160,6 +199,14 @@ __host__ __device__ __forceinline__ double quot(double a, double b, double y) {
 }
 
 template <int W>
+__host__ __device__ __forceinline__ bool all_finite(const double* s) {
+  bool finite = true;
+#pragma unroll
+  for (int k = 0; k < W; ++k) finite = finite && __builtin_isfinite(s[k]);
+  return finite;
+}
+
+template <int W>
 struct CentredRow;
 template <>
 struct CentredRow<8> {
@@ -186,7 +233,7 @@ struct CentredRow<2> {
 // (mhd_staggering.hpp:59-70): the value of the reference's exact rational
 // collocation.  The numerator is a compensated dot product (Ogita, Rump and
 // Oishi's Dot2: at most 64 eps^2/4 sum|w s| from the exact sum, bounded by
-// certified_sum's 512 eps^2); ties and heavy cancellation take the chain.
+// certified_sum's 512 eps^2); ties and heavy cancellation take cr_sum_each.
 template <int W>
 __host__ __device__ __forceinline__ double colloc_centred(const double* s) {
 #pragma clang fp contract(off)
@@ -200,7 +247,7 @@ __host__ __device__ __forceinline__ double colloc_centred(const double* s) {
     e = e + (t + lo);
     mag = mag + __builtin_fabs(p);
   }
-  if (!__builtin_isfinite(mag)) {
+  if (!__builtin_isfinite(mag) && !all_finite<W>(s)) {
     double acc = 0.0;
 #pragma unroll
     for (int k = 0; k < W; ++k) acc = acc + R::w[k] * s[k];
@@ -208,12 +255,13 @@ __host__ __device__ __forceinline__ double colloc_centred(const double* s) {
   }
   double r;
   if (!certified_sum(sum, e, mag, r))
-    r = cr_sum_chain([&](auto f) {
+    r = cr_sum_each([&](auto f) {
+      const double zero = opaque_zero();
 #pragma unroll
       for (int k = 0; k < W; ++k) {
-        const double p = R::w[k] * s[k];
+        const double x = s[k] + zero, p = R::w[k] * x;
         f(p);
-        f(__builtin_fma(R::w[k], s[k], -p));
+        f(__builtin_fma(R::w[k], x, -p));
       }
     });
   // A numerator near the bottom of the exponent range leaves no exact residual.
@@ -237,7 +285,7 @@ __host__ __device__ __forceinline__ double colloc_centred_fma(const double* s) {
 // product-quotient terms ((w_q b_k) s_k / (x_q - k)) / den_q, den_q the
 // correctly rounded sum of b_k / (x_q - k).  den depends on (rel, q) alone and
 // is tabulated.  The 4 W terms are summed in double-double and certified; they
-// are formed again, by division, for the chain where that fails, so none is
+// are formed again, by division, for cr_sum_each where that fails, so none is
 // stored.  (Formed
 // once, stored and expanded in registers with den summed on the device, the
 // two ghost strips took 28 us at any grid size, a quarter of a small step.)
@@ -302,20 +350,24 @@ __host__ __device__ __forceinline__ double one_sided(const double* s, int rel) {
 #pragma unroll
   for (int k = 0; k < W; ++k) zero = zero && s[k] == 0.0;
   if (zero) return 0.0;
-  double sum = 0.0, e = 0.0, mag = 0.0, plain = 0.0;
+  double sum = 0.0, e = 0.0, mag = 0.0;
   one_sided_terms<W, false>(s, rel, [&](double t) {
     double lo;
     two_sum(sum, t, sum, lo);
     e = e + lo;
     mag = mag + __builtin_fabs(t);
-    plain = plain + t;
   });
-  if (!__builtin_isfinite(mag)) return plain;
+  if (!__builtin_isfinite(mag) && !all_finite<W>(s)) {
+    // The quotients' residuals are no numbers here: the terms are divided.
+    double acc = 0.0;
+    one_sided_terms<W, true>(s, rel, [&](double t) { acc = acc + t; });
+    return acc;
+  }
   // Quotients near the bottom of the exponent range have no exact residual:
   // they are divided.
   double r;
   if (!certified_sum(sum, e, mag, r) || mag < 0x1p-900)
-    r = cr_sum_chain([&](auto f) { one_sided_terms<W, true>(s, rel, f); });
+    r = cr_sum_each([&](auto f) { one_sided_terms<W, true>(s, rel, f); });
   return r;
 }
 
