@@ -368,6 +368,15 @@ struct PointEz {
   __host__ __device__ __forceinline__ bool unsure() const { return dense & (qabs(q) <= T(32) * Lim<T>::eps * mag); }
 };
 
+// E_z of a cell average as PointEz forms a point's, so that equal states give
+// equal values whichever a cell takes.
+template <class T>
+__host__ __device__ __forceinline__ T average_ez(T rho, T mx, T my, T bx, T by) {
+#pragma clang fp contract(off)
+  const T ir = rcp_near(rho), vx = mx * ir, vy = my * ir;
+  return fm(-vx, by, vy * bx);
+}
+
 // Neighbour-difference rows of the point recovery: point q is
 // s[H] + sum_m step[q][m] (s[m+1] - s[m]), and the running-mean weights of the
 // Gauss average.

@@ -688,7 +688,8 @@ __host__ __device__ __forceinline__ void reconstruct_face(const GridD& g, int di
 // (mhd_ct.hip:414-420): velocities by division, two rounded products added
 // once.  On the device the quotients come from fdiv (within an ulp of the
 // division).  The corner's one-dimensional shortcuts test cell E_z values for
-// exact equality; equal states still give equal values.
+// exact equality: MP5/MP7 cells form theirs as the quadrature's points do
+// (average_ez), so that equal states give equal values.
 template <class T>
 __host__ __device__ __forceinline__ T physical_ez(T rho, T mx, T my, T bx, T by) {
 #pragma clang fp contract(off)
