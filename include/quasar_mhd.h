@@ -345,8 +345,9 @@ int qmhd_solver_plain_faces(qmhd_solver* s, int64_t* plain, int64_t* total);
  * learned form's cheap-face tile, both directions (0: 64x4, 1: 32x8, 2: 128x2,
  * 3: 16x16, 4: 8x32 cells); [9] MP5/MP7 corner kernel (1: 16x16 LDS tile,
  * 0: one thread per corner in the [2,3] block); [10] accepted as [8], without
- * effect (the y faces of a cell are taken with its x faces); [11] reserved (0).  qmhd_solver_autotune times every
- * candidate of each knob over `trial_steps` steps (the live state is restored
+ * effect (the y faces of a cell are taken with its x faces); [11] reserved (0).
+ * qmhd_solver_autotune times every candidate of each knob that shapes a launch
+ * of the run's scheme over `trial_steps` steps (the live state is restored
  * afterwards) and keeps the fastest. */
 #define QMHD_TUNING_INTS 12
 int qmhd_solver_autotune(qmhd_solver* s, int trial_steps, int32_t* tuning_out);

@@ -722,7 +722,9 @@ class Solver {
     const int kinds[3] = {QMHD_KERNEL_FLUX, QMHD_KERNEL_UPDATE, QMHD_KERNEL_CORNER};
     // MP5/MP7 corners: the LDS tile, or one thread per corner in the best block.
     if (order_ >= 5) tuning_.corner_tiled = 0;
-    for (int k = 0; k < 3; ++k) {
+    // (MP5/MP7 take the fluxes in their own tiles, the flux block shapes the
+    // other orders' launches only.)
+    for (int k = order_ >= 5 ? 1 : 0; k < 3; ++k) {
       dim3 best = *knobs[k];
       double best_ms = std::numeric_limits<double>::infinity();
       for (const dim3& c : shapes) {
