@@ -88,15 +88,6 @@ __host__ __device__ __forceinline__ void schedule_fence() {
 #endif
 }
 
-// Whether any lane of the wave has `b` (the host runs one lane).
-__host__ __device__ __forceinline__ bool any_lane(bool b) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  return __any(b);
-#else
-  return b;
-#endif
-}
-
 // What the solver needs of one state, in the frame of the face normal.
 template <class T>
 struct Side {

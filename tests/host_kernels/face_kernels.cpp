@@ -5,9 +5,28 @@
 
 using namespace qmhd;
 
+// The reference's test of L R = I, every row and column formed by itself.
+template <class T>
+static bool usable_plainly(const CharBasis<T>& B) {
+#pragma clang fp contract(off)
+  for (int i = 0; i < 7; ++i)
+    for (int j = 0; j < 7; ++j) {
+      T r[7], l[7], col[7], row[7];
+      basis_rows(B, i, r, l);
+      basis_lrow(B, l, row);
+      basis_rows(B, j, r, l);
+      basis_rcol(B, r, col);
+      T dot = row[0] * col[0];
+      for (int k = 1; k < 7; ++k) dot = dot + row[k] * col[k];
+      if (!fin(dot) || qabs(dot - T(i == j ? 1 : 0)) > T(1024) * Lim<T>::eps) return false;
+    }
+  return true;
+}
+
 // Per state of s8 (n rows of rho, mx, my, mz, E, bx, by, bz): bit 0 the closed
 // forms stand, bit 1 the basis counts as usable without its test, bit 2 the
-// reference-ordered test finds it usable.
+// reference-ordered test finds it usable, bit 3 that test without shared
+// products does.
 template <class T>
 static void decisions(long n, const double* s8, double gamma, int32_t* out) {
   for (long t = 0; t < n; ++t) {
@@ -18,7 +37,7 @@ static void decisions(long n, const double* s8, double gamma, int32_t* out) {
     const bool quick = basis_quick(s, T(gamma), w, conditioned);
     CharBasis<T> B;
     basis_scalars(s, T(gamma), B);
-    out[t] = (quick ? 1 : 0) | (conditioned ? 2 : 0) | (basis_usable(B) ? 4 : 0);
+    out[t] = (quick ? 1 : 0) | (conditioned ? 2 : 0) | (basis_usable(B) ? 4 : 0) | (usable_plainly(B) ? 8 : 0);
   }
 }
 
