@@ -87,15 +87,18 @@ __device__ __forceinline__ bf16x4 lds4(const uint16_t* a) {
 // d2^T, d1 = W2 d2 and dW1 = X^T d1 with H1, d2, d1 and X rounded to BF16 as the
 // forward pass rounds them.  Bound by one wave's latency through a pass: with a
 // partial's passes one after another on one wave a minibatch of 4096 in 4
-// passes ran 64 waves on 16 CUs, 21.8 us; now 12.7 us.
+// passes ran 64 waves on 16 CUs, 21.8 us; now 12.7 us.  A wave with a partial of
+// its own (GROUP 1) writes it as it is: through LDS 100 samples took 2 us more.
+template <int GROUP>
 __global__ __launch_bounds__(256) void mlp_grad_kernel(const uint16_t* __restrict__ packed,
                                                        const float* __restrict__ p, const float* __restrict__ x,
                                                        const float* __restrict__ target,
                                                        const float* __restrict__ weight,
                                                        const long long* __restrict__ order, long long n, int chunks,
-                                                       int group, long long partials, float* __restrict__ partial) {
+                                                       long long partials, float* __restrict__ partial) {
   using namespace mlp;
-  __shared__ float sums[kGradWaves][kPartialStride];
+  constexpr int group = GROUP;
+  __shared__ float sums[GROUP > 1 ? kGradWaves : 1][GROUP > 1 ? kPartialStride : 1];
   __shared__ __align__(16) uint16_t xs_t[kGradWaves][kInPad][16];
   __shared__ __align__(16) uint16_t h1s[kGradWaves][kH][16];
   __shared__ __align__(16) uint16_t d2s[kGradWaves][kH][16];
@@ -183,7 +186,8 @@ __global__ __launch_bounds__(256) void mlp_grad_kernel(const uint16_t* __restric
     }
     __syncthreads();
   }
-  float* out = sums[wv];
+  if (GROUP == 1 && unit >= partials) return;
+  float* out = GROUP > 1 ? sums[wv] : partial + unit * kPartialStride;
 #pragma unroll
   for (int ft = 0; ft < kKs1; ++ft)
 #pragma unroll
@@ -216,6 +220,7 @@ __global__ __launch_bounds__(256) void mlp_grad_kernel(const uint16_t* __restric
     out[kOffB3] = sb3;
     out[kParams] = sl;
   }
+  if (GROUP == 1) return;
   __syncthreads();
   for (int g = 0; g < kGradWaves / group; ++g) {
     const long long to = static_cast<long long>(blockIdx.x) * (kGradWaves / group) + g;
@@ -438,8 +443,12 @@ void launch_mlp_grad(const uint16_t* packed, const float* params, const float* x
   const long long partials = mlp_grad_waves(n, chunks);
   const int group = chunks >= 4 ? 4 : chunks >= 2 ? 2 : 1;
   const long long per_block = kGradWaves / group, blocks = (partials + per_block - 1) / per_block;
-  hipLaunchKernelGGL(mlp_grad_kernel, dim3(static_cast<unsigned>(blocks)), dim3(64 * kGradWaves), 0, stream, packed,
-                     params, x, target, weight, order, n, chunks, group, partials, partial);
+  const dim3 grid(static_cast<unsigned>(blocks)), block(64 * kGradWaves);
+  auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, block, 0, stream, packed, params, x, target, weight, order, n, chunks, partials,
+                       partial);
+  };
+  group == 4 ? launch(mlp_grad_kernel<4>) : group == 2 ? launch(mlp_grad_kernel<2>) : launch(mlp_grad_kernel<1>);
   hipLaunchKernelGGL(mlp_reduce_kernel, dim3((kPartialStride + 63) / 64), dim3(64), 0, stream, partial, partials, grad);
 }
 
