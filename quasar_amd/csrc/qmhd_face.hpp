@@ -257,7 +257,6 @@ __host__ __device__ __forceinline__ St<T> hlld_sides(const St<T>& L, const St<T>
   f.bx = T(0);
   f.by = fm(by, ux, fm(-bn, uy, d6));
   f.bz = fm(bz, ux, fm(-bn, uz, d7));
-  if (upwind) return f;
   ok = ok && fin(f.rho) && fin(f.en);
   if (!negligible) ok = ok && fin(f.mx) && fin(f.my) && fin(f.mz) && fin(f.by) && fin(f.bz);
   if (!ok) {
@@ -265,7 +264,13 @@ __host__ __device__ __forceinline__ St<T> hlld_sides(const St<T>& L, const St<T>
     a.en = enL;
     b.en = enR;
     a.bx = b.bx = bn;
-    f = hll_combine(a, b, phys_flux_of(a, l.ir, l.p), phys_flux_of(b, r.ir, r.p), sl, sr);
+    // The speeds' minima and maxima drop a NaN.  The reference's choices keep
+    // the right state's, and its speeds then lead to the left state's flux.
+    const T right = r.vx + r.cf;
+    if (right != right)
+      f = phys_flux_of(a, l.ir, l.p);
+    else if (!upwind)
+      f = hll_combine(a, b, phys_flux_of(a, l.ir, l.p), phys_flux_of(b, r.ir, r.p), sl, sr);
   }
   return f;
 }

@@ -79,6 +79,56 @@ static void fluxes_of(int order, int lf, long n, const double* s, int dir, doubl
     fluxes<T, 7, false>(n, s, dir, T(gamma), flux, rate);
 }
 
+template <class T, int ORDER>
+static void mp_faces(long n, const double* cells, const double* bn, double gamma, double* out16, int32_t* settled) {
+  for (long t = 0; t < n; ++t) {
+    St<T> l, r;
+    const double* v = cells + static_cast<std::size_t>(t) * 8 * (ORDER + 1);
+    auto cell = [&](int c, int q) { return T(v[c * (ORDER + 1) + q]); };
+    settled[t] = mp_face<T, ORDER>(cell, T(bn[t]), T(gamma), l, r);
+    for (int c = 0; c < 8; ++c) {
+      out16[16 * t + c] = comp(l, c);
+      out16[16 * t + 8 + c] = comp(r, c);
+    }
+  }
+}
+
+// The rows and points of the cell E_z kernel: x values at a node, then y values,
+// each a centre and weighted neighbour differences, E_z by running means.
+template <class T, int ORDER>
+static void cell_ezs(long n, const double* s, double* ez, int32_t* ok) {
+  using R = NodeRows<T, ORDER>;
+  constexpr int W = R::NM + 1, H = W / 2;
+  QuadRows rows;
+  build_quad_rows(rows);
+  for (long t = 0; t < n; ++t) {
+    const double* v = s + static_cast<std::size_t>(t) * 8 * W * W;
+    T whole = T(0);
+    ok[t] = 1;
+    for (int qx = 0; qx < R::NQ; ++qx) {
+      T mean = T(0);
+      for (int qy = 0; qy < R::NQ; ++qy) {
+        PointEz<T> pt;
+        for (int c = 0; c < 8; ++c) {
+          T column[W];
+          for (int y = 0; y < W; ++y) {
+            const double* row = v + (c * W + y) * W;
+            column[y] = T(row[H]);
+            for (int m = 0; m + 1 < W; ++m) column[y] = fm(R::step(rows, qx, m), T(row[m + 1]) - T(row[m]), column[y]);
+          }
+          T p = column[H];
+          for (int m = 0; m + 1 < W; ++m) p = fm(R::step(rows, qy, m), column[m + 1] - column[m], p);
+          pt.take(c, p);
+        }
+        if (!pt.sure()) ok[t] = 0;
+        mean = qy == 0 ? pt.ez : fm(R::mean(rows, qy), pt.ez - mean, mean);
+      }
+      whole = qx == 0 ? mean : fm(R::mean(rows, qx), mean - whole, whole);
+    }
+    ez[t] = whole;
+  }
+}
+
 extern "C" {
 
 void fk_fluxes(int fp32, int order, int lf, long n, const double* s, int dir, double gamma, double* flux, double* rate) {
@@ -99,16 +149,19 @@ void fk_basis_decisions(int fp32, long n, const double* s8, double gamma, int32_
 // the normal); out16 the left and right states, settled whether they stand.
 void fk_mp_faces(int order, long n, const double* cells, const double* bn, double gamma, double* out16,
                  int32_t* settled) {
-  for (long t = 0; t < n; ++t) {
-    St<double> l, r;
-    const double* v = cells + static_cast<std::size_t>(t) * 8 * (order + 1);
-    auto cell = [&](int c, int q) { return v[c * (order + 1) + q]; };
-    settled[t] = order == 5 ? mp_face<double, 5>(cell, bn[t], gamma, l, r) : mp_face<double, 7>(cell, bn[t], gamma, l, r);
-    for (int c = 0; c < 8; ++c) {
-      out16[16 * t + c] = comp(l, c);
-      out16[16 * t + 8 + c] = comp(r, c);
-    }
-  }
+  order == 5 ? mp_faces<double, 5>(n, cells, bn, gamma, out16, settled)
+             : mp_faces<double, 7>(n, cells, bn, gamma, out16, settled);
+}
+void fk_mp_faces_fp32(int order, long n, const double* cells, const double* bn, double gamma, double* out16,
+                      int32_t* settled) {
+  order == 5 ? mp_faces<float, 5>(n, cells, bn, gamma, out16, settled)
+             : mp_faces<float, 7>(n, cells, bn, gamma, out16, settled);
+}
+
+// Cell E_z of n cells by the kernel's quadrature: 8 planes by W x W averages
+// each (rows, then columns); ok where every point is certainly admissible.
+void fk_cell_ez(int order, long n, const double* s, double* ez, int32_t* ok) {
+  order == 5 ? cell_ezs<double, 5>(n, s, ez, ok) : cell_ezs<double, 7>(n, s, ez, ok);
 }
 
 }  // extern "C"
