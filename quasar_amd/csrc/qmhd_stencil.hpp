@@ -116,31 +116,55 @@ __host__ __device__ __forceinline__ double opaque_zero() {
   return z;
 }
 
+// Rounds the sum of four accumulators, each under the rounding of the one before
+// it or not, with cr_sum's half-even correction.
+__host__ __device__ __forceinline__ double rounded_chain(double* c) {
+#pragma clang fp contract(off)
+#pragma unroll
+  for (int pass = 0; pass < 3; ++pass)
+#pragma unroll
+    for (int q = 2; q >= 0; --q) two_sum(c[q], c[q + 1], c[q], c[q + 1]);
+  const double t[4] = {c[3], c[2], c[1], c[0]};
+  return cr_sum<4>(t);
+}
+
 // Correctly rounded sum of the terms that each(f) hands to f (at most 32; NaN
-// where one or the sum is not finite, as the expansion arithmetic gives).
-// Error-free extraction (Rump, Ogita and Oishi 2008): against a power of two
-// above all partial sums every term splits into a multiple of that power's last
-// bit, which add exactly, and a rest for the next, 2^46 smaller power.  Four
-// chained accumulators take the exact sums of the slices, from the top, and are
-// rounded with cr_sum's half-even correction; what they lose lies 159 bits and
-// more under a leading part that no later slice reaches.  The rare path behind
-// certified_sum: the terms are formed again for every slice, so its registers
-// do not grow with their number (cr_sum<16> keeps 16 partials).
+// where one or the sum is not finite, as the expansion arithmetic gives).  The
+// rare path behind certified_sum (a one-sided closure in a thousand is a tie);
+// the terms are formed again, so its registers do not grow with their number
+// (cr_sum<16> keeps 16 partials).  First in four chained accumulators: every
+// two-sum error moves one accumulator down, and the sum is exact while the last
+// one does not round.  Where it does (terms that cancel over more than 159
+// bits), by error-free extraction (Rump, Ogita and Oishi 2008): against a power
+// of two above all partial sums every term splits into a multiple of that
+// power's last bit, which add exactly, and a rest for the next, 2^46 smaller
+// power; the accumulators take the slices from the top, and what they lose lies
+// 159 bits and more under a leading part that no later slice reaches.
 template <class E>
 __host__ __device__ __forceinline__ double cr_sum_each(E each) {
 #pragma clang fp contract(off)
+  double c[4] = {0.0, 0.0, 0.0, 0.0};
+  bool exact = true;
+  each([&](double t) {
+    two_sum(c[0], t, c[0], t);
+    two_sum(c[1], t, c[1], t);
+    two_sum(c[2], t, c[2], t);
+    two_sum(c[3], t, c[3], t);
+    exact = exact && t == 0.0;
+  });
+  if (exact) return rounded_chain(c);
   double top = 0.0, bad = 0.0;
   each([&](double t) {
     bad = bad + (t - t);
     top = __builtin_fmax(top, __builtin_fabs(t));
   });
   if (bad != 0.0) return bad;
-  if (top == 0.0) return 0.0;
   int e;
   (void)__builtin_frexp(top, &e);
   // Sums of terms next to the largest number are taken 2^60 smaller.
   const double unit = e > 1000 ? 0x1p-60 : 1.0, first = __builtin_ldexp(1.0, (e > 1000 ? e - 60 : e) + 6);
-  double c[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+  for (int q = 0; q < 4; ++q) c[q] = 0.0;
   bool more = true;
 #pragma nounroll
   for (double sigma = first; more; sigma = sigma * 0x1p-46) {
@@ -159,12 +183,7 @@ __host__ __device__ __forceinline__ double cr_sum_each(E each) {
     two_sum(c[2], slice, c[2], slice);
     c[3] = c[3] + slice;
   }
-#pragma unroll
-  for (int pass = 0; pass < 3; ++pass)
-#pragma unroll
-    for (int q = 2; q >= 0; --q) two_sum(c[q], c[q + 1], c[q], c[q + 1]);
-  const double t[4] = {c[3], c[2], c[1], c[0]};
-  const double r = cr_sum<4>(t) * (1.0 / unit);
+  const double r = rounded_chain(c) * (1.0 / unit);
   return __builtin_isfinite(r) ? r : r - r;
 }
 
