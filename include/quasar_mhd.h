@@ -372,8 +372,8 @@ int qmhd_batch_create(qmhd_solver* const* runs, int count, qmhd_batch** out);
 /* Tile work-queue batch: every run's step is recorded once, and each launch
  * of the step becomes one launch over the tiles of all runs (per-run argument
  * records and tile ranges in device memory; a workgroup finds its tile's
- * run by binary search), so a graph launch advances every run with as many
- * kernel launches as one run's step makes.  The runs must use the same
+ * run among the runs' first tiles), so a graph launch advances every run with
+ * as many kernel launches as one run's step makes.  The runs must use the same
  * scheme, form and launch shapes (set one tuning on all of them).
  * queue_blocks: 0 for one workgroup per tile, where each run ends bit for
  * bit where its own loop would; else a persistent grid of that many

@@ -81,8 +81,10 @@ __host__ __device__ __forceinline__ float qsqrt(float x) { return __builtin_sqrt
 
 // Reciprocal, quotient and square root for the face solvers (signal speeds,
 // Riemann fans), where a last-bit difference moves no decision the reference
-// makes exactly (the characteristic basis keeps qsqrt and IEEE division).  On
-// the device, FP64 starts from the hardware's approximate v_rcp_f64 /
+// makes exactly.  The wave basis that rounds as the reference's does keeps
+// qsqrt and IEEE division; the closed-form basis, taken where a bound shows
+// that the reference's test must pass, divides through sqrt_pos and rcp_near
+// (qmhd_face.hpp).  On the device, FP64 starts from the hardware's approximate v_rcp_f64 /
 // v_rsq_f64 (about 2^-23 relative error) and refines it with Newton steps.
 // On an MI355X, over 2^18 inputs spanning 2^-60..2^60, every refined
 // reciprocal and square root was within 0.5 ulp of the exact value, as IEEE
@@ -91,8 +93,9 @@ __host__ __device__ __forceinline__ float qsqrt(float x) { return __builtin_sqrt
 // and eleven here).  frcp and fdiv expect a finite, nonzero, normal divisor
 // and give a non-finite result otherwise (every caller tests its inputs or
 // its result for finiteness); fdiv rounds twice, so it can differ from a/b in
-// the last bit.  fsqrt keeps sqrt's results for 0 and +inf.  The host and
-// FP32 use the IEEE operations.
+// the last bit.  fsqrt keeps sqrt's results for 0 and +inf.  The host uses the
+// IEEE operations, and so do these forms in FP32; the FP32 face solver takes
+// rcp_near and sqrt_pos.
 __host__ __device__ __forceinline__ double frcp(double x) {
 #if defined(__HIP_DEVICE_COMPILE__)
   double r = __builtin_amdgcn_rcp(x);

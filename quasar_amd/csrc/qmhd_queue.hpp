@@ -14,7 +14,7 @@
 // every run's step, checks that the runs issue the same kernels with the same
 // block shapes, and replays each launch slot as one launch over the
 // concatenated tiles of all runs, each workgroup mapping its tile to its run
-// by binary search over the runs' first tiles: one workgroup per tile
+// by a ballot over the runs' first tiles: one workgroup per tile
 // (<kernel>_queue), or a persistent grid of `cap` workgroups looping over the
 // tiles (queue_kernel<Q>, through the tile function).
 #pragma once

@@ -460,7 +460,8 @@ __host__ __device__ inline double face_to_cell(const GridD& g, const double* f, 
   return axis_face(g, f, axis, cell, fixed);
 }
 
-// The same value (every padded cell takes one rule).
+// The same value under the name of the ghost cells' rule (every padded cell
+// takes one); for host code that asks for it by that name.
 __host__ __device__ inline double face_to_cell_ghost(const GridD& g, const double* f, int axis, int cell, int fixed) {
   return face_to_cell(g, f, axis, cell, fixed);
 }
@@ -721,12 +722,8 @@ __host__ __device__ __forceinline__ T physical_ez(T rho, T mx, T my, T bx, T by)
 // Transverse quadrature (include/quasar/numerics/finite_volume_quadrature.hpp:
 // 12-68): a point value (or a Gauss average) from N samples with the exact
 // constant-sample shortcut, which returns the centre sample when all N agree.
-// Every sample is read before the test and the test does not short-circuit,
-// so the N reads (from LDS in the cell E_z kernel) go out together: written
-// as `constant && s[t] == ...`, a sample was read only after the comparisons
-// before it, two or three LDS round trips per call (FP64 cell E_z 726 -> 706 us
-// per 2048^2 launch).  A select in place of the early return hoists every
-// read of the kernel's y pass: 188 VGPRs, one wave per SIMD fewer, 791 us.
+// The step's kernels form these values from weighted neighbour differences
+// (qmhd_face.hpp); this form is what host code holds them against.
 template <class T, int N>
 __host__ __device__ __forceinline__ T point_from_averages(const T* s, const double* w) {
   T x[N];
