@@ -164,4 +164,9 @@ void fk_cell_ez(int order, long n, const double* s, double* ez, int32_t* ok) {
   order == 5 ? cell_ezs<double, 5>(n, s, ez, ok) : cell_ezs<double, 7>(n, s, ez, ok);
 }
 
+// Edge values of n rows of order + 1 averages.
+void fk_edge_interp(int order, long n, const double* e, double* out) {
+  for (long t = 0; t < n; ++t) out[t] = edge_interp(order, e + t * (order + 1));
+}
+
 }  // extern "C"
