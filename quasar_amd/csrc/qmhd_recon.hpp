@@ -346,7 +346,9 @@ __host__ __device__ __forceinline__ bool mp_face(Cell cell, T bn, T gamma, St<T>
   for (int c = 0; c < 8; ++c) set_comp(ref, c, fm(T(0.5), cell(c, H), T(0.5) * cell(c, H + 1)));
   WaveBasis<T> B;
   bool conditioned, usable = true;
-  if (!basis_quick(ref, gamma, B, conditioned)) usable = basis_exact(ref, gamma, conditioned, B);
+  // The hint keeps the exact basis out of the closed forms' way: 2048^2 FP64, both
+  // directions, 671 us without it, 637 with it.
+  if (__builtin_expect(!basis_quick(ref, gamma, B, conditioned), 0)) usable = basis_exact(ref, gamma, conditioned, B);
   auto difference = [&](int q, T d[7]) {
     d[0] = cell(0, q) - ref.rho;
     d[1] = cell(1, q) - ref.mx;
