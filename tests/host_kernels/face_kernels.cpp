@@ -164,6 +164,15 @@ void fk_cell_ez(int order, long n, const double* s, double* ez, int32_t* ok) {
   order == 5 ? cell_ezs<double, 5>(n, s, ez, ok) : cell_ezs<double, 7>(n, s, ez, ok);
 }
 
+// The energy's sum when a state takes its face's normal field: the reconstruction's
+// (with whether it is certain) and the correctly rounded one.
+void fk_sum_of_three(long n, const double* abc, double* sum, int32_t* sure, double* exact) {
+  for (long t = 0; t < n; ++t) {
+    sure[t] = sum_of_three(abc[3 * t], abc[3 * t + 1], abc[3 * t + 2], sum[t]);
+    exact[t] = cr_sum<3>(abc + 3 * t);
+  }
+}
+
 // Edge values of n rows of order + 1 averages.
 void fk_edge_interp(int order, long n, const double* e, double* out) {
   for (long t = 0; t < n; ++t) out[t] = edge_interp(order, e + t * (order + 1));
