@@ -37,7 +37,8 @@ __host__ __device__ __forceinline__ float hi2(float a, float b) { return __built
 // hardware's reciprocal square root).  One Goldschmidt step leaves the inverse
 // 19 epsilon off in FP64, so where it is asked for it takes one more against
 // the rounded root: within 2 epsilon, as a quotient of the rounded root is (the
-// wave basis and the Alfven speeds divide by roots).
+// wave basis and the Alfven speeds divide by roots).  2048^2 FP64, both
+// directions: flux 997 -> 1012 us for it, reconstruction 643 -> 651.
 __host__ __device__ __forceinline__ double sqrt_pos(double x, double& half_inv) {
 #if defined(__HIP_DEVICE_COMPILE__)
   const double y = __builtin_amdgcn_rsq(x);
